@@ -17,7 +17,7 @@ extern "C" {
  * exercised; a negative value removes the limit. */
 TT_API tt_status tt_testing_fail_allocations(long long allowed);
 
-/* Compares the line kernel's short square root (v_sqrt_f32 and one residual
+/* Compares the sort kernel's short square root (v_sqrt_f32 and one residual
  * test per neighbour) with the correctly rounded sqrtf on the GPU for the
  * float bit patterns [lo, lo + count), skipping its documented exceptions
  * (0, 2^-96) and the negative denormals: the number of patterns whose
@@ -25,6 +25,11 @@ TT_API tt_status tt_testing_fail_allocations(long long allowed);
  * (0xFFFFFFFF if none). */
 TT_API tt_status tt_testing_short_sqrt(tt_context *ctx, uint32_t lo, uint64_t count,
                                        uint64_t *mismatches, uint32_t *first_bad);
+
+/* The same for the line kernel's root (v_rsq_f32 and one Newton step), on 0,
+ * NaN and [2^-96, 2^127). */
+TT_API tt_status tt_testing_line_root(tt_context *ctx, uint32_t lo, uint64_t count,
+                                      uint64_t *mismatches, uint32_t *first_bad);
 
 /* Runs the FP64 matrix-core products of the nearest-orthonormal iteration
  * on a strided batch of `count` column-major matrices (device pointers,

@@ -281,7 +281,7 @@ struct KernelTimer {
 // rewrite the context's tables) cannot change what the graph reads.
 struct BatchPlan {
     std::vector<int64_t> key;
-    DevBuf desc, imgT, trig, tab, counter, bbox, ckpt, spec, jobs;
+    DevBuf desc, pairs, trig, tab, counter, bbox, ckpt, spec, jobs;
     ttk::DftParams dft = {};      // P3 spectra of every image (jobs in `jobs`)
     // launch parameters of the captured stages (reused for timed eager runs)
     ttk::BatchSinoParams sp = {};
@@ -308,7 +308,7 @@ struct BatchPlan {
     {
         drop_graph();
         desc.release();
-        imgT.release();
+        pairs.release();
         trig.release();
         tab.release();
         counter.release();
@@ -345,7 +345,7 @@ struct tt_context {
     hipEvent_t ev_in = nullptr, ev_out = nullptr;
     hipStream_t own = nullptr;
     hipStream_t stream = nullptr;
-    DevBuf imgT, trig, tab345, io_a, io_b, med_x, med_s, sino_ck;
+    DevBuf pairs, trig, tab345, io_a, io_b, med_x, med_s, sino_ck;
     DevBuf p3_spec;
     DevBuf bw_sino, bw_dsino, bw_z, bw_rec, bw_rec67, bw_part, bw_t6src, bw_t7src, bw_p2src;
     DevBuf nos_med, nos_a, nos_u, nos_v, nos_s, nos_e, nos_c, nos_info, nos_sweeps;
@@ -578,7 +578,7 @@ TT_API tt_status tt_context_destroy(tt_context *ctx)
     (void)hipSetDevice(ctx->device);
     (void)hipStreamSynchronize(ctx->stream);
     DevBuf *bufs[] = {&ctx->p3_spec,
-                      &ctx->imgT, &ctx->trig, &ctx->tab345,
+                      &ctx->pairs, &ctx->trig, &ctx->tab345,
                       &ctx->io_a, &ctx->io_b, &ctx->med_x,
                       &ctx->med_s, &ctx->sino_ck, &ctx->bw_sino, &ctx->bw_dsino, &ctx->bw_z,
                       &ctx->bw_rec, &ctx->bw_rec67, &ctx->bw_part, &ctx->bw_p2src, &ctx->bw_t6src,
@@ -700,6 +700,25 @@ TT_API int tt_angle_count(float angle_step_deg)
     return (int)floor(360.0 / (double)angle_step_deg);
 }
 
+namespace {
+
+// The image's pixel pairs (both directions) and bounding box into the
+// context's workspaces.
+tt_status image_pairs(tt_context *ctx, const float *d_image, int n)
+{
+    const size_t cnt = ttk::image_pair_count(n);
+    TT_HIP(ctx->pairs.ensure(2 * sizeof(float2) * cnt));
+    TT_HIP(ctx->bbox.ensure(ttk::kBboxInts * sizeof(int)));
+    TT_HIP(ctx->timer.begin(TT_KERNEL_AUX, ctx->stream));
+    TT_HIP(ttk::launch_image_pairs(d_image, n, ctx->pairs.as<float2>(),
+                                   ctx->pairs.as<float2>() + cnt, ctx->bbox.as<int>(),
+                                   ctx->stream));
+    TT_HIP(ctx->timer.end(ctx->stream));
+    return TT_OK;
+}
+
+}  // namespace
+
 TT_API tt_status tt_sinograms(tt_context *ctx, const float *d_image, int n,
                               int n_angles, float angle_step_deg,
                               const int32_t *tcodes, int nt, float *d_sino,
@@ -755,16 +774,11 @@ TT_API tt_status tt_sinograms(tt_context *ctx, const float *d_image, int n,
     TT_TRY(ctx->ensure_trig(n_angles, angle_step_deg));
     if (do345)
         TT_TRY(ctx->ensure_tab345(n));
-    TT_HIP(ctx->imgT.ensure(sizeof(float) * (size_t)n * n));
-    TT_HIP(ctx->bbox.ensure(ttk::kBboxInts * sizeof(int)));
-    TT_HIP(ctx->timer.begin(TT_KERNEL_AUX, st));
-    TT_HIP(ttk::launch_transpose(d_image, ctx->imgT.as<float>(), n, st));
-    TT_HIP(ttk::launch_image_bbox(d_image, n, ctx->bbox.as<int>(), st));
-    TT_HIP(ctx->timer.end(st));
+    TT_TRY(image_pairs(ctx, d_image, n));
 
     ttk::SinoParams p = {};
-    p.img = d_image;
-    p.imgT = ctx->imgT.as<float>();
+    p.pair = ctx->pairs.as<float2>();
+    p.pairT = p.pair + ttk::image_pair_count(n);
     p.trig = ctx->trig.as<float2>();
     p.tab345 = do345 ? ctx->tab345.as<float2>() : nullptr;
     p.sino = d_sino;
@@ -785,8 +799,8 @@ TT_API tt_status tt_sinograms(tt_context *ctx, const float *d_image, int n,
     TT_HIP(ctx->timer.end(st));
     if (do6 || do7) {
         ttk::SortTParams q = {};
-        q.img = d_image;
-        q.imgT = ctx->imgT.as<float>();
+        q.pair = ctx->pairs.as<float2>();
+        q.pairT = q.pair + ttk::image_pair_count(n);
         q.trig = ctx->trig.as<float2>();
         q.sino = d_sino;
         q.med_x = med_x;
@@ -1017,7 +1031,7 @@ int layout_dft_jobs(std::vector<ttk::DftJob> &jobs, bool forward, int *bm, int *
 hipError_t enqueue_batch(tt_context *ctx, const ttk::BatchSinoParams &sp,
                          const ttk::BatchCircusParams &cp, int nimg, int nmax,
                          bool need_x, bool need_s, bool do345, int wpb, int blocks,
-                         bool with_transpose, bool with_circus, hipStream_t st,
+                         bool with_pairs, bool with_circus, hipStream_t st,
                          bool timed = false)
 {
     KernelTimer *T = timed ? &ctx->timer : nullptr;
@@ -1032,14 +1046,13 @@ hipError_t enqueue_batch(tt_context *ctx, const ttk::BatchSinoParams &sp,
         if (T && e == hipSuccess)
             e = T->end(st);
     };
-    if (with_transpose)
+    if (with_pairs)
         stage(TT_KERNEL_AUX, [&] {
-            hipError_t r = ttk::launch_transpose_batched(sp.images, nimg, nmax, st);
-            return r == hipSuccess ? ttk::launch_image_bbox_batched(sp.images, nimg, nmax, st)
-                                   : r;
+            return ttk::launch_image_pairs_batched(sp.images, nimg, nmax, sp.counter, st);
         });
     stage(TT_KERNEL_SINO_T05, [&] {
-        hipError_t r = ttk::launch_reset_counter(sp.counter, st);
+        // (the pair pass has zeroed the work counter)
+        hipError_t r = with_pairs ? hipSuccess : ttk::launch_reset_counter(sp.counter, st);
         return r == hipSuccess
                    ? ttk::launch_sino_t05_batched(sp, need_x, need_s, do345, wpb, blocks, st)
                    : r;
@@ -1071,17 +1084,12 @@ hipError_t enqueue_backward(tt_context *ctx, const BackwardPlan &P, hipStream_t 
     const bool p3 = P.p3s.np3 > 0;
     if (!P.saved) {
         stage(TT_KERNEL_AUX, [&] {
-            hipError_t r = ttk::launch_transpose_batched(B.sp.images, B.nimg, B.nmax, st);
-            return r == hipSuccess
-                       ? ttk::launch_image_bbox_batched(B.sp.images, B.nimg, B.nmax, st)
-                       : r;
+            return ttk::launch_image_pairs_batched(B.sp.images, B.nimg, B.nmax, B.sp.counter,
+                                                   st);
         });
-        stage(TT_KERNEL_SINO_T05, [&] {
-            hipError_t r = ttk::launch_reset_counter(B.sp.counter, st);
-            return r == hipSuccess ? ttk::launch_sino_t05_batched(B.sp, true, true, B.do345,
-                                                                  B.waves_per_block, B.blocks,
-                                                                  st)
-                                   : r;
+        stage(TT_KERNEL_SINO_T05, [&] {  // (the pair pass has zeroed the work counter)
+            return ttk::launch_sino_t05_batched(B.sp, true, true, B.do345, B.waves_per_block,
+                                                B.blocks, st);
         });
         if (p3)
             stage(TT_KERNEL_P3_DFT, [&] { return ttk::launch_dft_gemm(P.fdp, true, B.nmax, st); });
@@ -1242,8 +1250,8 @@ TT_API tt_status tt_forward_batched(tt_context *ctx, const tt_image *images,
         std::vector<ttk::BatchImage> d(nimg);
         size_t tot = 0;
         for (int i = 0; i < nimg; i++)
-            tot += (size_t)images[i].n * images[i].n;
-        TT_HIP(B.imgT.ensure(sizeof(float) * tot));
+            tot += 2 * ttk::image_pair_count(images[i].n);
+        TT_HIP(B.pairs.ensure(sizeof(float2) * tot));
         TT_HIP(B.bbox.ensure(ttk::kBboxInts * sizeof(int) * (size_t)nimg));
         size_t ck = 0;  // the line kernel's walk checkpoints, image after image
         for (int i = 0; i < nimg; i++)
@@ -1290,8 +1298,9 @@ TT_API tt_status tt_forward_batched(tt_context *ctx, const tt_image *images,
             b.bbox = B.bbox.as<int>() + ttk::kBboxInts * k;
             b.ckpt = B.ckpt.as<float2>() + cko;
             cko += (size_t)ttk::sino_ckpt_blocks(im.n) * im.n * n_angles;
-            b.imgT = B.imgT.as<float>() + off;
-            off += (size_t)im.n * im.n;
+            b.pair = B.pairs.as<float2>() + off;
+            b.pairT = b.pair + ttk::image_pair_count(im.n);
+            off += 2 * ttk::image_pair_count(im.n);
             b.sino = im.d_sino;
             // with d_saved the medians and T3..T5 integrals a backward needs
             b.med_x = sv && need_x ? (int32_t *)(sv + SL.med_x) : nullptr;
@@ -1365,8 +1374,7 @@ TT_API tt_status tt_forward_batched(tt_context *ctx, const tt_image *images,
         const int cus = device_cus(ctx->device);
         int best_w = 4, best_b = cus * 4;
         if (ctx->autotune) {
-            TT_HIP(ttk::launch_transpose_batched(sp.images, nimg, nmax, own));
-            TT_HIP(ttk::launch_image_bbox_batched(sp.images, nimg, nmax, own));
+            TT_HIP(ttk::launch_image_pairs_batched(sp.images, nimg, nmax, sp.counter, own));
             hipEvent_t e0, e1;
             TT_HIP(hipEventCreate(&e0));
             TT_HIP(hipEventCreate(&e1));
@@ -1593,17 +1601,12 @@ tt_status forward_for_adjoint(tt_context *ctx, const float *d_image, int n, int 
     TT_HIP(ctx->med_s.ensure(sizeof(int32_t) * lines));
     TT_TRY(ctx->ensure_trig(A, step));
     TT_TRY(ctx->ensure_tab345(n));
-    TT_HIP(ctx->imgT.ensure(sizeof(float) * (size_t)n * n));
-    TT_HIP(ctx->bbox.ensure(ttk::kBboxInts * sizeof(int)));
+    TT_TRY(image_pairs(ctx, d_image, n));
     hipStream_t st = ctx->stream;
-    TT_HIP(ctx->timer.begin(TT_KERNEL_AUX, st));
-    TT_HIP(ttk::launch_transpose(d_image, ctx->imgT.as<float>(), n, st));
-    TT_HIP(ttk::launch_image_bbox(d_image, n, ctx->bbox.as<int>(), st));
-    TT_HIP(ctx->timer.end(st));
     ttk::SinoParams p = {};
     p.bbox = ctx->bbox.as<int>();
-    p.img = d_image;
-    p.imgT = ctx->imgT.as<float>();
+    p.pair = ctx->pairs.as<float2>();
+    p.pairT = p.pair + ttk::image_pair_count(n);
     p.trig = ctx->trig.as<float2>();
     p.tab345 = ctx->tab345.as<float2>();
     p.sino = ctx->bw_sino.as<float>();
@@ -1627,8 +1630,8 @@ tt_status forward_for_adjoint(tt_context *ctx, const float *d_image, int n, int 
         TT_HIP(ctx->bw_t6src.ensure(sizeof(int32_t) * lines));
         TT_HIP(ctx->bw_t7src.ensure(sizeof(int32_t) * lines));
         ttk::SortTParams q = {};
-        q.img = d_image;
-        q.imgT = ctx->imgT.as<float>();
+        q.pair = ctx->pairs.as<float2>();
+        q.pairT = q.pair + ttk::image_pair_count(n);
         q.trig = ctx->trig.as<float2>();
         q.sino = ctx->bw_sino.as<float>();
         q.med_x = ctx->med_x.as<int32_t>();
@@ -2297,9 +2300,9 @@ TT_API tt_status tt_backward_batched(tt_context *ctx, const tt_image_grad *image
         std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
             return images[a].n > images[b].n;
         });
-        size_t sq = 0, ln = 0, spec_tot = 0;
+        size_t pr = 0, ln = 0, spec_tot = 0;
         for (int i = 0; i < nimg; i++) {
-            sq += (size_t)images[i].n * images[i].n;
+            pr += 2 * ttk::image_pair_count(images[i].n);
             ln += (size_t)images[i].n * n_angles;
             spec_tot += (size_t)nt * n_angles * 2 * (images[i].n / 2 + 1);
         }
@@ -2308,7 +2311,7 @@ TT_API tt_status tt_backward_batched(tt_context *ctx, const tt_image_grad *image
         const bool p2src = p2 && nmax <= 2048;
         // without saved line data the forward is recomputed into workspaces
         if (!saved) {
-            TT_HIP(B.imgT.ensure(sizeof(float) * sq));
+            TT_HIP(B.pairs.ensure(sizeof(float2) * pr));
             TT_HIP(P.sino.ensure(sizeof(float) * nt * ln));
             TT_HIP(P.z.ensure(sizeof(float2) * 3 * ln));
             TT_HIP(P.medx.ensure(sizeof(int32_t) * ln));
@@ -2338,7 +2341,7 @@ TT_API tt_status tt_backward_batched(tt_context *ctx, const tt_image_grad *image
         int ftiles = 0, btiles = 0;
         size_t so = 0;
         std::vector<ttk::BatchImage> d(nimg);
-        size_t po = 0, lo = 0, cko = 0;
+        size_t po = 0, lo = 0, cko = 0, pro = 0;
         int cols = 0;
         for (int k = 0; k < nimg; k++) {
             const tt_image_grad &im = images[order[k]];
@@ -2368,7 +2371,9 @@ TT_API tt_status tt_backward_batched(tt_context *ctx, const tt_image_grad *image
                 b.bbox = B.bbox.as<int>() + ttk::kBboxInts * k;
                 b.ckpt = B.ckpt.as<float2>() + cko;
                 cko += (size_t)ttk::sino_ckpt_blocks(im.n) * im.n * n_angles;
-                b.imgT = B.imgT.as<float>() + po;
+                b.pair = B.pairs.as<float2>() + pro;
+                b.pairT = b.pair + ttk::image_pair_count(im.n);
+                pro += 2 * ttk::image_pair_count(im.n);
                 b.sino = P.sino.as<float>() + nt * lo;
                 b.med_x = P.medx.as<int32_t>() + lo;
                 b.med_s = P.meds.as<int32_t>() + lo;
@@ -2710,8 +2715,11 @@ TT_API tt_status tt_testing_nos_product(tt_context *ctx, int trans_a, int sym, i
     return TT_OK;
 }
 
-TT_API tt_status tt_testing_short_sqrt(tt_context *ctx, uint32_t lo, uint64_t count,
-                                       uint64_t *mismatches, uint32_t *first_bad)
+namespace {
+
+// Runs one of the square-root checks on [lo, lo + count).
+tt_status root_check(tt_context *ctx, bool root, uint32_t lo, uint64_t count,
+                     uint64_t *mismatches, uint32_t *first_bad)
 {
     TT_CHECK(ctx && mismatches && first_bad, "NULL argument");
     TT_CHECK(count <= ((uint64_t)1 << 32) - lo, "range past the last bit pattern");
@@ -2726,7 +2734,7 @@ TT_API tt_status tt_testing_short_sqrt(tt_context *ctx, uint32_t lo, uint64_t co
     if (e == hipSuccess)
         e = hipMemcpy(d_f, &none, sizeof none, hipMemcpyHostToDevice);
     if (e == hipSuccess)
-        e = ttk::launch_short_sqrt_check(lo, count, d_m, d_f, ctx->stream);
+        e = ttk::launch_short_sqrt_check(root, lo, count, d_m, d_f, ctx->stream);
     unsigned long long m = 0;
     unsigned int f = 0;
     if (e == hipSuccess)
@@ -2740,4 +2748,18 @@ TT_API tt_status tt_testing_short_sqrt(tt_context *ctx, uint32_t lo, uint64_t co
     *mismatches = m;
     *first_bad = f;
     return TT_OK;
+}
+
+}  // namespace
+
+TT_API tt_status tt_testing_short_sqrt(tt_context *ctx, uint32_t lo, uint64_t count,
+                                       uint64_t *mismatches, uint32_t *first_bad)
+{
+    return root_check(ctx, false, lo, count, mismatches, first_bad);
+}
+
+TT_API tt_status tt_testing_line_root(tt_context *ctx, uint32_t lo, uint64_t count,
+                                      uint64_t *mismatches, uint32_t *first_bad)
+{
+    return root_check(ctx, true, lo, count, mismatches, first_bad);
 }

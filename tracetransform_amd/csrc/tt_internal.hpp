@@ -20,8 +20,8 @@ struct Slots {
 // Forward T-functional sweep for one padded image (T0..T5).  One wave owns
 // 64 adjacent columns of one angle; each lane streams its column's rows.
 struct SinoParams {
-    const float *img;     // n x n column-major
-    const float *imgT;    // n x n row-major copy (transpose of img)
+    const float2 *pair;   // pixel pairs along the columns (see launch_image_pairs)
+    const float2 *pairT;  // pixel pairs along the rows
     const float2 *trig;   // [A] (cos(-theta), sin(-theta)) as float
     const float2 *tab345; // [3][n] (re, im) tables of T3, T4, T5
     float *sino;          // [nt][A][n]
@@ -60,12 +60,12 @@ struct LineRecord67 {
 // One image of a batch (device array, ordered by first item).
 struct BatchImage {
     const float *img;     // n x n column-major
-    // (the batched forward writes neither medians nor T3..T5 integrals)
-    const float *imgT;    // row-major copy (written by the batched transpose)
+    float2 *pair;         // pixel pairs along the columns (see launch_image_pairs)
+    float2 *pairT;        // pixel pairs along the rows
     float *sino;          // [nt][A][n]
     int32_t *med_x;
     int32_t *med_s;
-    const int *bbox;      // non-zero pixels' bounds {x0, x1, y0, y1} + flag, or null
+    int *bbox;            // non-zero pixels' bounds {x0, x1, y0, y1} + flag, or null
     float2 *ckpt;         // [sino_ckpt_blocks(n)][A][n] walk prefixes (workspace)
     int n;
     int nb;               // column tiles per angle tile (batched line kernel)
@@ -117,8 +117,8 @@ struct BatchCircusParams {
 // Sort-based T-functionals T6/T7 for one padded image: one workgroup owns one
 // (angle, column) line at a time.
 struct SortTParams {
-    const float *img;     // n x n column-major
-    const float *imgT;    // row-major copy
+    const float2 *pair;   // pixel pairs along the columns (see launch_image_pairs)
+    const float2 *pairT;  // pixel pairs along the rows
     const float2 *trig;
     float *sino;
     int32_t *med_x;
@@ -255,11 +255,12 @@ size_t dft_lds_bytes(int nmax);
 hipError_t launch_dft_gemm(const DftParams &p, bool forward, int nmax, hipStream_t s);
 hipError_t launch_p3_vjp_scale(const P3ScaleParams &p, int max_cols, hipStream_t s);
 
-// Test hook: mismatches of the line kernel's short square root against
-// sqrtf over float bit patterns [lo, lo + count) (mism and first in device
-// memory, first initialised to 0xFFFFFFFF by the caller).
-hipError_t launch_short_sqrt_check(uint32_t lo, uint64_t count, unsigned long long *mism,
-                                   unsigned int *first, hipStream_t s);
+// Test hook: mismatches of the sort kernel's short square root (root: of the
+// line kernel's) against sqrtf over float bit patterns [lo, lo + count) (mism
+// and first in device memory, first initialised to 0xFFFFFFFF by the caller).
+hipError_t launch_short_sqrt_check(bool root, uint32_t lo, uint64_t count,
+                                   unsigned long long *mism, unsigned int *first,
+                                   hipStream_t s);
 
 // Steps either side of the path and the orthonormal step.
 hipError_t launch_resize(const float *in, int in_rows, int in_cols, float *out,
@@ -338,19 +339,31 @@ hipError_t launch_records(const RecordParams &p, hipStream_t s);
 hipError_t launch_gather(const GatherParams &p, hipStream_t s);
 hipError_t launch_circus_vjp(const CircusVjpParams &p, hipStream_t s);
 
-hipError_t launch_transpose(const float *in, float *out, int n, hipStream_t s);
+// The two pixel-pair copies the sampling kernels read, image_pair_count(n)
+// entries each: pair[X n + Y] = (p(X, Y), p(X + 1, Y)) for the column-major
+// image p, pairT[Y n + X] = (p(X, Y), p(X, Y + 1)), zero past the last row or
+// column.  The 2 x 2 taps of a bilinear sample are then 16 consecutive bytes
+// of either copy: one load a sample instead of two.  The same pass finds the
+// bounding box {x0, x1, y0, y1} (columns, rows) of the non-zero pixels, for
+// the line kernels' row ranges; an all-zero image gives x0 > x1.  Word 4 of
+// bbox is 1 when some pixel is neither 0 nor in [2^-45, 2^120] (then a
+// bilinear sample can be negative, a positive value below 2^-96, infinite or
+// NaN, and the kernels take the library's square root), else 0.  bbox
+// holds kBboxInts words: the result, then scratch for the blocks' boxes.
+constexpr int kPairBlocks = 512;  // at most, per image
+constexpr int kBboxInts = 8 * (1 + kPairBlocks);
+__host__ __device__ inline size_t image_pair_count(int n)
+{
+    return (size_t)n * n + 2;  // a sample at the last pixel loads one pair more
+}
+hipError_t launch_image_pairs(const float *img, int n, float2 *pair, float2 *pairT, int *bbox,
+                              hipStream_t s);
+// The same for every image of a batch (into images[k].pair, pairT, bbox);
+// counter: a word the same launches set to zero.
+hipError_t launch_image_pairs_batched(const BatchImage *images, int nimg, int nmax,
+                                      unsigned int *counter, hipStream_t s);
 hipError_t launch_pad(const float *in, int rows, int cols, float *out, int n,
                       int dfx, int dfy, hipStream_t s);
-// Bounding box {x0, x1, y0, y1} (columns, rows) of the non-zero pixels of an
-// n x n column-major image, for the line kernels' row ranges; an all-zero
-// image gives x0 > x1.  Word 4 is 1 when some pixel is negative or in
-// (0, 2^-45) (then a bilinear sample can be a negative or a positive value
-// below 2^-96), else 0.  kBboxInts words per image.
-constexpr int kBboxInts = 8;
-hipError_t launch_image_bbox(const float *img, int n, int *bbox, hipStream_t s);
-// The same for every image of a batch (bbox of image k at images[k].bbox).
-hipError_t launch_image_bbox_batched(const BatchImage *images, int nimg, int nmax,
-                                     hipStream_t s);
 // Checkpoints of the median walks the T0..T5 line kernel keeps per line:
 // the prefixes at the starts of its 64-step blocks after the first, up to
 // this many (a wave of one angle and 64 columns spans at most n + 64 steps
@@ -389,8 +402,6 @@ hipError_t launch_circus(const CircusParams &p, hipStream_t s);
 
 // Batched path; `waves_per_block` in {1, 2, 4} and `blocks` (persistent grid)
 // are the autotuned launch shape.
-hipError_t launch_transpose_batched(const BatchImage *d_images, int nimg,
-                                    int nmax, hipStream_t s);
 hipError_t launch_reset_counter(unsigned int *counter, hipStream_t s);
 hipError_t launch_sino_t05_batched(const BatchSinoParams &p, bool need_x,
                                    bool need_s, bool do345, int waves_per_block,

@@ -16,30 +16,29 @@ namespace ttk {
 
 namespace {
 
-// 8-byte load from a 4-byte aligned address (unaligned dwordx2 is legal for
-// global memory on CDNA).
-typedef float f2u __attribute__((ext_vector_type(2), aligned(4)));
+// 16-byte load from an 8-byte aligned address (legal for global memory on
+// CDNA): two neighbouring pixel pairs.
+typedef float f4p __attribute__((ext_vector_type(4), aligned(8)));
 
 // A pointer every lane of the wave holds, made visibly wave-uniform (its
 // two halves read from the first lane), so that loads from it can take the
 // scalar-base form.
-__device__ __forceinline__ const float *uniform_ptr(const float *p)
+__device__ __forceinline__ const float2 *uniform_ptr(const float2 *p)
 {
     const uint64_t v = reinterpret_cast<uint64_t>(p);
     const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
     const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-    return reinterpret_cast<const float *>(((uint64_t)hi << 32) | lo);
+    return reinterpret_cast<const float2 *>(((uint64_t)hi << 32) | lo);
 }
 
 // Load at a 32-bit byte offset from a wave-uniform base in global memory:
 // the scalar-base + vector-offset form of global loads (no 64-bit VALU
 // math, no flat addressing).
-__device__ __forceinline__ f2u ld2b(const float *base, uint32_t byte_off)
+__device__ __forceinline__ f4p ld4b(const float2 *base, uint32_t byte_off)
 {
     typedef const char __attribute__((address_space(1))) *gbyte;
-    typedef const float __attribute__((address_space(1))) *gfloat;
-    const gfloat q = (gfloat)((gbyte)base + byte_off);
-    return f2u{q[0], q[1]};
+    typedef const f4p __attribute__((address_space(1))) *gf4;
+    return *(gf4)((gbyte)base + byte_off);
 }
 
 __device__ __forceinline__ int wave_id()
@@ -63,51 +62,74 @@ __device__ __forceinline__ int xcd_block()
 // pxc = px*c and pxns = px*(-s) precomputed per lane (each is one rounded
 // product, as in the reference).  Strict bounds 0 <= x,y < n-1; the four
 // taps are evaluated left to right with the reference's association.
-// TR selects the row-major copy of the image so that lanes stepping along x
-// read contiguous memory; the tap values (hence the result) are identical.
+// src is the pixel-pair copy of the image that the lanes step along: TR (along
+// x) pairs of rows, else pairs of columns; the four taps are one 16-byte load.
+// The L1 looks up one line per four lanes of a load whatever the load's width,
+// about 25 cycles per load and CU, and two 8-byte loads a sample (one per
+// image row) made that the line kernel's bound: 0.87 ms against 0.59 for the
+// samples of 1449^2 pixels at 360 angles (a copy of 2 x 2 quads, four times
+// the image, reads 0.97: it leaves the L2).
 // ---------------------------------------------------------------------------
-template <bool TR>
-__device__ __forceinline__ float rot_sample(const float *__restrict__ src,
-                                            int n, float lim, float o,
-                                            float pxc, float pxns, float c,
-                                            float s, float py)
+// A sample whose load is under way: its taps, fractions and whether it lies
+// inside the image.
+struct Tap {
+    f4p q;
+    float fx, fy;
+    bool in;
+};
+
+// CHK: test the position against the image's bounds (without it the caller
+// knows that the position is inside).
+template <bool TR, bool CHK>
+__device__ __forceinline__ Tap rot_load(const float2 *__restrict__ src, int n, float lim,
+                                        float o, float pxc, float pxns, float c, float s,
+                                        float py)
 {
+    Tap t;
     float x = pxc + py * s;
     float y = pxns + py * c;
     x = x + o;
     y = y + o;
-    // 0 <= x < lim as one unsigned compare of the bit patterns: x is never
-    // -0 (a sum with o > 0 rounds an exact zero to +0), non-negative floats
-    // order as their bits, and negative values and NaN compare above lim
-    const bool inb = __float_as_uint(x) < __float_as_uint(lim) &&
-                     __float_as_uint(y) < __float_as_uint(lim);
     // for 0 <= x the integer part is the truncating conversion and the
     // fraction x - floor(x) is exact (modf's split)
-    const float fx = __builtin_amdgcn_fractf(x);
-    const float fy = __builtin_amdgcn_fractf(y);
+    t.fx = __builtin_amdgcn_fractf(x);
+    t.fy = __builtin_amdgcn_fractf(y);
     // unsigned 32-bit offsets from a wave-uniform base: global loads in
     // scalar-base + vector-offset form, no 64-bit address arithmetic
-    const uint32_t X = inb ? (uint32_t)x : 0u;
-    const uint32_t Y = inb ? (uint32_t)y : 0u;
-    const uint32_t un = (uint32_t)n;
-    float s00, s01, s10, s11;
-    // X, Y < n <= 2730, so X * n fits the 24-bit multiplier
-    if (!TR) {
-        const uint32_t o0 = (__umul24(X, un) + Y) * 4u;
-        const f2u a = ld2b(src, o0);
-        const f2u b = ld2b(src, o0 + 4u * un);
-        s00 = a.x; s10 = a.y; s01 = b.x; s11 = b.y;
-    } else {
-        const uint32_t o0 = (__umul24(Y, un) + X) * 4u;
-        const f2u a = ld2b(src, o0);
-        const f2u b = ld2b(src, o0 + 4u * un);
-        s00 = a.x; s01 = a.y; s10 = b.x; s11 = b.y;
+    uint32_t X = (uint32_t)x, Y = (uint32_t)y;
+    t.in = true;
+    if constexpr (CHK) {
+        // 0 <= x < lim as one unsigned compare of the bit patterns: x is never
+        // -0 (a sum with o > 0 rounds an exact zero to +0), non-negative floats
+        // order as their bits, and negative values and NaN compare above lim
+        t.in = __float_as_uint(x) < __float_as_uint(lim) &&
+               __float_as_uint(y) < __float_as_uint(lim);
+        X = t.in ? X : 0u;
+        Y = t.in ? Y : 0u;
     }
-    const float ofx = 1.0f - fx;
-    const float ofy = 1.0f - fy;
-    const float v = s00 * ofx * ofy + s01 * fx * ofy + s10 * ofx * fy +
-                    s11 * fx * fy;
-    return inb ? v : 0.0f;
+    const uint32_t un = (uint32_t)n;
+    // X, Y < n <= 2730, so X * n fits the 24-bit multiplier
+    t.q = ld4b(src, (TR ? __umul24(Y, un) + X : __umul24(X, un) + Y) * 8u);
+    return t;
+}
+
+template <bool TR, bool CHK>
+__device__ __forceinline__ float rot_value(const Tap &t)
+{
+    const float s00 = t.q.x, s01 = TR ? t.q.z : t.q.y, s10 = TR ? t.q.y : t.q.z, s11 = t.q.w;
+    const float ofx = 1.0f - t.fx;
+    const float ofy = 1.0f - t.fy;
+    const float v = s00 * ofx * ofy + s01 * t.fx * ofy + s10 * ofx * t.fy +
+                    s11 * t.fx * t.fy;
+    return !CHK || t.in ? v : 0.0f;
+}
+
+template <bool TR>
+__device__ __forceinline__ float rot_sample(const float2 *__restrict__ src, int n, float lim,
+                                            float o, float pxc, float pxns, float c, float s,
+                                            float py)
+{
+    return rot_value<TR, true>(rot_load<TR, true>(src, n, lim, o, pxc, pxns, c, s, py));
 }
 
 // Square root of a line sample, correctly rounded.  FS: v_sqrt_f32 and one
@@ -132,10 +154,31 @@ __device__ __forceinline__ float line_sqrt(float x)
     }
 }
 
+// The line kernel's root: FS: v_rsq_f32, its product with x and one Newton
+// step with an exact residual (fma), 7 issue slots of a line_sqrt<true>'s 11.
+// Equal to the correctly rounded root on 0 and on every float in
+// [2^-96, 2^127) (checked on the GPU over all of them); NaN gives NaN.  The
+// image flag rules out samples elsewhere: negative ones, (0, 2^-96), infinite.
+template <bool FS>
+__device__ __forceinline__ float line_root(float x)
+{
+    if constexpr (!FS) {
+        return sqrtf(x);
+    } else {
+        // (the addend keeps the reciprocal root of 0 finite and rounds away
+        // from 2^-96 on)
+        const float y = __builtin_amdgcn_rsqf(x + 0x1p-126f);
+        const float g = x * y;
+        return fmaf(fmaf(-g, g, x), 0.5f * y, g);
+    }
+}
+
 // Test hook: line_sqrt<true> against the correctly rounded sqrtf on the
 // float bit patterns [lo, lo + count), outside its documented exceptions
 // ((0, 2^-96) and the negative denormals).  Counts the patterns whose
 // results differ (NaN results compare equal) and keeps the smallest one.
+// ROOT: line_root<true> instead, on 0, NaN and [2^-96, 2^127).
+template <bool ROOT>
 __global__ __launch_bounds__(kBlock) void short_sqrt_check_kernel(uint32_t lo, uint64_t count,
                                                                  unsigned long long *mism,
                                                                  unsigned int *first)
@@ -147,10 +190,12 @@ __global__ __launch_bounds__(kBlock) void short_sqrt_check_kernel(uint32_t lo, u
         const uint32_t b = lo + (uint32_t)i;
         const bool tiny = b > 0u && b < 0x0F800000u;           // (0, 2^-96)
         const bool negden = b > 0x80000000u && b < 0x80800000u;  // negative denormals
-        if (tiny || negden)
-            continue;
         const float x = __uint_as_float(b);
-        const float a = line_sqrt<true>(x), r = line_sqrt<false>(x);
+        if (ROOT ? !(x == 0.0f || x != x || (x >= 0x1p-96f && x < 0x1p127f))
+                 : tiny || negden)
+            continue;
+        const float a = ROOT ? line_root<true>(x) : line_sqrt<true>(x);
+        const float r = line_sqrt<false>(x);
         const bool same = __float_as_uint(a) == __float_as_uint(r) || (a != a && r != r);
         if (!same) {
             bad++;
@@ -174,8 +219,34 @@ __global__ __launch_bounds__(kBlock) void short_sqrt_check_kernel(uint32_t lo, u
 // T1/T2 (c++/src/functionals.cpp:104-129) and T3/T4/T5
 // (c++/src/functionals.cpp:200-213) over the same rows as the reference.
 // ---------------------------------------------------------------------------
-// Where one line's results go.  slot[t] is the output slot of T-code t
-// (-1 if not requested); tabn is the row stride of the T3..T5 tables in LDS.
+// Wave minimum and maximum as wave-uniform values, by data-parallel moves
+// (rows of 16 lanes, then across rows): no LDS traffic.  Every lane of the
+// wave must be active.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int dpp_i(int v)
+{
+    return __builtin_amdgcn_update_dpp(v, v, CTRL, ROWS, 0xf, false);
+}
+template <class Op>
+__device__ __forceinline__ int wave_reduce_u(int v, Op op)
+{
+    v = op(v, dpp_i<0x111, 0xf>(v));  // row_shr 1, 2, 4, 8: lane 15 of each row
+    v = op(v, dpp_i<0x112, 0xf>(v));
+    v = op(v, dpp_i<0x114, 0xf>(v));
+    v = op(v, dpp_i<0x118, 0xf>(v));
+    v = op(v, dpp_i<0x142, 0xa>(v));  // row_bcast 15 into rows 1 and 3
+    v = op(v, dpp_i<0x143, 0xc>(v));  // row_bcast 31 into rows 2 and 3
+    return __builtin_amdgcn_readlane(v, kWave - 1);
+}
+__device__ __forceinline__ int wave_min_u(int v)
+{
+    return wave_reduce_u(v, [](int a, int b) { return a < b ? a : b; });
+}
+__device__ __forceinline__ int wave_max_u(int v)
+{
+    return wave_reduce_u(v, [](int a, int b) { return a > b ? a : b; });
+}
+
 __device__ __forceinline__ int wave_max_i(int v)
 {
 #pragma unroll
@@ -239,6 +310,32 @@ __device__ __forceinline__ int2 line_rows(const int *bbox, int n, int col, float
     return int2{(int)ceil(lo), (int)floor(hi)};
 }
 
+// Rows of a line whose sample position lies inside the image with a margin of
+// 0.05 pixels, far above the rounding of the positions and of this bound
+// (below 0.005 for n <= 2730): their samples need no bounds test.  [lo, hi]
+// (lo > hi: none), not clipped to [0, n).
+__device__ __forceinline__ int2 inside_rows(int n, int col, float c, float s)
+{
+    const float o = (float)(n - 1) * 0.5f, px = (float)col - o;
+    const float a = 0.05f - o, b = o - 0.05f;  // bounds of position - o
+    float lo = -1e6f, hi = 1e6f;
+    auto slab = [&](float base, float slope) {
+        if (fabsf(slope) < 1e-6f) {
+            // the position moves by less than 0.003 over the line
+            if (!(base >= a + 0.01f && base <= b - 0.01f))
+                hi = -2e6f;
+            return;
+        }
+        const float inv = 1.0f / slope;
+        const float p = (a - base) * inv, q = (b - base) * inv;
+        lo = fmaxf(lo, fminf(p, q));
+        hi = fminf(hi, fmaxf(p, q));
+    };
+    slab(px * c, s);
+    slab(-px * s, c);
+    return int2{(int)ceilf(lo + o), (int)floorf(hi + o)};
+}
+
 // Outputs in global memory, typed so (pointers from a batch descriptor are
 // generic): their stores and loads are global, not flat, operations.
 typedef float __attribute__((address_space(1))) *gf32;
@@ -277,12 +374,19 @@ struct LineDst {
 // the line alone, so the 64-step blocks of pass 2 (v in [64 k, 64 k + 64))
 // hold the same rows of a line whatever other lines share its wave: the
 // results of a line do not depend on the tile that computes it.  Steps run
-// from G, the smallest first row plus skew in the wave, in groups of 8: slot
-// j of the stride-8 accumulators takes the rows of steps G + 8k + j, i.e.
-// Eigen's accumulator (j + G - d) mod 8, and the slots are rotated back
-// after the pass.  Rows outside [0, n) (and outside [0, a8) for the stride-8
-// accumulators) are masked; a group all of whose lanes are inside skips the
-// masks.
+// from G, the smallest first row plus skew in the wave rounded down to a
+// multiple of 8, in groups of 8: slot j of the stride-8 accumulators takes
+// the rows of steps 8k + j, i.e. Eigen's accumulator (j - d) mod 8, and the
+// slots are rotated back after the pass.  Rows outside [0, n) (and outside
+// [0, a8) for the stride-8 accumulators) are masked and positions outside
+// the image tested; a group all of whose lanes are inside (steps [va, vb),
+// nearly all of them) does neither.  The schedule's bounds are wave-uniform
+// scalars, so the loops run on the scalar unit.
+//
+// The groups whose samples need no test load four rows ahead of the four
+// they work on, so that a wave that is nearly alone on its SIMD (a small
+// image) does not wait for each load: the samples of two half groups
+// alternate in two register sets.
 //
 // With CK, pass 1 also runs the median walks' sequential prefixes (the
 // same float additions in the same row order as the walk) and stores them
@@ -295,12 +399,23 @@ struct LineDst {
 // the steps from there on.  A negative or NaN sample (S of the square roots
 // NaN, or a negative minimum) keeps the full walk.  [lo, hi] is the lane's
 // row range that can hold non-zero samples (lo > hi: none).
+//
+// Pass 2 goes by the same groups.  While some lane has not passed its tests,
+// a group's eight samples are walked first (branch-free: the median is a
+// select of the row), and its integrals taken only if some lane has passed
+// by the group's end; rows before a lane's median enter with distance 0.
+// Once every lane has passed, a row is its sample and the multiply-adds.
+//
+// T0..T5 of 1449^2 pixels at 360 angles: 1500 -> TIME us, and of 93^2 pixels
+// at 180 angles, one wave per three SIMDs, 58 -> TIME us; bound by VALU issue
+// (about 24 half-rate slots a row in pass 1, of which the bilinear sample is
+// 14; adds and multiplies issue twice as fast as the rest on this chip).
 template <bool TR, bool NEED_X, bool NEED_S, bool DO345, bool CK, bool FS>
-__device__ __forceinline__ void sino_line(const LineDst &p, const float *src,
+__device__ __forceinline__ void sino_line(const LineDst &p, const float2 *src,
                                           const float2 *s_tab, int a, int col,
                                           bool active, float c, float s, int lo, int hi)
 {
-    const int n = p.n;
+    const int n = __builtin_amdgcn_readfirstlane(p.n);
     src = uniform_ptr(src);
     const float o = (float)((n - 1) / 2.0);
     const float lim = (float)(n - 1);
@@ -309,21 +424,53 @@ __device__ __forceinline__ void sino_line(const LineDst &p, const float *src,
     const float pxns = px * (-s);
     const size_t line = (size_t)a * n + col;
     const size_t plane = (size_t)p.A * n;
-    constexpr int kNone = 1 << 30;
+    constexpr int kNone = 1 << 28;
 
     // ---- schedule --------------------------------------------------------
     int dl = (int)rintf((float)col * (fabsf(c) > fabsf(s) ? -s / c : c / s));
-    dl -= wave_min_i(dl) & ~63;
-    const int dmin = wave_min_i(dl), dmax = wave_max_i(dl);
+    dl -= wave_min_u(dl) & ~63;
     const int ncap = sino_ckpt_blocks(n);
     const int a8 = n & ~7;
     const int a4 = n & ~3;
     const int r0 = lo > 0 ? lo : 0;
     const int r1 = hi + 1 < n ? hi + 1 : n;
     const bool any = active && r1 > r0;  // the lanes past the last column follow it
-    const int G = wave_min_i(any ? r0 + dl : kNone);
-    const int V1 = wave_max_i(any ? (r1 < a8 ? r1 : a8) + dl : -kNone);
-    const int V2 = wave_max_i(any ? r1 + dl : -kNone);
+    const int G = wave_min_u(any ? r0 + dl : kNone) & ~7;
+    const int V = wave_max_u(any ? r1 + dl : -kNone);
+    const int V1 = wave_max_u(any ? (r1 < a8 ? r1 : a8) + dl : -kNone);
+    const int2 ins = inside_rows(n, col, c, s);
+    const int va = (wave_max_u((ins.x > 0 ? ins.x : 0) + dl) + 7) & ~7;
+    const int vb1 = (wave_min_u((ins.y + 1 < a8 ? ins.y + 1 : a8) + dl)) & ~7;  // pass 1
+    const int vb2 = (wave_min_u((ins.y + 1 < n ? ins.y + 1 : n) + dl)) & ~7;    // pass 2
+
+    auto load = [&](auto chk, float py) {
+        return rot_load<TR, decltype(chk)::value>(src, n, lim, o, pxc, pxns, c, s, py);
+    };
+    struct Half {
+        Tap t[4];
+    };
+    // samples of the steps v .. v + 3, untested
+    auto load_half = [&](int v) {
+        Half h;
+        const float py0 = (float)(v - dl) - o;
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            h.t[j] = load(std::false_type{}, py0 + (float)j);
+        return h;
+    };
+    // the eight samples of the group from step v, tested and with the rows
+    // outside [0, n) zero
+    auto load_masked = [&](int v, float *x) {
+        const int rb = v - dl;
+        const float py0 = (float)rb - o;
+        Tap t[8];
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+            t[j] = load(std::true_type{}, py0 + (float)j);
+#pragma unroll
+        for (int j = 0; j < 8; j++)
+            x[j] = (unsigned)(rb + j) < (unsigned)n ? rot_value<TR, true>(t[j]) : 0.0f;
+    };
 
     // ---- pass 1: Eigen-order sums -------------------------------------
     float rx[8], rs[8];
@@ -334,43 +481,53 @@ __device__ __forceinline__ void sino_line(const LineDst &p, const float *src,
     }
     constexpr bool WALK = CK && (NEED_X || NEED_S);
     float cx = 0.0f, cs = 0.0f, vmin = 0.0f;  // walk prefixes, smallest sample
-    // one group of 8 steps from step v (MASK: some lane has a row outside
-    // [0, a8)); row coordinates py = row - o are integers or half-integers
-    // far below 2^23, so stepping them by whole rows is exact
-    auto group = [&](auto mask_c, int v) {
-        constexpr bool MASK = decltype(mask_c)::value;
-        const int rb = v - dl;
-        const float py0 = (float)rb - o;
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-            float x = rot_sample<TR>(src, n, lim, o, pxc, pxns, c, s, py0 + (float)j);
-            bool chain = true;
-            if constexpr (MASK) {
-                x = (unsigned)(rb + j) < (unsigned)n ? x : 0.0f;
-                chain = (unsigned)(rb + j) < (unsigned)a8;
-            }
-            const float sv = NEED_S ? line_sqrt<FS>(x) : 0.0f;
-            rx[j] += chain ? x : 0.0f;
-            if (NEED_S)
-                rs[j] += chain ? sv : 0.0f;
-            if (WALK && NEED_X)
-                cx += x;
-            if (WALK && NEED_S)
-                cs += sv;
-            if (WALK && !NEED_S)
-                vmin = fminf(vmin, x);
-        }
+    auto add = [&](int j, float x, bool chain) {
+        const float sv = NEED_S ? line_root<FS>(x) : 0.0f;
+        rx[j] += chain ? x : 0.0f;
+        if (NEED_S)
+            rs[j] += chain ? sv : 0.0f;
+        if (WALK && NEED_X)
+            cx += x;
+        if (WALK && NEED_S)
+            cs += sv;
+        if (WALK && !NEED_S)
+            vmin = fminf(vmin, x);
     };
-    for (int v = G; v < V1; v += 8) {
-        if (WALK && v > G && ((v - G) & 63) == 0 && active && (v - G) / 64 <= ncap)
+    auto checkpoint = [&](int v) {
+        if (WALK && v > G && ((v - G) & 63) == 0 && (v - G) / 64 <= ncap && active)
             p.ckpt[(size_t)((v - G) / 64 - 1) * plane + line] = f2v{cx, cs};
-        if (v >= dmax && v + 8 - dmin <= a8)
-            group(std::false_type{}, v);
-        else
-            group(std::true_type{}, v);
+    };
+    // row coordinates py = row - o are integers or half-integers far below
+    // 2^23, so stepping them by whole rows is exact
+    for (int v = G; v < V1;) {
+        if (v >= va && v < vb1) {
+            const int ve = V1 < vb1 ? (V1 + 7) & ~7 : vb1;
+            const int vl = ve < vb1 ? ve : vb1;  // groups up to here are untested
+            Half h0 = load_half(v);
+            for (; v < vl; v += 8) {
+                checkpoint(v);
+                Half h1 = load_half(v + 4);
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    add(j, rot_value<TR, false>(h0.t[j]), true);
+                // (the last group loads its own rows again)
+                h0 = load_half(v + 8 < vl ? v + 8 : v);
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    add(4 + j, rot_value<TR, false>(h1.t[j]), true);
+            }
+        } else {
+            checkpoint(v);
+            float x[8];
+            load_masked(v, x);
+#pragma unroll
+            for (int j = 0; j < 8; j++)
+                add(j, x[j], (unsigned)(v - dl + j) < (unsigned)a8);
+            v += 8;
+        }
     }
-    // slot j holds accumulator (j + d) mod 8: rotate it back
-    const int d = (G - dl) & 7;
+    // slot j holds accumulator (j - d) mod 8: rotate it back
+    const int d = (0 - dl) & 7;
 #pragma unroll
     for (int b = 1; b < 8; b <<= 1) {
         const bool on = (d & b) != 0;
@@ -386,6 +543,9 @@ __device__ __forceinline__ void sino_line(const LineDst &p, const float *src,
             rs[m] = ts[m];
         }
     }
+    // rows from a8 on: all zero samples (which change no sum) unless some
+    // line of the wave has non-zero rows there
+    const bool tail = n < 8 || wave_max_u(r1) > a8;
     float Sx, Ss;
     if (a4 == 0) {
         Sx = 0.0f;
@@ -395,7 +555,7 @@ __device__ __forceinline__ void sino_line(const LineDst &p, const float *src,
                                            (float)r - o);
             Sx = r == 0 ? v : Sx + v;
             if (NEED_S)
-                Ss = r == 0 ? line_sqrt<FS>(v) : Ss + line_sqrt<FS>(v);
+                Ss = r == 0 ? line_root<FS>(v) : Ss + line_root<FS>(v);
         }
     } else {
         float ax[4], as[4];
@@ -404,12 +564,12 @@ __device__ __forceinline__ void sino_line(const LineDst &p, const float *src,
             ax[j] = rx[j] + rx[j + 4];
             as[j] = rs[j] + rs[j + 4];
         }
-        if (a4 > a8) {
+        if (a4 > a8 && tail) {
 #pragma unroll
             for (int j = 0; j < 4; j++) {
                 const float v = rot_sample<TR>(src, n, lim, o, pxc, pxns, c, s,
                                                (float)(a8 + j) - o);
-                const float sv = NEED_S ? line_sqrt<FS>(v) : 0.0f;
+                const float sv = NEED_S ? line_root<FS>(v) : 0.0f;
                 if (n >= 8) {
                     ax[j] += v;
                     as[j] += sv;
@@ -421,12 +581,12 @@ __device__ __forceinline__ void sino_line(const LineDst &p, const float *src,
         }
         Sx = (ax[0] + ax[2]) + (ax[1] + ax[3]);
         Ss = (as[0] + as[2]) + (as[1] + as[3]);
-        for (int r = a4; r < n; r++) {
+        for (int r = a4; tail && r < n; r++) {
             const float v = rot_sample<TR>(src, n, lim, o, pxc, pxns, c, s,
                                            (float)r - o);
             Sx += v;
             if (NEED_S)
-                Ss += line_sqrt<FS>(v);
+                Ss += line_root<FS>(v);
         }
     }
 
@@ -445,40 +605,33 @@ __device__ __forceinline__ void sino_line(const LineDst &p, const float *src,
         int nck = V1 > G ? (V1 - G - 1) / 64 : 0;
         nck = nck < ncap ? nck : ncap;
         int b0 = 0;
-        float2 cb = {0.0f, 0.0f};
-        if (nck > 0 && !__ballot(active && bad)) {
-            for (int b = 1; b <= nck; b += 4) {
-                float2 ck[4];
+        if (nck > 0 && !__builtin_amdgcn_ballot_w64(active && bad)) {
+            for (int b = 1; b <= nck; b += 8) {
+                f2v ck[8];
 #pragma unroll
-                for (int u = 0; u < 4; u++)
-                    if (b + u <= nck)
-                    {
-                        const f2v cv = p.ckpt[(size_t)(b + u - 1) * plane + line];
-                        ck[u] = float2{cv.x, cv.y};
-                    }
+                for (int u = 0; u < 8; u++) {
+                    // (a block past the last reads the last again)
+                    const int bu = b + u <= nck ? b + u : nck;
+                    ck[u] = active ? p.ckpt[(size_t)(bu - 1) * plane + line] : f2v{0.0f, 0.0f};
+                }
                 bool stop = false;
 #pragma unroll
-                for (int u = 0; u < 4; u++) {
-                    if (stop || b + u > nck)
-                        break;
+                for (int u = 0; u < 8; u++) {
                     const bool pass = (NEED_X && 2.0f * ck[u].x >= Sx) ||
                                       (NEED_S && 2.0f * ck[u].y >= Ss);
-                    if (__ballot(active && pass)) {
-                        stop = true;
-                    } else {
+                    stop = stop || b + u > nck ||
+                           __builtin_amdgcn_ballot_w64(active && pass) != 0;
+                    if (!stop) {
                         b0 = b + u;
-                        cb = ck[u];
+                        Px = ck[u].x;
+                        Ps = ck[u].y;
                     }
                 }
                 if (stop)
                     break;
             }
         }
-        if (b0 > 0) {
-            start = G + 64 * b0;
-            Px = cb.x;
-            Ps = cb.y;
-        }
+        start = G + 64 * b0;
     }
 
     // ---- pass 2: median walk + integrals -----------------------------
@@ -492,7 +645,9 @@ __device__ __forceinline__ void sino_line(const LineDst &p, const float *src,
     // lines.
     double t1 = 0.0, t2 = 0.0;
     double r3 = 0.0, i3 = 0.0, r4 = 0.0, i4 = 0.0, r5 = 0.0, i5 = 0.0;
-    int m = -1, sm = -1;
+    float f1 = 0.0f, f2 = 0.0f;
+    float f3r = 0.0f, f3i = 0.0f, f4r = 0.0f, f4i = 0.0f, f5r = 0.0f, f5i = 0.0f;
+    int m = kNone, sm = kNone;  // not passed yet
     const bool do3 = p.slot.s[3] >= 0, do4 = p.slot.s[4] >= 0, do5 = p.slot.s[5] >= 0;
     if (lo > 0 || lo > hi) {
         // the walk's first row is a zero: it passes there iff S <= 0
@@ -501,71 +656,136 @@ __device__ __forceinline__ void sino_line(const LineDst &p, const float *src,
         if (NEED_S && 2.0f * 0.0f >= Ss)
             sm = 0;
     }
-    for (int vb = start, ve; vb < V2; vb = ve) {
-        ve = (vb & ~63) + 64;
-        ve = ve < V2 ? ve : V2;
-        // every lane's rows of the block inside [0, n)
-        const bool full = vb >= dmax && ve - dmin <= n;
-        float f1 = 0.0f, f2 = 0.0f;
-        float f3r = 0.0f, f3i = 0.0f, f4r = 0.0f, f4i = 0.0f, f5r = 0.0f, f5i = 0.0f;
-        int r = vb - dl;
-        float py = (float)r - o;
-        for (int v = vb; v < ve; v++, r++, py += 1.0f) {
-            if (!full && (unsigned)r >= (unsigned)n)
-                continue;
-            const float x = rot_sample<TR>(src, n, lim, o, pxc, pxns, c, s, py);
-            if (NEED_X) {
-                if (m < 0) {
-                    Px += x;
-                    if (2.0f * Px >= Sx)
-                        m = r;
-                }
-                if (m >= 0) {
-                    const float rr = (float)(r - m);
-                    const float vr = x * rr;
-                    f1 += vr;
-                    f2 = fmaf(vr, rr, f2);
-                }
-            }
-            if (NEED_S) {
-                if (sm < 0) {
-                    Ps += line_sqrt<FS>(x);
-                    if (2.0f * Ps >= Ss)
-                        sm = r;
-                } else if (DO345) {
-                    // one 16-byte and one 8-byte LDS read per row for all three
-                    // tables (rows interleaved by the kernel prologue)
-                    const int q = r - sm;
-                    const float4 w34 = reinterpret_cast<const float4 *>(s_tab)[q];
-                    const float2 w5 = s_tab[2 * p.tabn + q];
-                    if (do3) {
-                        f3r = fmaf(w34.x, x, f3r);
-                        f3i = fmaf(w34.y, x, f3i);
-                    }
-                    if (do4) {
-                        f4r = fmaf(w34.z, x, f4r);
-                        f4i = fmaf(w34.w, x, f4i);
-                    }
-                    if (do5) {
-                        f5r = fmaf(w5.x, x, f5r);
-                        f5i = fmaf(w5.y, x, f5i);
-                    }
-                }
-            }
+    if (!active)  // a copy of another lane's line: nothing waits for it
+        m = sm = 0;
+    const float4 *tab34 = reinterpret_cast<const float4 *>(s_tab);
+    const float2 *tab5 = s_tab + 2 * p.tabn;
+    // T1/T2 and T3..T5 of one row: its sample, distance from the x-median and
+    // table rows at the distance from the root median (zero at distance 0)
+    auto integrate12 = [&](float x, float rr) {
+        const float vr = x * rr;
+        f1 += vr;
+        f2 = fmaf(vr, rr, f2);
+    };
+    // (all three, whichever are stored: a test per row costs more)
+    auto integrate345 = [&](float x, float4 w34, float2 w5) {
+        f3r = fmaf(w34.x, x, f3r);
+        f3i = fmaf(w34.y, x, f3i);
+        f4r = fmaf(w34.z, x, f4r);
+        f4i = fmaf(w34.w, x, f4i);
+        f5r = fmaf(w5.x, x, f5r);
+        f5i = fmaf(w5.y, x, f5i);
+    };
+    auto flush = [&] {
+        if (NEED_X) {
+            t1 += f1;
+            t2 += f2;
+            f1 = f2 = 0.0f;
         }
-        t1 += f1;
-        t2 += f2;
-        r3 += f3r;
-        i3 += f3i;
-        r4 += f4r;
-        i4 += f4i;
-        r5 += f5r;
-        i5 += f5i;
+        if (DO345) {
+            r3 += f3r;
+            i3 += f3i;
+            r4 += f4r;
+            i4 += f4i;
+            r5 += f5r;
+            i5 += f5i;
+            f3r = f3i = f4r = f4i = f5r = f5i = 0.0f;
+        }
+    };
+    bool done = false;  // every lane has passed (wave-uniform)
+    for (int v = start; v < V;) {
+        const bool plain = v >= va && v < vb2;
+        if (plain && done) {
+            // the untested groups up to the end of this 64-step block
+            int ve = (v & ~63) + 64;
+            ve = ve < vb2 ? ve : vb2;
+            ve = ve < V ? ve : (V + 7) & ~7;
+            const int rb = v - dl;
+            float rr = (float)(rb - m);
+            const float4 *w34 = tab34 + (rb - sm);
+            const float2 *w5 = tab5 + (rb - sm);
+            auto use = [&](const Half &h, int base) {
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const float x = rot_value<TR, false>(h.t[j]);
+                    if (NEED_X) {
+                        integrate12(x, rr);
+                        rr += 1.0f;
+                    }
+                    if (DO345)
+                        integrate345(x, w34[base + j], w5[base + j]);
+                }
+            };
+            Half h0 = load_half(v);
+            for (; v < ve; v += 8) {
+                Half h1 = load_half(v + 4);
+                use(h0, 0);
+                h0 = load_half(v + 8 < ve ? v + 8 : v);
+                use(h1, 4);
+                w34 += 8;
+                w5 += 8;
+            }
+        } else {
+            float x[8];
+            if (plain) {
+                const Half h0 = load_half(v), h1 = load_half(v + 4);
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    x[j] = rot_value<TR, false>(h0.t[j]);
+                    x[4 + j] = rot_value<TR, false>(h1.t[j]);
+                }
+            } else {
+                load_masked(v, x);
+            }
+            const int rb = v - dl;
+            if (!done) {
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    const int r = rb + j;
+                    const bool row = (unsigned)r < (unsigned)n;
+                    if (NEED_X) {
+                        Px += x[j];
+                        m = row && m == kNone && 2.0f * Px >= Sx ? r : m;
+                    }
+                    if (NEED_S) {
+                        Ps += line_root<FS>(x[j]);
+                        sm = row && sm == kNone && 2.0f * Ps >= Ss ? r : sm;
+                    }
+                }
+            }
+            const bool passed = (NEED_X && m != kNone) || (NEED_S && sm != kNone);
+            if (__builtin_amdgcn_ballot_w64(active && passed)) {
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    const int r = rb + j;
+                    if (NEED_X)
+                        integrate12(x[j], (float)(r > m ? r - m : 0));
+                    if (DO345) {
+                        int q = r - sm;
+                        const float xq = q > 0 ? x[j] : 0.0f;
+                        q = q > 0 ? q : 0;
+                        q = q < n ? q : 0;  // a row past the last: sample 0
+                        integrate345(xq, tab34[q], tab5[q]);
+                    }
+                }
+            }
+            if (!done)
+                done = !__builtin_amdgcn_ballot_w64((NEED_X && m == kNone) ||
+                                                    (NEED_S && sm == kNone));
+            v += 8;
+        }
+        if ((v & 63) == 0)
+            flush();
     }
-    if (m < 0)
+    flush();
+    if (m == kNone) {
         m = n - 1;
-    if (sm < 0)
+        t1 = t2 = 0.0;
+    }
+    if (sm == kNone) {
         sm = n - 1;
+        r3 = i3 = r4 = i4 = r5 = i5 = 0.0;
+    }
     if (!active)
         return;
     if (NEED_X && p.med_x)
@@ -595,8 +815,8 @@ __device__ __forceinline__ void sino_line(const LineDst &p, const float *src,
 // One line, with the image copy whose fast axis the lanes step along (TR)
 // and the square root the image's bounding-box flag allows (FS).
 template <bool NEED_X, bool NEED_S, bool DO345, bool CK>
-__device__ __forceinline__ void sino_line_any(const LineDst &dst, const float *img,
-                                              const float *imgT, const int *bbox,
+__device__ __forceinline__ void sino_line_any(const LineDst &dst, const float2 *pair,
+                                              const float2 *pairT, const int *bbox,
                                               const float2 *s_tab, int a, int col,
                                               bool active, float2 cs, int lo, int hi)
 {
@@ -604,16 +824,16 @@ __device__ __forceinline__ void sino_line_any(const LineDst &dst, const float *i
     const bool tr = __builtin_amdgcn_readfirstlane(fabsf(cs.x) > fabsf(cs.y));
     const bool fs = bbox && bbox[4] == 0;
     if (tr && fs)
-        sino_line<true, NEED_X, NEED_S, DO345, CK, true>(dst, imgT, s_tab, a, col, active,
+        sino_line<true, NEED_X, NEED_S, DO345, CK, true>(dst, pairT, s_tab, a, col, active,
                                                          cs.x, cs.y, lo, hi);
     else if (tr)
-        sino_line<true, NEED_X, NEED_S, DO345, CK, false>(dst, imgT, s_tab, a, col, active,
+        sino_line<true, NEED_X, NEED_S, DO345, CK, false>(dst, pairT, s_tab, a, col, active,
                                                           cs.x, cs.y, lo, hi);
     else if (fs)
-        sino_line<false, NEED_X, NEED_S, DO345, CK, true>(dst, img, s_tab, a, col, active,
+        sino_line<false, NEED_X, NEED_S, DO345, CK, true>(dst, pair, s_tab, a, col, active,
                                                           cs.x, cs.y, lo, hi);
     else
-        sino_line<false, NEED_X, NEED_S, DO345, CK, false>(dst, img, s_tab, a, col, active,
+        sino_line<false, NEED_X, NEED_S, DO345, CK, false>(dst, pair, s_tab, a, col, active,
                                                            cs.x, cs.y, lo, hi);
 }
 
@@ -652,7 +872,7 @@ __global__ __launch_bounds__(kBlock) void sino_t05_kernel(SinoParams p)
     const float2 cs = p.trig[a];
     const LineDst dst = {p.sino, p.med_x, p.med_s, p.z345, p.ckpt, p.n, p.A, p.n, p.slot};
     const int2 rows = line_rows(p.bbox, p.n, col, cs.x, cs.y);
-    sino_line_any<NEED_X, NEED_S, DO345, true>(dst, p.img, p.imgT, p.bbox, s_tab, a, col,
+    sino_line_any<NEED_X, NEED_S, DO345, true>(dst, p.pair, p.pairT, p.bbox, s_tab, a, col,
                                                active, cs, rows.x, rows.y);
 }
 
@@ -670,7 +890,7 @@ __global__ __launch_bounds__(kBlock) void sino_t05_kernel(SinoParams p)
 // not depend on the tile.
 // ---------------------------------------------------------------------------
 template <bool NEED_X, bool NEED_S, bool DO345>
-__global__ __launch_bounds__(kBlock) void sino_t05_batched_kernel(BatchSinoParams p)
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void sino_t05_batched_kernel(BatchSinoParams p)
 {
     extern __shared__ __align__(16) float2 s_tab[];
     if (DO345) {
@@ -719,7 +939,7 @@ __global__ __launch_bounds__(kBlock) void sino_t05_batched_kernel(BatchSinoParam
         const LineDst dst = {im.sino, im.med_x, im.med_s, im.z345, im.ckpt, im.n, p.A, p.tabn,
                              p.slot};
         const int2 rows = line_rows(im.bbox, im.n, col, cs.x, cs.y);
-        sino_line_any<NEED_X, NEED_S, DO345, true>(dst, im.img, im.imgT, im.bbox, s_tab, a,
+        sino_line_any<NEED_X, NEED_S, DO345, true>(dst, im.pair, im.pairT, im.bbox, s_tab, a,
                                                    col, active, cs, rows.x, rows.y);
     }
 }
@@ -736,55 +956,142 @@ __global__ void reset_counters_kernel(unsigned int *c, int count)
         c[threadIdx.x] = 0u;
 }
 
-// Row-major copies of every image of a batch: grid.y walks the images.
-__global__ __launch_bounds__(kBlock) void transpose_batched_kernel(
-    const BatchImage *images)
+// The pixel pairs of an n x n column-major image and the box of its non-zero
+// pixels (launch_image_pairs): block `block` of nblocks takes 32 x 32 tiles
+// through LDS (33 x 33, the pairs' second pixels included) and leaves its
+// box in box[0..4].
+__device__ __forceinline__ void image_pairs_block(const float *img, int n, float2 *pair,
+                                                  float2 *pairT, int block, int nblocks,
+                                                  int *box)
 {
-    __shared__ float tile[32][33];
-    const BatchImage im = images[blockIdx.y];
-    const int n = im.n;
+    __shared__ float tile[33][35];
+    __shared__ int s_b[5][kBlock / kWave];
     const int tiles = (n + 31) / 32;
-    float *out = const_cast<float *>(im.imgT);
-    for (int t = blockIdx.x; t < tiles * tiles; t += gridDim.x) {
+    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+    int x0 = n, x1 = -1, y0 = n, y1 = -1;
+    bool narrow = false;  // a pixel that is not 0 or in [2^-45, 2^120]
+    for (int t = block; t < tiles * tiles; t += nblocks) {
         const int bx = (t % tiles) * 32, by = (t / tiles) * 32;
-        const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+        for (int i = threadIdx.x; i < 33 * 33; i += kBlock) {
+            const int k = i / 33, r = i - 33 * k;
+            const int col = bx + k, row = by + r;
+            const bool in = col < n && row < n;
+            const float v = in ? img[(size_t)col * n + row] : 0.0f;
+            tile[k][r] = v;
+            narrow = narrow || !(v == 0.0f || (v >= 0x1p-45f && v <= 0x1p120f));
+            if (v != 0.0f) {
+                x0 = col < x0 ? col : x0;
+                x1 = col > x1 ? col : x1;
+                y0 = row < y0 ? row : y0;
+                y1 = row > y1 ? row : y1;
+            }
+        }
+        __syncthreads();
+#pragma unroll
         for (int k = ty; k < 32; k += 8) {
             const int col = bx + k, row = by + tx;
             if (col < n && row < n)
-                tile[k][tx] = im.img[(size_t)col * n + row];
-        }
-        __syncthreads();
-        for (int k = ty; k < 32; k += 8) {
-            const int row = by + k, col = bx + tx;
-            if (col < n && row < n)
-                out[(size_t)row * n + col] = tile[tx][k];
+                pair[(size_t)col * n + row] = float2{tile[k][tx], tile[k + 1][tx]};
+            const int rowT = by + k, colT = bx + tx;
+            if (colT < n && rowT < n)
+                pairT[(size_t)rowT * n + colT] = float2{tile[tx][k], tile[tx][k + 1]};
         }
         __syncthreads();
     }
-}
-
-// ---------------------------------------------------------------------------
-// Helpers: transpose (for the row-major copy) and pad.
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(kBlock) void transpose_kernel(const float *in,
-                                                           float *out, int n)
-{
-    __shared__ float tile[32][33];
-    const int bx = blockIdx.x * 32, by = blockIdx.y * 32;
-    const int tx = threadIdx.x & 31, ty = threadIdx.x >> 5;  // 32 x 8
-    for (int k = ty; k < 32; k += 8) {
-        const int col = bx + k, row = by + tx;
-        if (col < n && row < n)
-            tile[k][tx] = in[(size_t)col * n + row];
+    if (block == 0 && threadIdx.x < 2) {  // what a sample's second pair may load
+        pair[(size_t)n * n + threadIdx.x] = float2{0.0f, 0.0f};
+        pairT[(size_t)n * n + threadIdx.x] = float2{0.0f, 0.0f};
+    }
+    x0 = wave_min_i(x0);
+    x1 = wave_max_i(x1);
+    y0 = wave_min_i(y0);
+    y1 = wave_max_i(y1);
+    const int nw = __ballot(narrow) != 0;
+    const int w = threadIdx.x / kWave;
+    if ((threadIdx.x & (kWave - 1)) == 0) {
+        s_b[0][w] = x0;
+        s_b[1][w] = x1;
+        s_b[2][w] = y0;
+        s_b[3][w] = y1;
+        s_b[4][w] = nw;
     }
     __syncthreads();
-    for (int k = ty; k < 32; k += 8) {
-        const int row = by + k, col = bx + tx;
-        if (col < n && row < n)
-            out[(size_t)row * n + col] = tile[tx][k];
+    if (threadIdx.x == 0) {
+        int nr = s_b[4][0];
+        for (int k = 1; k < kBlock / kWave; k++) {
+            x0 = s_b[0][k] < x0 ? s_b[0][k] : x0;
+            x1 = s_b[1][k] > x1 ? s_b[1][k] : x1;
+            y0 = s_b[2][k] < y0 ? s_b[2][k] : y0;
+            y1 = s_b[3][k] > y1 ? s_b[3][k] : y1;
+            nr |= s_b[4][k];
+        }
+        box[0] = x0;
+        box[1] = x1;
+        box[2] = y0;
+        box[3] = y1;
+        box[4] = nr;
     }
 }
 
+// bb[0..4] = the union of the blocks' boxes at bb + 8 (1 + block), by one wave.
+__device__ __forceinline__ void image_box_reduce(int n, int nblocks, int *bb)
+{
+    const int lane = threadIdx.x & (kWave - 1);
+    int x0 = n, x1 = -1, y0 = n, y1 = -1, nr = 0;
+    for (int k = lane; k < nblocks; k += kWave) {
+        const int *b = bb + 8 * (1 + k);
+        x0 = b[0] < x0 ? b[0] : x0;
+        x1 = b[1] > x1 ? b[1] : x1;
+        y0 = b[2] < y0 ? b[2] : y0;
+        y1 = b[3] > y1 ? b[3] : y1;
+        nr |= b[4];
+    }
+    x0 = wave_min_i(x0);
+    x1 = wave_max_i(x1);
+    y0 = wave_min_i(y0);
+    y1 = wave_max_i(y1);
+    const int narrow = __ballot(nr != 0) != 0;
+    if (lane == 0) {
+        bb[0] = x0;
+        bb[1] = x1;
+        bb[2] = y0;
+        bb[3] = y1;
+        bb[4] = narrow;
+    }
+}
+
+__global__ __launch_bounds__(kBlock) void image_pairs_kernel(const float *img, int n,
+                                                             float2 *pair, float2 *pairT,
+                                                             int *bb)
+{
+    image_pairs_block(img, n, pair, pairT, blockIdx.x, gridDim.x, bb + 8 * (1 + blockIdx.x));
+}
+
+__global__ void image_box_kernel(int n, int nblocks, int *bb)
+{
+    image_box_reduce(n, nblocks, bb);
+}
+
+// Every image of a batch: grid.y walks the images.
+__global__ __launch_bounds__(kBlock) void image_pairs_batched_kernel(const BatchImage *images)
+{
+    const BatchImage &im = images[blockIdx.y];
+    image_pairs_block(im.img, im.n, im.pair, im.pairT, blockIdx.x, gridDim.x,
+                      im.bbox + 8 * (1 + blockIdx.x));
+}
+
+__global__ void image_box_batched_kernel(const BatchImage *images, int nblocks,
+                                         unsigned int *counter)
+{
+    const BatchImage &im = images[blockIdx.x];
+    image_box_reduce(im.n, nblocks, im.bbox);
+    if (blockIdx.x == 0 && threadIdx.x == 0)
+        *counter = 0u;
+}
+
+// ---------------------------------------------------------------------------
+// Helper: pad.
+// ---------------------------------------------------------------------------
 __global__ __launch_bounds__(kBlock) void pad_kernel(const float *in, int rows,
                                                      int cols, float *out,
                                                      int n, int dfx, int dfy)
@@ -1834,7 +2141,7 @@ __device__ __forceinline__ bool sort_line(const SortTParams &p, int line, int wh
     const float px = (float)col - o;
     const float pxc = px * cs.x, pxns = px * (-cs.y);
     const bool tr = fabsf(cs.y) > fabsf(cs.x);
-    const float *src = tr ? p.imgT : p.img;
+    const float2 *src = tr ? p.pairT : p.pair;
     const bool t6 = which == 0;
     const int base = t6 ? p.med_s[line] : p.med_x[line];
     const int L = n - base;
@@ -1909,7 +2216,7 @@ __device__ __forceinline__ int sort_pair(const SortTParams &p, int line, float *
     const float px = (float)col - o;
     const float pxc = px * cs.x, pxns = px * (-cs.y);
     const bool tr = fabsf(cs.y) > fabsf(cs.x);
-    const float *src = tr ? p.imgT : p.img;
+    const float2 *src = tr ? p.pairT : p.pair;
     const int sm = p.med_s[line], m = p.med_x[line];
     const bool fs = p.bbox && p.bbox[4] == 0;  // short square roots (line_sqrt)
     const int L6 = n - sm, L7 = n - m;
@@ -2927,101 +3234,6 @@ __global__ __launch_bounds__(kBlock) void to_float_batched_kernel(const double *
     }
 }
 
-// Bounding box of the non-zero pixels of an n x n column-major image
-// (pixel (row Y, col X) at X * n + Y): bb = {x0, x1, y0, y1}, set to
-// {n, -1, n, -1} beforehand.  Block-local bounds, one atomic each per block.
-// Block b takes columns b, b + nblocks, ...; its threads stride down rows.
-__device__ __forceinline__ void bbox_accumulate(const float *img, int n, int block,
-                                                int nblocks, int *bb)
-{
-    __shared__ int s_b[5][kBlock / kWave];
-    int x0 = n, x1 = -1, y0 = n, y1 = -1;
-    bool narrow = false;  // a pixel below 0 or in (0, 2^-45)
-    for (int X = block; X < n; X += nblocks) {
-        const float *col = img + (size_t)X * n;
-#pragma unroll 4
-        for (int Y = threadIdx.x; Y < n; Y += kBlock) {
-            const float v = col[Y];
-            narrow = narrow || v < 0.0f || (v > 0.0f && v < 0x1p-45f);
-            if (v != 0.0f) {
-                x0 = X < x0 ? X : x0;
-                x1 = X > x1 ? X : x1;
-                y0 = Y < y0 ? Y : y0;
-                y1 = Y > y1 ? Y : y1;
-            }
-        }
-    }
-    x0 = wave_min_i(x0);
-    x1 = wave_max_i(x1);
-    y0 = wave_min_i(y0);
-    y1 = wave_max_i(y1);
-    const int nw = __ballot(narrow) != 0;
-    const int w = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1);
-    if (lane == 0) {
-        s_b[0][w] = x0;
-        s_b[1][w] = x1;
-        s_b[2][w] = y0;
-        s_b[3][w] = y1;
-        s_b[4][w] = nw;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        int nr = s_b[4][0];
-        for (int k = 1; k < kBlock / kWave; k++) {
-            x0 = s_b[0][k] < x0 ? s_b[0][k] : x0;
-            x1 = s_b[1][k] > x1 ? s_b[1][k] : x1;
-            y0 = s_b[2][k] < y0 ? s_b[2][k] : y0;
-            y1 = s_b[3][k] > y1 ? s_b[3][k] : y1;
-            nr |= s_b[4][k];
-        }
-        if (nr)
-            atomicOr(bb + 4, 1);
-        if (x1 >= 0) {
-            atomicMin(bb + 0, x0);
-            atomicMax(bb + 1, x1);
-            atomicMin(bb + 2, y0);
-            atomicMax(bb + 3, y1);
-        }
-    }
-}
-
-__global__ void bbox_init_kernel(int *bb, int n)
-{
-    if (threadIdx.x == 0) {
-        bb[0] = n;
-        bb[1] = -1;
-        bb[2] = n;
-        bb[3] = -1;
-        bb[4] = 0;
-    }
-}
-
-__global__ __launch_bounds__(kBlock) void image_bbox_kernel(const float *img, int n, int *bb)
-{
-    bbox_accumulate(img, n, blockIdx.x, gridDim.x, bb);
-}
-
-__global__ void bbox_init_batched_kernel(const BatchImage *images, int nimg)
-{
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < nimg) {
-        int *bb = const_cast<int *>(images[k].bbox);
-        const int n = images[k].n;
-        bb[0] = n;
-        bb[1] = -1;
-        bb[2] = n;
-        bb[3] = -1;
-        bb[4] = 0;
-    }
-}
-
-// grid.y walks the images
-__global__ __launch_bounds__(kBlock) void image_bbox_batched_kernel(const BatchImage *images)
-{
-    const BatchImage &im = images[blockIdx.y];
-    bbox_accumulate(im.img, im.n, blockIdx.x, gridDim.x, const_cast<int *>(im.bbox));
-}
-
 // out(i, j) = v(i, j) / sqrt(lambda_j) for count column-major k x k matrices
 // (eigenvectors v, eigenvalues lambda, k per matrix).
 __global__ __launch_bounds__(kBlock) void scale_eigvec_kernel(const double *v,
@@ -3155,13 +3367,6 @@ __global__ __launch_bounds__(kBlock) void nos_poly_kernel(const double *S, const
 // ---------------------------------------------------------------------------
 // Launchers
 // ---------------------------------------------------------------------------
-hipError_t launch_transpose(const float *in, float *out, int n, hipStream_t s)
-{
-    dim3 grid((n + 31) / 32, (n + 31) / 32);
-    transpose_kernel<<<grid, kBlock, 0, s>>>(in, out, n);
-    return hipGetLastError();
-}
-
 hipError_t launch_pad(const float *in, int rows, int cols, float *out, int n,
                       int dfx, int dfy, hipStream_t s)
 {
@@ -3269,15 +3474,28 @@ hipError_t launch_circus_batched(const BatchCircusParams &p, hipStream_t s)
     return hipGetLastError();
 }
 
-hipError_t launch_transpose_batched(const BatchImage *d_images, int nimg, int nmax,
-                                    hipStream_t s)
+// Blocks of one image's pair pass: one 32 x 32 tile each up to kPairBlocks.
+static int pair_blocks(int n)
 {
-    const int tiles = (nmax + 31) / 32;
-    int gx = tiles * tiles;
-    if (gx > 1024)
-        gx = 1024;
-    dim3 grid(gx, nimg);
-    transpose_batched_kernel<<<grid, kBlock, 0, s>>>(d_images);
+    const int tiles = (n + 31) / 32;
+    return tiles * tiles < kPairBlocks ? tiles * tiles : kPairBlocks;
+}
+
+hipError_t launch_image_pairs(const float *img, int n, float2 *pair, float2 *pairT, int *bbox,
+                              hipStream_t s)
+{
+    const int blocks = pair_blocks(n);
+    image_pairs_kernel<<<blocks, kBlock, 0, s>>>(img, n, pair, pairT, bbox);
+    image_box_kernel<<<1, kWave, 0, s>>>(n, blocks, bbox);
+    return hipGetLastError();
+}
+
+hipError_t launch_image_pairs_batched(const BatchImage *images, int nimg, int nmax,
+                                      unsigned int *counter, hipStream_t s)
+{
+    const int blocks = pair_blocks(nmax);
+    image_pairs_batched_kernel<<<dim3(blocks, nimg), kBlock, 0, s>>>(images);
+    image_box_batched_kernel<<<nimg, kWave, 0, s>>>(images, blocks, counter);
     return hipGetLastError();
 }
 
@@ -3512,10 +3730,13 @@ static int grid_for(size_t total)
     return (int)(b > 4096 ? 4096 : (b < 1 ? 1 : b));
 }
 
-hipError_t launch_short_sqrt_check(uint32_t lo, uint64_t count, unsigned long long *mism,
-                                   unsigned int *first, hipStream_t s)
+hipError_t launch_short_sqrt_check(bool root, uint32_t lo, uint64_t count,
+                                   unsigned long long *mism, unsigned int *first, hipStream_t s)
 {
-    short_sqrt_check_kernel<<<8192, kBlock, 0, s>>>(lo, count, mism, first);
+    if (root)
+        short_sqrt_check_kernel<true><<<8192, kBlock, 0, s>>>(lo, count, mism, first);
+    else
+        short_sqrt_check_kernel<false><<<8192, kBlock, 0, s>>>(lo, count, mism, first);
     return hipGetLastError();
 }
 
@@ -3543,25 +3764,6 @@ hipError_t launch_column_medians(const float *in, int n, int cols, int32_t *med,
     }
     const size_t shm = sizeof(float) * (((size_t)n + 3) & ~(size_t)3);
     column_median_kernel<<<cols, kBlock, shm, s>>>(in, n, med);
-    return hipGetLastError();
-}
-
-hipError_t launch_image_bbox(const float *img, int n, int *bbox, hipStream_t s)
-{
-    bbox_init_kernel<<<1, kWave, 0, s>>>(bbox, n);
-    // few blocks: each ends with up to five atomics on the same words, which
-    // serialise (256 blocks took 13.8 us on a 363 x 363 image, 64 take 7);
-    // large images keep 256 so that each thread's strided loop stays short
-    const int nb = n <= 512 ? (n < 64 ? n : 64) : 256;
-    image_bbox_kernel<<<nb, kBlock, 0, s>>>(img, n, bbox);
-    return hipGetLastError();
-}
-
-hipError_t launch_image_bbox_batched(const BatchImage *images, int nimg, int nmax,
-                                     hipStream_t s)
-{
-    bbox_init_batched_kernel<<<(nimg + kBlock - 1) / kBlock, kBlock, 0, s>>>(images, nimg);
-    image_bbox_batched_kernel<<<dim3(nmax < 64 ? nmax : 64, nimg), kBlock, 0, s>>>(images);
     return hipGetLastError();
 }
 
