@@ -1,0 +1,71 @@
+"""GPU tests of the wave sort behind P2, T6 and T7 at its edges: every network
+width (64 keys and powers of two up to 2048) from one row short to one row
+over, signed values, ties, both zeros, infinities, and NaN columns.  Ranks
+and values are the oracle's exactly; a column with a NaN has a NaN sum, which
+no prefix reaches: the last position, its value the largest with a positive
+NaN above everything.
+"""
+import numpy as np
+import pytest
+import torch
+
+from helpers import assert_same_indices
+from tracetransform_amd import core
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [2, 3, 63, 64, 65, 127, 128, 129, 255, 257, 511, 512, 513, 1023, 1025, 2047, 2048]
+
+
+def p2(cols):
+    circ, rank = core.circus(torch.from_numpy(cols[None]).cuda(), [(2,)], with_p2_rank=True)
+    return circ[0, 0].cpu().numpy(), rank[0, 0].cpu().numpy()
+
+
+@pytest.mark.parametrize("n", SIZES)
+def test_p2_edges(oracle, gpu, n):
+    rng = np.random.default_rng(n)
+    cols = np.stack([
+        rng.random(n),
+        rng.random(n) - 0.5,
+        np.round(rng.random(n) * 8) / 8,                     # ties
+        np.where(rng.random(n) < 0.5, 0.0, -0.0) + np.round(rng.random(n)),
+        -np.arange(n, dtype=np.float64),                     # descending
+        np.where(np.arange(n) == n // 2, np.inf, rng.random(n)),
+        np.full(n, 1e-42),                                   # denormal
+        np.zeros(n),
+    ]).astype(np.float32)
+    got, rank = p2(cols)
+    want, aux = oracle.circus(cols, n, len(cols), [(2,)])
+    assert_same_indices("rank", rank, aux["p2_rank"][0])
+    assert np.array_equal(got, want[0])
+
+
+@pytest.mark.parametrize("n", [5, 64, 300, 1500])
+def test_p2_nan_columns(gpu, n):
+    rng = np.random.default_rng(n)
+    cols = rng.random((3, n)).astype(np.float32)
+    cols[0, n // 3] = np.nan
+    cols[1, n - 1] = np.nan
+    cols[2, 0] = -np.float32(np.nan)
+    assert np.signbit(cols[2, 0])
+    got, rank = p2(cols)
+    assert (rank == n - 1).all()
+    assert np.isnan(got[0]) and np.isnan(got[1])
+    assert got[2] == np.nanmax(cols[2])
+
+
+@pytest.mark.parametrize("side", [60, 64, 90, 130, 182, 260, 364, 520])
+def test_t6_t7_widths(oracle, gpu, side):
+    # an image that fills its square: tails of every length up to the side
+    n, A, step = side, 6, 60.0
+    img = np.random.default_rng(side).random((n, n), dtype=np.float32)
+    img[:, ::7] = 0.0
+    sino, aux = core.sinograms(torch.from_numpy(img).cuda(), A, step, [6, 7], with_aux=True)
+    o, oaux = oracle.sinograms(np.ascontiguousarray(img).ravel(), n, A, step, [6, 7],
+                               nthreads=8)
+    assert_same_indices("t6_rank", aux["t6_rank"].cpu(), oaux["t6_rank"])
+    assert_same_indices("t6_src", aux["t6_src"].cpu(), oaux["t6_src"])
+    assert_same_indices("t7_rank", aux["t7_rank"].cpu(), oaux["t7_rank"])
+    assert_same_indices("t7_src", aux["t7_src"].cpu(), oaux["t7_src"])
+    assert np.array_equal(sino.cpu().numpy(), o)

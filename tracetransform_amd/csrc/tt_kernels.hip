@@ -1458,72 +1458,221 @@ __device__ __forceinline__ uint64_t shfl_xor64(uint64_t v, int m)
     return ((uint64_t)(uint32_t)hi << 32) | (uint32_t)lo;
 }
 
-__device__ __forceinline__ uint32_t shfl_xor_key(uint32_t v, int m)
+// The sort's keys: float (any values but NaN, -0 as +0) or uint64_t
+// (tail_key: the bits of a non-negative float, then an index).  The 64-bit
+// keys order as the doubles of the same bits (finite: the high word is at most
+// a float infinity, exponent field 0x7F8), so a compare-exchange of two keys of
+// either kind is a minimum and a maximum, the 64-bit ones at the rate of the
+// 32-bit ones on this chip (an integer compare of 64 bits needs four selects
+// more).  Written in assembly: the compiler's fmin would first quiet NaNs
+// that cannot occur.
+__device__ __forceinline__ uint64_t key_min(uint64_t a, uint64_t b)
 {
-    return (uint32_t)__shfl_xor((int)v, m, kWave);
+    uint64_t r;
+    asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ uint64_t key_max(uint64_t a, uint64_t b)
+{
+    uint64_t r;
+    asm("v_max_f64 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ float key_min(float a, float b)
+{
+    float r;
+    asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+__device__ __forceinline__ float key_max(float a, float b)
+{
+    float r;
+    asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+}
+// A key that no other sorts after.
+template <class Key>
+__device__ __forceinline__ Key key_last()
+{
+    if constexpr (sizeof(Key) == 8)
+        return 0x7FEFFFFFFFFFFFFFull;
+    else
+        return INFINITY;
+}
+// Float key of a value that is not NaN.
+__device__ __forceinline__ float key_of(float v) { return v == 0.0f ? 0.0f : v; }
+
+// Value of lane l ^ LX (LX = 1, 2, 4, 8) by data-parallel moves: full-rate
+// VALU instructions (two for 4), where a shuffle is an LDS access at a fifth of
+// that rate through one unit per CU.
+template <int LX>
+__device__ __forceinline__ uint32_t lane_xor(uint32_t v)
+{
+    static_assert(LX == 1 || LX == 2 || LX == 4 || LX == 8, "within a row of 16 lanes");
+    const int x = (int)v;
+    if constexpr (LX == 1)
+        return (uint32_t)__builtin_amdgcn_mov_dpp(x, 0xB1, 0xf, 0xf, true);  // quad 1 0 3 2
+    else if constexpr (LX == 2)
+        return (uint32_t)__builtin_amdgcn_mov_dpp(x, 0x4E, 0xf, 0xf, true);  // quad 2 3 0 1
+    else if constexpr (LX == 8)
+        return (uint32_t)__builtin_amdgcn_mov_dpp(x, 0x128, 0xf, 0xf, true);  // row_ror 8
+    // mirrored within 8 lanes (l ^ 7), then within 4 (l ^ 3)
+    const int h = __builtin_amdgcn_mov_dpp(x, 0x141, 0xf, 0xf, true);
+    return (uint32_t)__builtin_amdgcn_mov_dpp(h, 0x1B, 0xf, 0xf, true);
 }
 
-__device__ __forceinline__ uint64_t shfl_xor_key(uint64_t v, int m)
+// The values of the two lanes of the pair {l, l ^ LX}, the lower lane's first,
+// on both lanes (LX = 16 or 32): the swap of row halves with itself.
+template <int LX>
+__device__ __forceinline__ uint2 lane_pair(uint32_t v)
 {
-    return shfl_xor64(v, m);
+    static_assert(LX == 16 || LX == 32, "across rows of 16 lanes");
+    if constexpr (LX == 16) {
+        const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+        return uint2{r[0], r[1]};
+    } else {
+        const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+        return uint2{r[0], r[1]};
+    }
 }
 
-// Ascending bitonic sort of 64*KPL keys (uint32_t or uint64_t) held by one
+// One bitonic exchange between lanes l and l ^ LX, the lower lane keeping the
+// smaller key.  LX < 16: the upper lanes hold their keys negated, so that
+// both sides are the minimum of the own key and the negated other one.
+template <int LX>
+__device__ __forceinline__ void exchange(uint64_t &v, bool lower)
+{
+    const uint32_t lo = (uint32_t)v, hi = (uint32_t)(v >> 32);
+    if constexpr (LX >= 16) {
+        const uint2 pl = lane_pair<LX>(lo), ph = lane_pair<LX>(hi);
+        const uint64_t a = ((uint64_t)ph.x << 32) | pl.x, b = ((uint64_t)ph.y << 32) | pl.y;
+        const bool less = __longlong_as_double((long long)a) < __longlong_as_double((long long)b);
+        v = less == lower ? a : b;
+    } else {
+        const uint64_t b = ((uint64_t)lane_xor<LX>(hi) << 32) | lane_xor<LX>(lo);
+        asm("v_min_f64 %0, %0, -%1" : "+v"(v) : "v"(b));
+    }
+}
+template <int LX>
+__device__ __forceinline__ void exchange(float &v, bool lower)
+{
+    if constexpr (LX >= 16) {
+        const uint2 p = lane_pair<LX>(__float_as_uint(v));
+        // the median with -inf is the minimum, with +inf the maximum
+        asm("v_med3_f32 %0, %1, %2, %3"
+            : "=v"(v)
+            : "v"(p.x), "v"(p.y), "v"(lower ? -INFINITY : INFINITY));
+    } else {
+        const uint32_t b = lane_xor<LX>(__float_as_uint(v));
+        asm("v_min_f32 %0, %0, -%1" : "+v"(v) : "v"(b));
+    }
+}
+
+// Negates the keys of the lanes where the sign state changes.
+template <int KPL>
+__device__ __forceinline__ void key_sign(uint64_t (&k)[KPL], bool &neg, bool next)
+{
+    const uint64_t flip = neg != next ? 1ull << 63 : 0ull;
+#pragma unroll
+    for (int r = 0; r < KPL; r++)
+        k[r] ^= flip;
+    neg = next;
+}
+template <int KPL>
+__device__ __forceinline__ void key_sign(float (&k)[KPL], bool &neg, bool next)
+{
+    const uint32_t flip = neg != next ? 1u << 31 : 0u;
+#pragma unroll
+    for (int r = 0; r < KPL; r++)
+        k[r] = __uint_as_float(__float_as_uint(k[r]) ^ flip);
+    neg = next;
+}
+
+// Strides LX, LX / 2, .. 1 lanes of a merge; down: the lane's block descends,
+// i.e. ascends in its negated keys.
+template <int LX, int KPL, class Key>
+__device__ __forceinline__ void merge_lanes(Key (&k)[KPL], int lane, bool down, bool &neg)
+{
+    const bool lower = (lane & LX) == 0;
+    key_sign(k, neg, LX >= 16 ? down : down == lower);
+#pragma unroll
+    for (int r = 0; r < KPL; r++)
+        exchange<LX>(k[r], lower);
+    if constexpr (LX > 1)
+        merge_lanes<LX / 2>(k, lane, down, neg);
+}
+
+// In-lane strides S, S / 2, .. 1, ascending.
+template <int S, int KPL, class Key>
+__device__ __forceinline__ void merge_regs(Key (&k)[KPL])
+{
+#pragma unroll
+    for (int r = 0; r < KPL; r++) {
+        const int r2 = r ^ S;
+        if (r2 > r) {
+            const Key a = k[r], b = k[r2];
+            k[r] = key_min(a, b);
+            k[r2] = key_max(a, b);
+        }
+    }
+    if constexpr (S > 1)
+        merge_regs<S / 2>(k);
+}
+
+// Merges of LM lanes' keys, then of 2 LM, .. up to the wave.
+template <int LM, int KPL, class Key>
+__device__ __forceinline__ void merge_levels(Key (&k)[KPL], int lane, bool neg)
+{
+    const bool down = (lane & LM) != 0;
+    merge_lanes<LM / 2>(k, lane, down, neg);
+    if constexpr (KPL > 1 || LM == kWave)
+        key_sign(k, neg, down);
+    if constexpr (KPL > 1)
+        merge_regs<KPL / 2>(k);
+    if constexpr (LM < kWave)
+        merge_levels<2 * LM>(k, lane, neg);
+}
+
+// Ascending bitonic sort of 64*KPL keys (float or uint64_t) held by one
 // wave in registers, blocked layout: lane l holds positions l*KPL ..
 // l*KPL+KPL-1.  Merge sizes up to KPL stay inside a lane and are unrolled
 // with their directions known at compile time; for larger sizes the
 // direction depends on the lane only, strides of KPL and more exchange with
-// lane l ^ (stride / KPL) through shuffles.  Wave-synchronous: no barriers.
-// (DPP forms of the exchanges were measured slower here: they raise the
-// VGPR count and cost occupancy.)
+// lane l ^ (stride / KPL).  Descending blocks (and, across lanes, the upper
+// lane of a pair) hold their keys negated, so every exchange is the same
+// minimum and maximum on all lanes.  Wave-synchronous: no barriers; every lane
+// of the wave must be active.
+//
+// No exchange goes through LDS: shuffles (a ds_bpermute a word, 5.5 times a
+// VALU instruction's slot at full occupancy) were what the sorts of T6/T7
+// waited for.  T6/T7 of 1449^2 pixels at 360 angles 5.2 -> 3.8 ms, P2 of the
+// 276480 columns of 256 images 1.81 -> 1.35 ms; bound by VALU issue now (3.5
+// slots per 64-bit key and stride across lanes, 1 within a lane).
 template <int KPL, class Key>
 __device__ __forceinline__ void wave_bitonic_sort(Key (&k)[KPL], int lane)
 {
-    constexpr int M = kWave * KPL;
-    const bool lane_up = (lane & 1) == 0;  // direction of the size-KPL merge
 #pragma unroll
-    for (int size = 2; size <= KPL; size <<= 1) {
+    for (int size = 2; size < KPL; size <<= 1) {
 #pragma unroll
         for (int stride = size >> 1; stride > 0; stride >>= 1) {
 #pragma unroll
             for (int r = 0; r < KPL; r++) {
                 const int r2 = r ^ stride;
                 if (r2 > r) {
-                    const bool up = size == KPL ? lane_up : (r & size) == 0;
                     const Key a = k[r], b = k[r2];
-                    const bool sw = (a > b) == up;
-                    k[r] = sw ? b : a;
-                    k[r2] = sw ? a : b;
+                    const bool up = (r & size) == 0;
+                    k[r] = up ? key_min(a, b) : key_max(a, b);
+                    k[r2] = up ? key_max(a, b) : key_min(a, b);
                 }
             }
         }
     }
-    for (int size = 2 * KPL; size <= M; size <<= 1) {
-        const bool up = ((lane * KPL) & size) == 0;
-        for (int stride = size >> 1; stride >= KPL; stride >>= 1) {
-            const int lx = stride / KPL;
-            // the lower lane of each pair keeps the minimum when ascending
-            const bool keep_min = ((lane & lx) == 0) == up;
-#pragma unroll
-            for (int r = 0; r < KPL; r++) {
-                const Key o = shfl_xor_key(k[r], lx);
-                k[r] = ((k[r] < o) == keep_min) ? k[r] : o;
-            }
-        }
-#pragma unroll
-        for (int stride = KPL / 2; stride > 0; stride >>= 1) {
-#pragma unroll
-            for (int r = 0; r < KPL; r++) {
-                const int r2 = r ^ stride;
-                if (r2 > r) {
-                    const Key a = k[r], b = k[r2];
-                    const bool sw = (a > b) == up;
-                    k[r] = sw ? b : a;
-                    k[r2] = sw ? a : b;
-                }
-            }
-        }
+    bool neg = false;
+    if constexpr (KPL > 1) {
+        key_sign(k, neg, (lane & 1) != 0);  // direction of the size-KPL merge
+        merge_regs<KPL / 2>(k);
     }
+    merge_levels<2>(k, lane, neg);
 }
 
 // Wave-wide reductions.
@@ -1704,22 +1853,24 @@ __device__ __forceinline__ int weighted_median_walk_view(const TailView &v, int 
 // of the sorted part, takes the Eigen-order sum and the sequential walk over
 // the full sequence, and returns the key at the weighted-median position k.
 template <bool IDX>
-using TailKey = typename std::conditional<IDX, uint64_t, uint32_t>::type;
+using TailKey = typename std::conditional<IDX, uint64_t, float>::type;
 
 // Sort key of tail sample i: T6 w = float(i) * x with the index (stable
 // order, and the source row is an output); T7 the value x, with the index
 // when its source row is asked for (IDX7), else alone (equal values are
-// interchangeable).  Counts the zero keys of the index-carrying kinds.
+// interchangeable).  Only tails without a negative or NaN sample are sorted,
+// so the bits of a float order as its value.  Counts the zero keys of the
+// index-carrying kinds.
 template <bool T6, bool IDX7>
 __device__ __forceinline__ TailKey<T6 || IDX7> tail_key(const float *xs, int i, bool *zero)
 {
     const float x = xs[i];
     const float kv = T6 ? (float)i * x : x;
     *zero = kv == 0.0f;
-    if constexpr (T6 || IDX7)
-        return ((uint64_t)ord_key(kv) << 32) | (uint32_t)i;
+    if constexpr (T6 || IDX7)  // (-0 as +0, as ord_key)
+        return ((uint64_t)(__float_as_uint(kv) & 0x7FFFFFFFu) << 32) | (uint32_t)i;
     else
-        return ord_key(kv);
+        return key_of(kv);
 }
 
 // Highest lane index whose flag is set plus base, or `prev` when none is:
@@ -1749,10 +1900,10 @@ __device__ __forceinline__ uint64_t tail_key_at(const TailKey<IDX> (&key)[KR], i
 #pragma unroll
     for (int r = 0; r < KR; r++)
         kk = (r == pr) ? key[r] : kk;
-    if constexpr (IDX)
-        return lane_u64(kk, pl);
+    if constexpr (IDX)  // the orderable form of a non-negative value
+        return lane_u64(kk, pl) | (1ull << 63);
     else  // value key in the high word (no index asked for)
-        return (uint64_t)(uint32_t)lane_int((int)kk, pl) << 32;
+        return (uint64_t)ord_key(lane_float(kk, pl)) << 32;
 }
 
 // Second half of a sorted tail's median: the sorted part's keys are in
@@ -1780,9 +1931,9 @@ __device__ __forceinline__ uint64_t tail_finish(const TailKey<T6 || IDX7> (&key)
                 if constexpr (T6)
                     sq[r] = line_sqrt<FS>(xs[(uint32_t)key[r]]);
                 else if constexpr (IDX7)
-                    sq[r] = line_sqrt<FS>(ord_val((uint32_t)(key[r] >> 32)));
+                    sq[r] = line_sqrt<FS>(__uint_as_float((uint32_t)(key[r] >> 32)));
                 else
-                    sq[r] = line_sqrt<FS>(ord_val(key[r]));
+                    sq[r] = line_sqrt<FS>(key[r]);
             }
         }
     };
@@ -1827,7 +1978,7 @@ __device__ __forceinline__ uint64_t sorted_tail_median(float *xs, int L, int Le,
 #pragma unroll
     for (int r = 0; r < K; r++) {
         const int i = r * kWave + lane;  // any placement: the sort orders them
-        key[r] = (Key)~(Key)0;
+        key[r] = key_last<Key>();
         bool z = false;
         if (i < Le)
             key[r] = tail_key<T6, IDX7>(xs, i, &z);
@@ -1911,7 +2062,7 @@ __device__ __forceinline__ void sort_prefix(Key (&k)[KMAX], int K, int lane)
 // P2 of one sinogram column per wave, columns of up to kP2Max rows
 // (functionals.cpp:303-311, the weighted median of the sorted column with
 // the values as weights, :21-30): the column sorted in the wave's registers
-// (32-bit order keys: equal values are interchangeable), the sorted values
+// (value keys: equal values are interchangeable), the sorted values
 // into the wave's LDS row, the Eigen-order sum on lanes 0..7 and the
 // sequential walk on lane 0.  Entry q of the P list; four columns per
 // workgroup.
@@ -1951,21 +2102,39 @@ __device__ __forceinline__ void p2_wave(const float *x, int n, float *xs, int la
                                         float *res, int *rank, int *src = nullptr)
 {
     const int K = keys_per_lane<32>(n);
-    uint32_t key[32];
+    float key[32];
+    bool nan = false;
 #pragma unroll
     for (int r = 0; r < 32; r++) {
         const int i = r * kWave + lane;
-        key[r] = r < K && i < n ? ord_key(x[i]) : ~0u;
+        const float c = r < K && i < n ? x[i] : INFINITY;
+        nan = nan || c != c;
+        key[r] = key_of(c);
+    }
+    if (__builtin_amdgcn_ballot_w64(nan)) {
+        // a NaN sum: no prefix passes, the last position's value is the
+        // largest in the order of ord_key (a positive NaN where there is one)
+        uint32_t best = 0;
+        for (int i = lane; i < n; i += kWave) {
+            const uint32_t o = ord_key(x[i]);
+            best = o > best ? o : best;
+        }
+        best = (uint32_t)wave_max_u64(best);
+        *res = ord_val(best);
+        *rank = n - 1;
+        if (src)
+            *src = p2_source(x, n, *res, n - 1, lane);
+        return;
     }
     if (K <= 16)
-        sort_prefix<16>(reinterpret_cast<uint32_t(&)[16]>(key), K, lane);
+        sort_prefix<16>(reinterpret_cast<float(&)[16]>(key), K, lane);
     else
         wave_bitonic_sort<32>(key, lane);
 #pragma unroll
     for (int r = 0; r < 32; r++) {
         const int pos = lane * K + r;
         if (r < K && pos < n)
-            xs[pos] = ord_val(key[r]);
+            xs[pos] = key[r];
     }
     wave_lds_sync();
     const TailView v = {xs, 0, 0, n};
@@ -2289,7 +2458,7 @@ __device__ __forceinline__ int sort_pair(const SortTParams &p, int line, float *
     for (int r = 0; r < KMAX; r++) {
         const int i = r * kWave + lane;  // < 64 * K: within the first K slots
         bool z = false;
-        key6[r] = ~0ull;
+        key6[r] = key_last<uint64_t>();
         if (i < Le6)
             key6[r] = tail_key<true, false>(xs + o6, i, &z);
         ins6 += __popcll(__ballot(z));
@@ -2316,7 +2485,7 @@ __device__ __forceinline__ int sort_pair(const SortTParams &p, int line, float *
     for (int r = 0; r < KMAX; r++) {
         const int i = r * kWave + lane;
         bool z = false;
-        key7[r] = (Key7)~(Key7)0;
+        key7[r] = key_last<Key7>();
         if (i < Le7)
             key7[r] = tail_key<false, IDX7>(xs + o7, i, &z);
         if constexpr (IDX7)
@@ -2331,9 +2500,9 @@ __device__ __forceinline__ int sort_pair(const SortTParams &p, int line, float *
             const int p7 = lane * K7 + r;
             if (r < K7 && p7 < Le7) {
                 if constexpr (IDX7)
-                    xs[p7] = line_sqrt<FS>(ord_val((uint32_t)(key7[r] >> 32)));
+                    xs[p7] = line_sqrt<FS>(__uint_as_float((uint32_t)(key7[r] >> 32)));
                 else
-                    xs[p7] = line_sqrt<FS>(ord_val(key7[r]));
+                    xs[p7] = line_sqrt<FS>(key7[r]);
             }
         }
     };
@@ -2369,9 +2538,11 @@ __device__ __forceinline__ int sort_pair(const SortTParams &p, int line, float *
 // the two tails of a line together when both are requested.  The passes over
 // queued items (KMIN = KMAX) build only their widest network: a smaller code
 // and fewer spills than one network per width.  The occupancy hints are the
-// measured best (more waves beat the spills they cost).
+// measured best: the 8-key pass over 1449^2 pixels at 360 angles takes 1.64 ms
+// at 4 waves per SIMD (56 bytes spilled), 1.79 at 5 (more spills), 1.82 at 3;
+// the 16-key one 2.05 at 3 (none), 2.66 at 2.
 template <int KMAX, int KMIN, bool DEFER, bool IDX7>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(KMAX <= 4 ? 5 : KMAX <= 8 ? 6 : KMAX <= 16 ? 4 : 1)))
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(KMAX <= 4 ? 4 : KMAX <= 8 ? 4 : KMAX <= 16 ? 3 : 1)))
 void sino_sort_kernel(SortTParams p)
 {
     constexpr int M = kWave * KMAX;
