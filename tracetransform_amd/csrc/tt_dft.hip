@@ -7,10 +7,16 @@
 //   spec (2h x cols) = W^T x (n x cols),   h = n/2 + 1,
 // with W (n x 2h) = [cos(2 pi jk/n) | -sin(2 pi jk/n)].  Its adjoint applies
 // the same matrix the other way: ds (n x cols) = W y (2h x cols), y the
-// spectrum scaled per column and frequency.  Both are one kernel over a list
-// of jobs (one per image of a batch), so the single-image and the batched
-// path form their spectra with the same operations in the same order and
-// give the same P3 bit for bit.
+// spectrum scaled per column and frequency.  The cosine is even in j and the
+// sine odd, so positions j and n - j fold: the real parts are the product of
+// an h x h cosine matrix with x_j + x_(n-j), the imaginary parts that of a
+// sine matrix with x_j - x_(n-j), half the multiplications of W (and half the
+// terms, hence roundings, in each sum).  The adjoint's two products give the
+// even and odd parts C_j, S_j of ds, j <= n/2, and its consumer unfolds
+// ds_j = C_j - S_j, ds_(n-j) = C_j + S_j.  Both directions are one kernel over
+// a list of jobs (one per image of a batch), so the single-image and the
+// batched path form their spectra with the same operations in the same order
+// and give the same P3 bit for bit.
 #include "tt_internal.hpp"
 
 #include <math.h>
@@ -30,13 +36,8 @@ typedef float __attribute__((address_space(1))) *gfloat;
 // output rows x columns per workgroup: 128 x 128, 64 x 128 or 64 x 64
 constexpr int kDftBK = 16;   // reduction chunk
 
-// Twiddle index (u v) mod n of W(row, kk) for the first of four consecutive
-// kk and the step between them: W(row, kk) is the cosine or minus the sine
-// of 2 pi t / n.  FWD: out = W^T in, the output row m is a frequency (m < h:
-// real part, else imaginary part of frequency m - h) and kk a position;
-// otherwise out = W in, the output row is a position and kk runs over the
-// 2h spectrum entries (consecutive kk share u, and v steps by one except
-// across kk = h, handled by the caller).
+// (u v) mod n of the entry (row u, reduction index v) of the cosine or sine
+// matrix: cos or sin of 2 pi u v / n.
 __device__ __forceinline__ int phase_mod(int u, int v, int n, float inv_n)
 {
     // u v < 2730^2 < 2^23: exact in float; the quotient is off by at most one
@@ -44,25 +45,6 @@ __device__ __forceinline__ int phase_mod(int u, int v, int n, float inv_n)
     int t = uv - (int)__umul24((uint32_t)(int)((float)uv * inv_n), (uint32_t)n);
     t = t < 0 ? t + n : t;
     return t >= n ? t - n : t;
-}
-
-template <bool FWD>
-__device__ __forceinline__ float dft_weight(const float2 *tw, int n, int h, float inv_n,
-                                            int row, int kk)
-{
-    int u, v;
-    bool sn;
-    if (FWD) {
-        sn = row >= h;
-        u = sn ? row - h : row;
-        v = kk;
-    } else {
-        sn = kk >= h;
-        u = row;
-        v = sn ? kk - h : kk;
-    }
-    const float2 w = tw[phase_mod(u, v, n, inv_n)];
-    return sn ? -w.y : w.x;
 }
 
 __device__ __forceinline__ int find_job(const DftJob *jobs, int njobs, int tile)
@@ -78,15 +60,18 @@ __device__ __forceinline__ int find_job(const DftJob *jobs, int njobs, int tile)
     return lo;
 }
 
-// One BM x 128 output tile per workgroup of four waves (2 x 2 wave tiles of
-// BM/2 x 64, BM/16 MFMA accumulators each; BM = 128 for large launches,
-// 64 where 128-row tiles would leave CUs idle), reduction in chunks of 16,
-// double buffered: while the matrix cores work on one chunk (16 or 32
-// MFMAs per wave, the latter long enough to cover the next chunk's global
-// loads) the waves generate the next W chunk from the LDS twiddles (BM/16
-// consecutive entries per thread, the phase stepped by u) and load the next
-// input chunk into registers.
+// One BM x BN output tile per workgroup of four waves (2 x 2 wave tiles of
+// BM/2 x BN/2, up to four MFMA accumulators each; 128 x 128 for large
+// launches, smaller where those would leave CUs idle), all of it in the cosine
+// or all in the sine product, reduction in chunks of 16, double buffered:
+// while the matrix cores work on one chunk (16 or 32 MFMAs per wave, the
+// latter long enough to cover the next chunk's global loads) the waves
+// generate the next chunk of the matrix from the LDS twiddles (BM/16
+// consecutive entries per thread, the phase stepped by u) and load and fold
+// the next input chunk into registers.
 // Twiddles (cos, sin)(2 pi t / n) are rounded from double sincospi.
+// The 276480 columns (avg 407 rows) of 256 images: 1.53 ms unfolded, 0.99 ms
+// folded; FP32 matrix cores at 53 TFLOP/s of 157.
 template <bool FWD, int BM, int BN>
 __global__ __launch_bounds__(kBlock) void dft_gemm_kernel(DftParams p)
 {
@@ -94,14 +79,20 @@ __global__ __launch_bounds__(kBlock) void dft_gemm_kernel(DftParams p)
     constexpr int MB = BM / 64;  // 32-row blocks per wave
     constexpr int NB = BN / 64;  // 32-column blocks per wave
     __shared__ float sA[2][kDftBK][BM];
-    __shared__ float sB[2][kDftBK][BN];
+    __shared__ float sB[2][kDftBK][BN + 4];  // pitch: the loader's 16 rows in 64 banks
     extern __shared__ float2 s_tw[];
     const DftJob &jb = p.jobs ? p.jobs[find_job(p.jobs, p.njobs, blockIdx.x)] : p.job;
     const int n = jb.n, h = n / 2 + 1;
-    const int M = FWD ? 2 * h : n, Kd = FWD ? n : 2 * h;
+    // the cosine rows come first: frequencies 0..h-1 or positions 0..n/2; the
+    // sine rows are frequencies 0..h-1 or positions 1..(n-1)/2
     const int local = blockIdx.x - jb.tile0;
-    const int mtiles = (M + BM - 1) / BM;
-    const int m0 = (local % mtiles) * BM, c0 = (local / mtiles) * BN;
+    const int ctiles = (h + BM - 1) / BM;
+    const int srows = FWD ? h : n - h;
+    const int mtiles = ctiles + (srows + BM - 1) / BM;
+    const int mt = local % mtiles;
+    const bool sn = mt >= ctiles;
+    const int M = sn ? srows : h, Kd = h;
+    const int m0 = (sn ? mt - ctiles : mt) * BM, c0 = (local / mtiles) * BN;
     const int tid = threadIdx.x;
     for (int i = tid; i < n; i += kBlock) {
         double sn, cn;
@@ -113,68 +104,64 @@ __global__ __launch_bounds__(kBlock) void dft_gemm_kernel(DftParams p)
     const int wm = (wave & 1) * (BM / 2), wn = (wave >> 1) * (BN / 2);
     // W loader: row ar of the tile, reduction entries ak .. ak + EA - 1
     const int ar = tid % BM, ak = (tid / BM) * EA;
-    const int arow = m0 + ar;
-    // input loader: columns bc (and bc + 64) of the tile, entries bk .. bk + 3
-    const int bc = tid & 63, bk = (tid >> 6) * 4;
-    const int col0 = c0 + bc, col1 = c0 + 64 + bc;
-    const gcfloat src0 = (gcfloat)(jb.in + (size_t)(col0 < jb.cols ? col0 : 0) * jb.ld_in);
-    const gcfloat src1 = (gcfloat)(jb.in + (size_t)(col1 < jb.cols ? col1 : 0) * jb.ld_in);
-    float ra[EA], rb0[4], rb1[4];
+    const int arow = m0 + ar;                   // row of the cosine or sine part
+    const int urow = arow + (sn && !FWD ? 1 : 0);  // its frequency or position
+    // input loader: entry bk of the chunk of the columns bc + 16 i, so that 16
+    // lanes read one column's consecutive entries (a column per lane costs an
+    // L1 lookup per lane)
+    constexpr int EB = BN / 16;  // input entries per thread and chunk
+    const int bk = tid & 15, bc = tid >> 4;
+    const gcfloat src = (gcfloat)(jb.in + (size_t)c0 * jb.ld_in);
+    uint32_t off[EB];  // the columns' offsets (the last column past the end)
+#pragma unroll
+    for (int i = 0; i < EB; i++) {
+        const int c = c0 + bc + 16 * i;
+        off[i] = (uint32_t)((c < jb.cols ? c : jb.cols - 1) - c0) * (uint32_t)jb.ld_in;
+    }
+    float ra[EA], rb[EB], rm[EB];
     auto fetch = [&](int k0) {
         const int kk0 = k0 + ak;
-        if (arow < M && kk0 + EA - 1 < Kd && (FWD || kk0 + EA - 1 < h || kk0 >= h)) {
-            // EA consecutive kk of one half: one modular product, then steps
-            int u, v;
-            bool sn;
-            if (FWD) {
-                sn = arow >= h;
-                u = sn ? arow - h : arow;
-                v = kk0;
-            } else {
-                sn = kk0 >= h;
-                u = arow;
-                v = sn ? kk0 - h : kk0;
-            }
-            int t = phase_mod(u, v, n, inv_n);
-            const int du = u >= n ? u - n : u;
+        // EA consecutive kk: one modular product, then steps
+        int t = phase_mod(arow < M ? urow : 0, kk0 < Kd ? kk0 : 0, n, inv_n);
 #pragma unroll
-            for (int e = 0; e < EA; e++) {
-                const float2 w = s_tw[t];
-                ra[e] = sn ? -w.y : w.x;
-                t += du;
-                t = t >= n ? t - n : t;
-            }
-        } else {
-#pragma unroll
-            for (int e = 0; e < EA; e++) {
-                const int kk = kk0 + e;
-                ra[e] = arow < M && kk < Kd ? dft_weight<FWD>(s_tw, n, h, inv_n, arow, kk)
-                                            : 0.0f;
-            }
+        for (int e = 0; e < EA; e++) {
+            const float2 w = s_tw[t];
+            const float v = sn ? (FWD ? -w.y : w.y) : w.x;
+            ra[e] = arow < M && kk0 + e < Kd ? v : 0.0f;
+            t += arow < M ? urow : 0;
+            t = t >= n ? t - n : t;
         }
+        // the reduction's entry kk of a column: a sample and its mirror, or a
+        // spectrum's real or imaginary part (folded by store)
+        const int kk = k0 + bk;
+        const int at = kk < Kd ? kk : 0;
+        const uint32_t o0 = (uint32_t)(FWD ? at : sn ? h + at : at);
+        const uint32_t o1 = (uint32_t)(at > 0 ? n - at : 0);
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            const int kk = k0 + bk + e;
-            rb0[e] = col0 < jb.cols && kk < Kd ? src0[kk] : 0.0f;
-            if constexpr (NB == 2)
-                rb1[e] = col1 < jb.cols && kk < Kd ? src1[kk] : 0.0f;
+        for (int i = 0; i < EB; i++) {
+            rb[i] = src[off[i] + o0];
+            if constexpr (FWD)
+                rm[i] = src[off[i] + o1];
         }
     };
-    auto store = [&](int buf) {
+    auto store = [&](int buf, int k0) {
 #pragma unroll
         for (int e = 0; e < EA; e++)
             sA[buf][ak + e][ar] = ra[e];
+        const int kk = k0 + bk;
+        const bool in = kk < Kd, two = kk > 0 && 2 * kk < n;  // has a mirror of its own
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            sB[buf][bk + e][bc] = rb0[e];
-            if constexpr (NB == 2)
-                sB[buf][bk + e][64 + bc] = rb1[e];
+        for (int i = 0; i < EB; i++) {
+            float v = rb[i];
+            if constexpr (FWD)
+                v = two ? (sn ? v - rm[i] : v + rm[i]) : (sn ? 0.0f : v);
+            sB[buf][bk][bc + 16 * i] = in ? v : 0.0f;
         }
     };
     f32x16 acc00 = {}, acc01 = {}, acc10 = {}, acc11 = {};
     __syncthreads();  // twiddles
     fetch(0);
-    store(0);
+    store(0, 0);
     __syncthreads();
     int buf = 0;
     for (int k0 = 0; k0 < Kd; k0 += kDftBK) {
@@ -200,7 +187,7 @@ __global__ __launch_bounds__(kBlock) void dft_gemm_kernel(DftParams p)
             }
         }
         if (more)
-            store(buf ^ 1);
+            store(buf ^ 1, k0 + kDftBK);
         __syncthreads();
         buf ^= 1;
     }
@@ -210,7 +197,7 @@ __global__ __launch_bounds__(kBlock) void dft_gemm_kernel(DftParams p)
     for (int half = 0; half < NB; half++) {
         const int oc = c0 + wn + 32 * half + (lane & 31);
         if (oc < jb.cols) {
-            const gfloat dst = (gfloat)(jb.out + (size_t)oc * jb.ld_out);
+            const gfloat dst = (gfloat)(jb.out + (size_t)oc * jb.ld_out + (sn ? h : 0));
 #pragma unroll
             for (int mh = 0; mh < MB; mh++)
 #pragma unroll
@@ -323,8 +310,8 @@ hipError_t launch_p3_vjp_scale(const P3ScaleParams &p, int max_cols, hipStream_t
 int dft_job_tiles(int n, int cols, bool forward, int bm, int bn)
 {
     const int h = n / 2 + 1;
-    const int M = forward ? 2 * h : n;
-    return ((M + bm - 1) / bm) * ((cols + bn - 1) / bn);
+    const int srows = forward ? h : n - h;
+    return ((h + bm - 1) / bm + (srows + bm - 1) / bm) * ((cols + bn - 1) / bn);
 }
 
 }  // namespace ttk

@@ -199,7 +199,7 @@ size_t gather_lds_bytes(int tile, int waves, int tabn, bool do345, bool do12, bo
 struct CircusVjpParams {
     const float *sino;    // [nsino][ncols][n]
     const float *dcircus; // [nsino][np][ncols]
-    float *dsino;         // [nsino][ncols][n] (holds P3's part when p3_done)
+    float *dsino;         // [nsino][ncols][n] (holds P3's part, folded, when p3_done)
     int p3_done;
     const int32_t *p2src; // [nsino][ncols] P2 source rows, or null (then sorted here)
     const double *herm_w; // [nherm][n]
@@ -214,8 +214,10 @@ struct CircusVjpParams {
 // P3's transforms as GEMMs on the matrix cores (tt_dft.hip).  One job per
 // image: forward, out (2h x cols, ld_out) = W^T in (n x cols, ld_in), the
 // half spectra (real parts, then imaginary parts); adjoint, out (n x cols)
-// = W in (2h x cols).  W (n x 2h) = [cos(2 pi jk/n) | -sin(2 pi jk/n)],
-// h = n / 2 + 1.
+// = W in (2h x cols) folded: rows 0..h-1 hold the even part C_j (j <= n/2),
+// rows h..n-1 the odd part S_j (j = 1..(n-1)/2), W in at j being C_j - S_j and
+// at n - j C_j + S_j (dft_unfold).  W (n x 2h) = [cos(2 pi jk/n) |
+// -sin(2 pi jk/n)], h = n / 2 + 1.
 struct DftJob {
     const float *in;
     float *out;
@@ -252,6 +254,16 @@ struct P3ScaleParams {
 int dft_job_tiles(int n, int cols, bool forward, int bm, int bn);
 void dft_tile_shape(long long tiles128, long long tiles64, int *bm, int *bn);
 size_t dft_lds_bytes(int nmax);
+// Entry j of an adjoint column from its folded form f.
+template <class P>
+__device__ __forceinline__ float dft_unfold(P f, int n, int j)
+{
+    const int h = n / 2 + 1;
+    const int m = n - j;  // the mirrored position
+    if (j == 0 || j == m)
+        return f[j];
+    return j < m ? f[j] - f[h + j - 1] : f[m] + f[h + m - 1];
+}
 hipError_t launch_dft_gemm(const DftParams &p, bool forward, int nmax, hipStream_t s);
 hipError_t launch_p3_vjp_scale(const P3ScaleParams &p, int max_cols, hipStream_t s);
 
@@ -431,7 +443,7 @@ struct BatchAdjointParams {
     int do345;
     Slots slot;
     int code[kMaxP];
-    int p3_done;          // dsino holds P3's part (the DFT GEMMs ran first)
+    int p3_done;          // dsino holds P3's part, folded (the DFT GEMMs ran first)
 };
 hipError_t launch_circus_vjp_batched(const BatchAdjointParams &p, hipStream_t s);
 hipError_t launch_records_batched(const BatchAdjointParams &p, hipStream_t s);

@@ -3129,7 +3129,7 @@ __device__ __forceinline__ VjpLds vjp_lds(unsigned char *smem, int nmax)
 
 // J_P^T dC for the column x[0..n) already in L.x; dc[q * dc_stride] is the
 // upstream gradient of P-functional q at this column.  P3's part comes from
-// the DFT GEMMs (tt_dft.hip) and is already in out when p3_done; the P1, P2
+// the DFT GEMMs (tt_dft.hip) and is already in out (folded) when p3_done; the P1, P2
 // and Hermite parts are added to it and the sum written back to out.
 __device__ void circus_vjp_column(const VjpLds &L, int n, int np, const int *code,
                                   const int *herm, const double *herm_w,
@@ -3143,7 +3143,7 @@ __device__ void circus_vjp_column(const VjpLds &L, int n, int np, const int *cod
     while (m2 < n)
         m2 <<= 1;
     for (int i = threadIdx.x; i < n; i += kBlock)
-        L.ds[i] = p3_done ? out[i] : 0.0f;
+        L.ds[i] = p3_done ? dft_unfold(out, n, i) : 0.0f;
     __syncthreads();
     for (int q = 0; q < np; q++) {
         const float g = dc[q * dc_stride];
