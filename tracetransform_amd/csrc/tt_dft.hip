@@ -60,6 +60,39 @@ __device__ __forceinline__ int find_job(const DftJob *jobs, int njobs, int tile)
     return lo;
 }
 
+// X_0 of column c: the plain sum of the column, in its order.  It is the
+// largest term of P3 by far and nearly the same at every angle, and the z-score
+// of a signature subtracts most of it, so its rounding shows: folding it as
+// the other rows moved signature columns by 7e-5 where this moves them by 1e-5
+// (P3 of T0 of a noise image).  A thread per column, in workgroups of their own
+// beside the tiles: their loads hide behind the matrix work.
+__device__ __forceinline__ void dft_dc(const DftJob &jb, int c)
+{
+    if (c >= jb.cols)
+        return;
+    typedef float f4 __attribute__((ext_vector_type(4), aligned(4)));
+    typedef const f4 __attribute__((address_space(1))) *gcf4;
+    const gcfloat x = (gcfloat)(jb.in + (size_t)c * jb.ld_in);
+    float sum = 0.0f;
+    int j = 0;
+    for (; j + 16 <= jb.n; j += 16) {
+        f4 v[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+            v[e] = *(gcf4)(x + j + 4 * e);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            sum += v[e].x;
+            sum += v[e].y;
+            sum += v[e].z;
+            sum += v[e].w;
+        }
+    }
+    for (; j < jb.n; j++)
+        sum += x[j];
+    ((gfloat)(jb.out + (size_t)c * jb.ld_out))[0] = sum;
+}
+
 // One BM x BN output tile per workgroup of four waves (2 x 2 wave tiles of
 // BM/2 x BN/2, up to four MFMA accumulators each; 128 x 128 for large
 // launches, smaller where those would leave CUs idle), all of it in the cosine
@@ -70,8 +103,8 @@ __device__ __forceinline__ int find_job(const DftJob *jobs, int njobs, int tile)
 // consecutive entries per thread, the phase stepped by u) and load and fold
 // the next input chunk into registers.
 // Twiddles (cos, sin)(2 pi t / n) are rounded from double sincospi.
-// The 276480 columns (avg 407 rows) of 256 images: 1.53 ms unfolded, 0.99 ms
-// folded; FP32 matrix cores at 53 TFLOP/s of 157.
+// The 276480 columns (avg 407 rows) of 256 images: 1.53 ms unfolded, 1.04 ms
+// folded (X_0 included); FP32 matrix cores at 51 TFLOP/s of 157.
 template <bool FWD, int BM, int BN>
 __global__ __launch_bounds__(kBlock) void dft_gemm_kernel(DftParams p)
 {
@@ -89,11 +122,16 @@ __global__ __launch_bounds__(kBlock) void dft_gemm_kernel(DftParams p)
     const int ctiles = (h + BM - 1) / BM;
     const int srows = FWD ? h : n - h;
     const int mtiles = ctiles + (srows + BM - 1) / BM;
+    const int tid = threadIdx.x;
+    const int ntiles = (jb.cols + BN - 1) / BN;
+    if (FWD && local >= mtiles * ntiles) {
+        dft_dc(jb, (local - mtiles * ntiles) * kBlock + tid);
+        return;
+    }
     const int mt = local % mtiles;
     const bool sn = mt >= ctiles;
     const int M = sn ? srows : h, Kd = h;
     const int m0 = (sn ? mt - ctiles : mt) * BM, c0 = (local / mtiles) * BN;
-    const int tid = threadIdx.x;
     for (int i = tid; i < n; i += kBlock) {
         double sn, cn;
         sincospi(2.0 * (double)i / (double)n, &sn, &cn);
@@ -205,7 +243,7 @@ __global__ __launch_bounds__(kBlock) void dft_gemm_kernel(DftParams p)
                     const int om =
                         m0 + wm + 32 * mh + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
                     const f32x16 &acc = mh ? (half ? acc11 : acc10) : (half ? acc01 : acc00);
-                    if (om < M)
+                    if (om < M && !(FWD && !sn && om == 0))
                         dst[om] = acc[r];
                 }
         }
@@ -311,7 +349,8 @@ int dft_job_tiles(int n, int cols, bool forward, int bm, int bn)
 {
     const int h = n / 2 + 1;
     const int srows = forward ? h : n - h;
-    return ((h + bm - 1) / bm + (srows + bm - 1) / bm) * ((cols + bn - 1) / bn);
+    return ((h + bm - 1) / bm + (srows + bm - 1) / bm) * ((cols + bn - 1) / bn) +
+           (forward ? (cols + kBlock - 1) / kBlock : 0);
 }
 
 }  // namespace ttk
