@@ -1,4 +1,5 @@
-"""GPU tests of the wave sort behind P2, T6 and T7 at its edges: every network
+"""GPU tests of the one-wave circus kernel and of the wave sort behind P2, T6
+and T7 at its edges: every network
 width (64 keys and powers of two up to 2048) from one row short to one row
 over, signed values, ties, both zeros, infinities, and NaN columns.  Ranks
 and values are the oracle's exactly; a column with a NaN has a NaN sum, which
@@ -9,7 +10,7 @@ import numpy as np
 import pytest
 import torch
 
-from helpers import assert_same_indices
+from helpers import assert_same_indices, normwise_err
 from tracetransform_amd import core
 
 pytestmark = pytest.mark.gpu
@@ -39,6 +40,23 @@ def test_p2_edges(oracle, gpu, n):
     want, aux = oracle.circus(cols, n, len(cols), [(2,)])
     assert_same_indices("rank", rank, aux["p2_rank"][0])
     assert np.array_equal(got, want[0])
+
+
+@pytest.mark.parametrize("n", [2, 3, 64, 512, 513, 1024, 1025, 2048, 2049, 2730])
+def test_p1_p2_p3_key_widths(oracle, gpu, n):
+    # the kernel's three key widths and the longer columns' own kernel, the
+    # functionals in any order and repeated
+    rng = np.random.default_rng(n)
+    cols = (rng.random((5, n)) * 3).astype(np.float32)
+    pf = [(3,), (1,), (2,), (1,), (3,)]
+    got, rank = core.circus(torch.from_numpy(cols[None]).cuda(), pf, with_p2_rank=True)
+    _, aux = oracle.circus(cols, n, 5, pf)
+    want = oracle.circus_f64(cols, n, 5, pf, aux["p2_src"], geometry=1)
+    got = got[0].cpu().numpy()
+    assert_same_indices("rank", rank[0, 2].cpu(), aux["p2_rank"][2])
+    for q in range(len(pf)):
+        assert normwise_err(got[q], want[q]) <= 1e-5, pf[q]
+    assert np.array_equal(got[0], got[4]) and np.array_equal(got[1], got[3])
 
 
 @pytest.mark.parametrize("n", [5, 64, 300, 1500])

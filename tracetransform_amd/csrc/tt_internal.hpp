@@ -110,8 +110,8 @@ struct BatchCircusParams {
     int nmax;
     int np;
     int code[kMaxP];
-    int p2_wave;          // P2 entries written by circus_p2_batched_kernel (launcher's)
-    int with_circus;      // circus_p2_batched_kernel writes circus values
+    int wave_done;        // P1..P3 entries written by circus_wave_batched_kernel (launcher's)
+    int with_circus;      // circus_wave_batched_kernel writes circus values
 };
 
 // Sort-based T-functionals T6/T7 for one padded image: one workgroup owns one
@@ -157,7 +157,7 @@ struct CircusParams {
     int np;
     int code[kMaxP];
     int herm[kMaxP];      // row of herm_w for Hermite entries
-    int p2_wave;          // P2 entries written by circus_p2_kernel (launcher's)
+    int wave_done;        // P1..P3 entries written by circus_wave_kernel (launcher's)
 };
 
 struct RecordParams {

@@ -1268,7 +1268,7 @@ __device__ __forceinline__ CircusLds circus_lds(float *smem, int nmax)
 __device__ void circus_column(const CircusLds &L, int n, int np, const int *code,
                               const int *herm, const double *herm_w, float *out,
                               size_t out_stride, int32_t *p2rank,
-                              const float *spec, int spec_h, bool skip_p2)
+                              const float *spec, int spec_h, bool wave_done)
 {
     __shared__ float s_red[kBlock / kWave];
     __shared__ double s_red_d[kBlock / kWave];
@@ -1280,8 +1280,8 @@ __device__ void circus_column(const CircusLds &L, int n, int np, const int *code
         m2 <<= 1;
     for (int q = 0; q < np; q++) {
         const int cd = code[q];
-        if (cd == 2 && skip_p2)
-            continue;  // written by circus_p2_kernel
+        if (cd != 0 && wave_done)
+            continue;  // written by circus_wave_kernel
         float res = 0.0f;
         if (cd == 1) {
             float acc = 0.0f;
@@ -1351,7 +1351,7 @@ __global__ __launch_bounds__(kBlock) void circus_kernel(CircusParams p)
     circus_column(L, n, p.np, p.code, p.herm, p.herm_w, p.out + o, p.ncols,
                   p.p2rank ? p.p2rank + o : nullptr,
                   p.p3_spec ? p.p3_spec + (size_t)colg * 2 * p.p3_h : nullptr, p.p3_h,
-                  p.p2_wave != 0);
+                  p.wave_done != 0);
 }
 
 // Every sinogram column of a batch; the image is found by binary search over
@@ -1383,7 +1383,7 @@ __global__ __launch_bounds__(kBlock) void circus_batched_kernel(BatchCircusParam
     const int h = n / 2 + 1;
     circus_column(L, n, p.np, p.code, herm_none, nullptr,
                   im.circus + (size_t)t * p.np * p.A + a, p.A, nullptr,
-                  im.spec ? im.spec + (size_t)lc * 2 * h : nullptr, h, p.p2_wave != 0);
+                  im.spec ? im.spec + (size_t)lc * 2 * h : nullptr, h, p.wave_done != 0);
 }
 
 // ---------------------------------------------------------------------------
@@ -2098,14 +2098,15 @@ __device__ __forceinline__ int p2_source(const float *x, int n, float v, int k, 
 // P2 of the column x[0..n) (n <= kP2Max) by one wave, sorted values in xs;
 // the value and its rank are valid on lane 0, and with src its source row
 // (every lane).
+template <int KMAX>
 __device__ __forceinline__ void p2_wave(const float *x, int n, float *xs, int lane,
                                         float *res, int *rank, int *src = nullptr)
 {
-    const int K = keys_per_lane<32>(n);
-    float key[32];
+    const int K = keys_per_lane<KMAX>(n);
+    float key[KMAX];
     bool nan = false;
 #pragma unroll
-    for (int r = 0; r < 32; r++) {
+    for (int r = 0; r < KMAX; r++) {
         const int i = r * kWave + lane;
         const float c = r < K && i < n ? x[i] : INFINITY;
         nan = nan || c != c;
@@ -2126,12 +2127,16 @@ __device__ __forceinline__ void p2_wave(const float *x, int n, float *xs, int la
             *src = p2_source(x, n, *res, n - 1, lane);
         return;
     }
-    if (K <= 16)
-        sort_prefix<16>(reinterpret_cast<float(&)[16]>(key), K, lane);
-    else
-        wave_bitonic_sort<32>(key, lane);
+    if constexpr (KMAX <= 16) {
+        sort_prefix<KMAX>(key, K, lane);
+    } else {
+        if (K <= 16)
+            sort_prefix<16>(reinterpret_cast<float(&)[16]>(key), K, lane);
+        else
+            wave_bitonic_sort<KMAX>(key, lane);
+    }
 #pragma unroll
-    for (int r = 0; r < 32; r++) {
+    for (int r = 0; r < KMAX; r++) {
         const int pos = lane * K + r;
         if (r < K && pos < n)
             xs[pos] = key[r];
@@ -2149,49 +2154,127 @@ __device__ __forceinline__ void p2_wave(const float *x, int n, float *xs, int la
         *src = p2_source(x, n, xs[k], k, lane);
 }
 
-__global__ __launch_bounds__(kBlock) void circus_p2_kernel(CircusParams p, int q)
+// P1 of the column x[0..n) by one wave: the sum of |x[i - 1] - x[i]|.
+__device__ __forceinline__ float p1_wave(const float *x, int n, int lane)
 {
-    __shared__ float s_x[kBlock / kWave][kP2Max];
+    float acc = 0.0f;
+    for (int i = 1 + lane; i < n; i += kWave)
+        acc += fabsf(x[i - 1] - x[i]);
+    return wave_sum(acc);
+}
+
+// P3 from a column's half spectrum (tt_dft.hip) by one wave, mod in LDS (n / 2
+// + 1 floats): (|X| / N)^4 in double (c++/src/functionals.cpp:332-360 takes
+// pow(hypot(Re/N, Im/N), 4)), mirrored onto k > N/2, and the trapz sum over
+// the reference's float abscissae lin[p] = -1 + 2p/(N-1) (:53-60; the
+// quotient corrected by its remainder, the division's own result).
+__device__ __forceinline__ float p3_wave(const float *spec, int h, int n, float *mod, int lane)
+{
+    const int half = n / 2;
+    const double inv_n = 1.0 / (double)n, den = (double)(n - 1), inv_d = 1.0 / den;
+    for (int k = lane; k <= half; k += kWave) {
+        const double re = (double)spec[k] * inv_n, im = (double)spec[h + k] * inv_n;
+        const double m2 = fma(re, re, im * im);
+        mod[k] = (float)(m2 * m2);
+    }
+    wave_lds_sync();
+    auto lin = [&](int i) {
+        const double a = 2.0 * (double)i, q = a * inv_d;
+        return (float)(-1.0 + fma(fma(-q, den, a), inv_d, q));
+    };
+    float acc = 0.0f;
+    for (int i = lane; i < n - 1; i += kWave) {
+        const int m0 = i <= half ? i : n - i, m1 = i < half ? i + 1 : n - i - 1;
+        acc += (lin(i + 1) - lin(i)) * (mod[m1] + mod[m0]);
+    }
+    const float r = (float)(wave_sum(acc) * 0.5);
+    wave_lds_sync();
+    return r;
+}
+
+// P1, P2 and P3 of one sinogram column by one wave (xs: the wave's 64 KMAX
+// floats of LDS), results q of the P list at out[q * stride] (out may be
+// null: only the source row is wanted), P2's rank and source row where asked
+// for.  Hermite entries are left to the workgroup kernel.
+template <int KMAX>
+__device__ __forceinline__ void circus_wave_column(const float *x, int n, float *xs, int lane,
+                                                   int np, const int *code, float *out,
+                                                   size_t stride, int32_t *p2rank,
+                                                   int32_t *p2src, const float *spec, int h)
+{
+    float r1 = 0.0f, r2 = 0.0f, r3 = 0.0f;
+    int rank = 0, src = -1;
+    bool p1 = false, p2 = p2src != nullptr, p3 = false;
+    for (int q = 0; out && q < np; q++) {
+        p1 = p1 || code[q] == 1;
+        p2 = p2 || code[q] == 2;
+        p3 = p3 || code[q] == 3;
+    }
+    if (p3)
+        r3 = p3_wave(spec, h, n, xs, lane);
+    if (p1)
+        r1 = p1_wave(x, n, lane);
+    if (p2)
+        p2_wave<KMAX>(x, n, xs, lane, &r2, &rank, p2src ? &src : nullptr);
+    if (lane != 0)
+        return;
+    for (int q = 0; out && q < np; q++) {
+        if (code[q] == 0)
+            continue;
+        out[q * stride] = code[q] == 1 ? r1 : code[q] == 2 ? r2 : r3;
+        if (p2rank && code[q] == 2)
+            p2rank[q * stride] = rank;
+    }
+    if (p2src)
+        *p2src = src;
+}
+
+// One wave per sinogram column of up to 64 KMAX rows, four columns per
+// workgroup.  KMAX is the smallest of 8, 16 and 32 that holds the longest
+// column: the keys set the registers, hence the waves in flight that hide the
+// sequential walk.  One pass over the columns for all three
+// functionals, where P1 and P3 took a workgroup per column in a launch of
+// their own: P1-P3 of the 276480 columns (avg 407 rows) of 256 images
+// 2.23 -> 1.28 ms.
+template <int KMAX>
+__global__ __launch_bounds__(kBlock) void circus_wave_kernel(CircusParams p)
+{
+    __shared__ float s_x[kBlock / kWave][kWave * KMAX];
     const int w = wave_id(), lane = threadIdx.x & (kWave - 1);
     const int colg = blockIdx.x * (kBlock / kWave) + w;
     if (colg >= p.ncols * p.nsino)
         return;
-    float res;
-    int k;
-    p2_wave(p.sino + (size_t)colg * p.n, p.n, s_x[w], lane, &res, &k);
-    if (lane == 0) {
-        const int sg = colg / p.ncols, col = colg - sg * p.ncols;
-        const size_t o = ((size_t)sg * p.np + q) * p.ncols + col;
-        p.out[o] = res;
-        if (p.p2rank)
-            p.p2rank[o] = k;
-    }
+    const int sg = colg / p.ncols, col = colg - sg * p.ncols;
+    const size_t o = (size_t)sg * p.np * p.ncols + col;
+    circus_wave_column<KMAX>(p.sino + (size_t)colg * p.n, p.n, s_x[w], lane, p.np, p.code,
+                             p.out + o, p.ncols, p.p2rank ? p.p2rank + o : nullptr, nullptr,
+                             p.p3_spec ? p.p3_spec + (size_t)colg * 2 * p.p3_h : nullptr,
+                             p.p3_h);
 }
 
 // P2's source row of every sinogram column (the adjoint's one-hot), columns
-// up to kP2Max rows: src[colg] for the n-row columns of sino.
+// up to 64 KMAX rows: src[colg] for the n-row columns of sino.
+template <int KMAX>
 __global__ __launch_bounds__(kBlock) void p2_source_kernel(const float *sino, int n, int cols,
                                                            int32_t *src)
 {
-    __shared__ float s_x[kBlock / kWave][kP2Max];
+    __shared__ float s_x[kBlock / kWave][kWave * KMAX];
     const int w = wave_id(), lane = threadIdx.x & (kWave - 1);
     const int colg = blockIdx.x * (kBlock / kWave) + w;
     if (colg >= cols)
         return;
-    float res;
-    int k, sr;
-    p2_wave(sino + (size_t)colg * n, n, s_x[w], lane, &res, &k, &sr);
-    if (lane == 0)
-        src[colg] = sr;
+    circus_wave_column<KMAX>(sino + (size_t)colg * n, n, s_x[w], lane, 0, nullptr, nullptr, 0,
+                             nullptr, src + colg, nullptr, 0);
 }
 
 // The same over every sinogram column of a batch (image found by binary
-// search over the descriptors' first-column offsets; every n <= kP2Max).
-// Writes the circus value (with circus) and the source row (into the
+// search over the descriptors' first-column offsets; every n <= 64 KMAX).
+// Writes the circus values (with_circus) and P2's source row (into the
 // image's p2src [nt][A], when set).
-__global__ __launch_bounds__(kBlock) void circus_p2_batched_kernel(BatchCircusParams p, int q)
+template <int KMAX>
+__global__ __launch_bounds__(kBlock) void circus_wave_batched_kernel(BatchCircusParams p)
 {
-    __shared__ float s_x[kBlock / kWave][kP2Max];
+    __shared__ float s_x[kBlock / kWave][kWave * KMAX];
     const int w = wave_id(), lane = threadIdx.x & (kWave - 1);
     const int colg = blockIdx.x * (kBlock / kWave) + w;
     if (colg >= p.cols)
@@ -2205,20 +2288,14 @@ __global__ __launch_bounds__(kBlock) void circus_p2_batched_kernel(BatchCircusPa
             hi = mid - 1;
     }
     const BatchImage &im = p.images[lo];
-    const int n = im.n;
+    const int n = im.n, h = n / 2 + 1;
     const int lc = colg - im.col0;
     const int t = lc / p.A;
     const int a = lc - t * p.A;
-    float res;
-    int k, sr = -1;
-    p2_wave(im.sino + ((size_t)t * p.A + a) * n, n, s_x[w], lane, &res, &k,
-            im.p2src ? &sr : nullptr);
-    if (lane == 0) {
-        if (p.with_circus)
-            im.circus[((size_t)t * p.np + q) * p.A + a] = res;
-        if (im.p2src)
-            im.p2src[lc] = sr;
-    }
+    circus_wave_column<KMAX>(im.sino + ((size_t)t * p.A + a) * n, n, s_x[w], lane, p.np, p.code,
+                             p.with_circus ? im.circus + (size_t)t * p.np * p.A + a : nullptr,
+                             p.A, nullptr, im.p2src ? im.p2src + lc : nullptr,
+                             im.spec ? im.spec + (size_t)lc * 2 * h : nullptr, h);
 }
 
 // findWeightedMedian of one column per wave (columns up to kP2Max rows, in
@@ -3106,24 +3183,22 @@ __global__ __launch_bounds__(1024) void gather_batched_kernel(BatchAdjointParams
 // derivative of sum_p w_p |X_q(p)|^4 / N^4, an inverse-DFT-shaped sum;
 // Hermite: its weights).
 // LDS layout of one circus-VJP workgroup for columns of height up to nmax.
+// (sq and key only where P2's source row is found by sorting here)
 struct VjpLds {
-    uint64_t *key;  // pow2 >= nmax
     float *x;       // nmax4
-    float *sq;      // nmax4
     float *ds;      // nmax4
+    float *sq;      // nmax4
+    uint64_t *key;  // pow2 >= nmax
 };
 
 __device__ __forceinline__ VjpLds vjp_lds(unsigned char *smem, int nmax)
 {
     const int n4 = (nmax + 3) & ~3;
-    int m2 = 1;
-    while (m2 < nmax)
-        m2 <<= 1;
     VjpLds l;
-    l.key = reinterpret_cast<uint64_t *>(smem);
-    l.x = reinterpret_cast<float *>(l.key + m2);
-    l.sq = l.x + n4;
-    l.ds = l.sq + n4;
+    l.x = reinterpret_cast<float *>(smem);
+    l.ds = l.x + n4;
+    l.sq = l.ds + n4;
+    l.key = reinterpret_cast<uint64_t *>(l.sq + n4);
     return l;
 }
 
@@ -3583,35 +3658,63 @@ static size_t circus_shm(int nmax)
     return sizeof(float) * (2 * n4 + m2);
 }
 
+// Calls f with the key width of columns of up to n (<= kP2Max) rows.
+template <class F>
+static void with_key_width(int n, F f)
+{
+    if (n <= 8 * kWave)
+        f(std::integral_constant<int, 8>{});
+    else if (n <= 16 * kWave)
+        f(std::integral_constant<int, 16>{});
+    else
+        f(std::integral_constant<int, 32>{});
+}
+
+static int wave_blocks(int cols)
+{
+    const int wpb = kBlock / kWave;
+    return (cols + wpb - 1) / wpb;
+}
+
 hipError_t launch_circus(const CircusParams &p, hipStream_t s)
 {
-    // P2 of columns up to kP2Max rows: one wave per column
+    // P1..P3 of columns up to kP2Max rows: one wave per column; Hermite
+    // entries, and every entry of longer columns: one workgroup per column
     CircusParams c = p;
-    c.p2_wave = 0;
-    bool other = false;
     const int cols = p.ncols * p.nsino;
-    const int wpb = kBlock / kWave;
+    bool wave = false, block = false;
     for (int q = 0; q < p.np; q++) {
-        if (p.code[q] == 2 && p.n <= kP2Max) {
-            circus_p2_kernel<<<(cols + wpb - 1) / wpb, kBlock, 0, s>>>(p, q);
-            c.p2_wave = 1;
-        } else {
-            other = true;
-        }
+        const bool w = p.code[q] != 0 && p.n <= kP2Max;
+        wave = wave || w;
+        block = block || !w;
     }
-    if (other)
+    c.wave_done = wave;
+    if (wave)
+        with_key_width(p.n, [&](auto K) {
+            circus_wave_kernel<decltype(K)::value><<<wave_blocks(cols), kBlock, 0, s>>>(c);
+        });
+    if (block)
         circus_kernel<<<cols, kBlock, circus_shm(p.n), s>>>(c);
     return hipGetLastError();
 }
-
 
 hipError_t launch_p2_source(const float *sino, int n, int cols, int32_t *src, hipStream_t s)
 {
     if (n > kP2Max)
         return hipErrorInvalidValue;
-    const int wpb = kBlock / kWave;
-    p2_source_kernel<<<(cols + wpb - 1) / wpb, kBlock, 0, s>>>(sino, n, cols, src);
+    with_key_width(n, [&](auto K) {
+        p2_source_kernel<decltype(K)::value>
+            <<<wave_blocks(cols), kBlock, 0, s>>>(sino, n, cols, src);
+    });
     return hipGetLastError();
+}
+
+static void launch_circus_wave_batched(const BatchCircusParams &p, hipStream_t s)
+{
+    with_key_width(p.nmax, [&](auto K) {
+        circus_wave_batched_kernel<decltype(K)::value>
+            <<<wave_blocks(p.cols), kBlock, 0, s>>>(p);
+    });
 }
 
 hipError_t launch_p2_source_batched(const BatchCircusParams &p, hipStream_t s)
@@ -3620,28 +3723,17 @@ hipError_t launch_p2_source_batched(const BatchCircusParams &p, hipStream_t s)
         return hipErrorInvalidValue;
     BatchCircusParams c = p;
     c.with_circus = 0;
-    const int wpb = kBlock / kWave;
-    circus_p2_batched_kernel<<<(p.cols + wpb - 1) / wpb, kBlock, 0, s>>>(c, 0);
+    launch_circus_wave_batched(c, s);
     return hipGetLastError();
 }
 
 hipError_t launch_circus_batched(const BatchCircusParams &p, hipStream_t s)
 {
-    // P2 of columns up to kP2Max rows: one wave per column
-    BatchCircusParams c = p;
-    c.p2_wave = 0;
-    bool other = false;
-    const int wpb = kBlock / kWave;
-    for (int q = 0; q < p.np; q++) {
-        if (p.code[q] == 2 && p.nmax <= kP2Max) {
-            circus_p2_batched_kernel<<<(p.cols + wpb - 1) / wpb, kBlock, 0, s>>>(p, q);
-            c.p2_wave = 1;
-        } else {
-            other = true;
-        }
-    }
-    if (other)
-        circus_batched_kernel<<<p.cols, kBlock, circus_shm(p.nmax), s>>>(c);
+    // as launch_circus (no Hermite entries in a batch)
+    if (p.nmax <= kP2Max)
+        launch_circus_wave_batched(p, s);
+    else
+        circus_batched_kernel<<<p.cols, kBlock, circus_shm(p.nmax), s>>>(p);
     return hipGetLastError();
 }
 
@@ -3833,24 +3925,26 @@ hipError_t launch_gather(const GatherParams &p, hipStream_t s)
     return hipGetLastError();
 }
 
-static size_t vjp_shm(int nmax)
+// sort: some P2 source row is found in the kernel (columns above kP2Max).
+static size_t vjp_shm(int nmax, bool sort)
 {
     int m2 = 1;
     while (m2 < nmax)
         m2 <<= 1;
     const size_t n4 = ((size_t)nmax + 3) & ~(size_t)3;
-    return sizeof(uint64_t) * m2 + sizeof(float) * 3 * n4;
+    return sort ? sizeof(uint64_t) * m2 + sizeof(float) * 3 * n4 : sizeof(float) * 2 * n4;
 }
 
 hipError_t launch_circus_vjp(const CircusVjpParams &p, hipStream_t s)
 {
-    circus_vjp_kernel<<<p.ncols * p.nsino, kBlock, vjp_shm(p.n), s>>>(p);
+    circus_vjp_kernel<<<p.ncols * p.nsino, kBlock, vjp_shm(p.n, !p.p2src), s>>>(p);
     return hipGetLastError();
 }
 
 hipError_t launch_circus_vjp_batched(const BatchAdjointParams &p, hipStream_t s)
 {
-    circus_vjp_batched_kernel<<<p.cols, kBlock, vjp_shm(p.nmax), s>>>(p);
+    // (the batch's P2 source rows come from the wave kernel up to kP2Max rows)
+    circus_vjp_batched_kernel<<<p.cols, kBlock, vjp_shm(p.nmax, p.nmax > kP2Max), s>>>(p);
     return hipGetLastError();
 }
 
