@@ -243,10 +243,11 @@ TT_API tt_status tt_batched_launch_shape(tt_context *ctx, int *waves_per_block,
  *     kernel: 64, 32 or 16 consecutive columns of line_angles consecutive
  *     angles, a multiple of 64 / line_columns up to 16 (candidates 1x64,
  *     2x64, 4x64, 2x32, 4x32, 4x16, 8x16);
- *   gather_tile x gather_tile pixels (32 or 16), gather_waves waves per
- *     workgroup (1..16), of the batched backward's transposed rotation.
+ *   gather_tile: pixel tiles of class 32 (30 x 32 pixels) or 16 (16 x 24),
+ *     gather_waves waves per workgroup (1..16), of the batched backward's
+ *     transposed rotation.
  * A line's results and a pixel's gradient are the same bits whatever the
- * tiles.  Zero fields mean the default (1x64, 32 pixels, the most waves that
+ * tiles.  Zero fields mean the default (1x64, class 32, the most waves that
  * fit the LDS) or, with autotuning, the tuned choice. */
 typedef struct tt_tiles {
     int32_t line_angles;

@@ -986,14 +986,13 @@ int layout_line_items(std::vector<ttk::BatchImage> &d, int A, LineTile t)
     return items;
 }
 
-// First gather tile of each image for tiles of side T; returns the total.
+// First gather tile of each image for tiles of class T; returns the total.
 int layout_gather_tiles(std::vector<ttk::BatchImage> &d, int T)
 {
     int tiles = 0;
     for (ttk::BatchImage &b : d) {
         b.tile0 = tiles;
-        const int t = (b.n + T - 1) / T;
-        tiles += t * t;
+        tiles += ttk::gather_tiles(b.n, T);
     }
     return tiles;
 }
@@ -1001,7 +1000,7 @@ int layout_gather_tiles(std::vector<ttk::BatchImage> &d, int T)
 // The most waves per workgroup (up to 16) whose gather LDS fits, or 0.
 int gather_waves_max(int T, int tabn, bool do345, bool do12)
 {
-    for (int waves : {16, 8, 4, 2, 1})
+    for (int waves = 16; waves >= 1; waves--)
         if (ttk::gather_lds_bytes(T, waves, tabn, do345, do12, false) <= kLdsLimit)
             return waves;
     return 0;
@@ -1660,8 +1659,8 @@ tt_status forward_for_adjoint(tt_context *ctx, const float *d_image, int n, int 
     return TT_OK;
 }
 
-// Launch shape of the transposed-rotation gather: 32 x 32 pixel tiles, the
-// most waves per workgroup (16, 8, 4, 2, 1) whose LDS (the T3..T5 tables once
+// Launch shape of the transposed-rotation gather: tiles of class 32, the
+// most waves per workgroup (16 to 1) whose LDS (the T3..T5 tables once
 // plus each wave's accumulators and staged columns) fits the 160 KiB of a
 // CU, and for a single image enough angle groups that tiles x groups waves
 // fill every SIMD four times over.
@@ -1673,7 +1672,7 @@ GatherLaunch choose_gather(int tiles32, int A, int cus, int tabn, bool do345, bo
                            bool do67, bool split_angles)
 {
     GatherLaunch g = {32, 1, 1};
-    for (int waves : {16, 8, 4, 2, 1}) {
+    for (int waves = 16; waves >= 1; waves--) {
         if (ttk::gather_lds_bytes(32, waves, tabn, do345, do12, do67) <= kLdsLimit) {
             g.waves = waves;
             break;
@@ -1699,12 +1698,6 @@ GatherLaunch choose_gather(int tiles32, int A, int cus, int tabn, bool do345, bo
         }
     }
     return g;
-}
-
-int tile_count(int n, int tile)
-{
-    const int t = (n + tile - 1) / tile;
-    return t * t;
 }
 
 
@@ -1740,7 +1733,7 @@ tt_status image_vjp(tt_context *ctx, int n, int A, const int *slot,
     g.A = A;
     g.do345 = slot[3] >= 0 || slot[4] >= 0 || slot[5] >= 0;
     g.do12 = slot[1] >= 0 || slot[2] >= 0;
-    const GatherLaunch gl = choose_gather(tile_count(n, 32), A, device_cus(ctx->device), n,
+    const GatherLaunch gl = choose_gather(ttk::gather_tiles(n, 32), A, device_cus(ctx->device), n,
                                           g.do345, g.do12, do67, true);
     g.tile = gl.tile;
     g.waves = gl.waves;
@@ -2330,7 +2323,7 @@ TT_API tt_status tt_backward_batched(tt_context *ctx, const tt_image_grad *image
         TT_HIP(P.rec.ensure(sizeof(ttk::LineRecord) * ln));
         if (p3s.np3 > 0)
             TT_HIP(P.y.ensure(sizeof(float) * spec_tot));
-        // gather tile: forced, 32 pixels, or tuned below
+        // gather tile: forced, class 32, or tuned below
         int gtile = ctx->force.gather_tile > 0 ? ctx->force.gather_tile : 32;
         int gwaves = ctx->force.gather_waves > 0 ? ctx->force.gather_waves
                                                  : gather_waves_max(gtile, nmax, do345, do12);

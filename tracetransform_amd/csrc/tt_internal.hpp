@@ -82,7 +82,7 @@ struct BatchImage {
     float *dimg;          // n x n
     int line0;            // first line (angle*n + col) over the batch
     int pix0;             // first pixel over the batch
-    int tile0;            // first gather tile over the batch (tiles of the launch's side)
+    int tile0;            // first gather tile over the batch (tiles of the launch's class)
 };
 
 struct BatchSinoParams {
@@ -174,7 +174,16 @@ struct RecordParams {
     Slots slot;
 };
 
-// Transposed rotation: one wave per (tile x tile pixel tile, angle group);
+// Pixels of a gather tile of class 32 or 16 (columns x rows: 30 x 32, 16 x 24).
+__host__ __device__ constexpr int gather_tx(int tile) { return tile == 16 ? 16 : 30; }
+__host__ __device__ constexpr int gather_ty(int tile) { return tile == 16 ? 24 : 32; }
+__host__ __device__ constexpr int gather_tiles(int n, int tile)
+{
+    return ((n + gather_tx(tile) - 1) / gather_tx(tile)) *
+           ((n + gather_ty(tile) - 1) / gather_ty(tile));
+}
+
+// Transposed rotation: one wave per (pixel tile, angle group);
 // with groups > 1 each group writes its partial image into part and
 // gather_reduce sums them in group order.
 struct GatherParams {
@@ -188,7 +197,7 @@ struct GatherParams {
     int A;
     int do345;
     int do12;                   // T1 or T2 requested
-    int tile;                   // 16 or 32
+    int tile;                   // tile class, 16 or 32
     int groups;                 // angle groups
     int waves;                  // waves per workgroup (1..8)
 };
@@ -435,7 +444,7 @@ struct BatchAdjointParams {
     int nmax;
     int lines;            // total lines (sum of A * n)
     int pixels;           // total pixels (sum of n * n)
-    int tiles;            // total gather tiles (of the launch's tile side)
+    int tiles;            // total gather tiles (of the launch's tile class)
     int cols;             // total sinogram columns (sum of nt * A)
     const float2 *trig;
     const float2 *tab345; // [3][tabn]
@@ -447,7 +456,7 @@ struct BatchAdjointParams {
 };
 hipError_t launch_circus_vjp_batched(const BatchAdjointParams &p, hipStream_t s);
 hipError_t launch_records_batched(const BatchAdjointParams &p, hipStream_t s);
-// Gather of a batch with tiles of side `tile` (16 or 32; images[].tile0 count
+// Gather of a batch with tiles of class `tile` (16 or 32; images[].tile0 count
 // such tiles) and `waves` waves per workgroup.
 hipError_t launch_gather_batched(const BatchAdjointParams &p, int tile, int waves,
                                  hipStream_t s);

@@ -2770,17 +2770,21 @@ __global__ __launch_bounds__(kBlock) void records_batched_kernel(BatchAdjointPar
 // held in LDS, one wave per tile.
 //
 // For every angle the wave visits the rotated samples (col, row) whose taps
-// can touch its T x T pixel tile: those whose exact source position lies in
-// the tile grown by one pixel, a square of side T + 1 turned by the angle.
-// They are enumerated as a parallelogram: the columns the square spans, and
-// in each column the rows of the narrower of the square's two slabs (one
-// slab is ignored, so up to twice the square's area at 45 degrees, 1.45x on
-// average).  Each sample is evaluated exactly as the forward evaluates it
+// can touch its pixel tile: those whose exact source position lies in the
+// tile grown by one pixel, a rectangle turned by the angle.  Each column's
+// rows are cut by both of the rectangle's slabs, and the lanes take them
+// without gaps: a work item is three consecutive rows of a column, starting
+// at a multiple of three, and the items of every third column (a column
+// class) are numbered through.  A lane finds the column of its item by
+// counting the bits of a wave-uniform mask of column starts.  The old layout
+// (16 columns x 4 rows of a parallelogram, one slab) had 1.7 to 2.5 lane
+// slots per sample; this one has 1.1.  Each sample is evaluated exactly as
+// the forward evaluates it
 // (rot_sample's float operations: coordinates, strict bounds, truncated taps
 // and modf fractions), its rotated-domain gradient G(row) comes from its
 // column's line record, and G times each of the four tap weights is added
-// into the tile's accumulators (LDS, with a one-pixel halo ring that is
-// discarded: those pixels belong to the neighbouring tiles).
+// into the tile's accumulators (LDS, with a halo that is discarded: those
+// pixels belong to the neighbouring tiles).
 //
 // Determinism without atomics: two samples whose lattice positions agree
 // modulo 3 in both coordinates are at least 3 apart, more than the 2 sqrt 2
@@ -2795,23 +2799,36 @@ __global__ __launch_bounds__(kBlock) void records_batched_kernel(BatchAdjointPar
 constexpr int kGatherFlush = 4;
 constexpr int kGatherTile = 32;
 constexpr int kGatherTabWords = 6;  // LDS floats per row of the T3..T5 tables
+constexpr int kGatherCols = 48;     // staged columns per angle, 16 a class
 
+// Tile class T (16 or 32) in pixels: the items of a column class, about
+// (TX + 1) (TY + 1) / 9 plus two thirds per column, just fill one or two
+// waves (30 x 32: 107 to 132 items, 4 % of the classes above 128; a 32 x 32
+// tile would need a third pass for nine classes in ten).
 template <int T>
 struct GatherShape {
-    static constexpr int P = T + 2;                    // accumulator side, with halo
-    static constexpr int ACC = ((P * P + 3) / 4) * 4;  // floats, padded to float4
-    static constexpr int KMAX = T == 16 ? 32 : 48;     // footprint columns per angle
-    static constexpr int NPIX = T * T / kWave;         // interior pixels per lane
-    static_assert(T == 16 || T == 32, "tiles of 16 or 32 pixels");
+    static constexpr int TX = gather_tx(T), TY = gather_ty(T);
+    static constexpr int P = TY + 5;                            // odd accumulator stride
+    static constexpr int ACC = (((TX + 4) * P + 3) / 4) * 4;    // floats, halo of two cells
+    static constexpr int NPIX = TX * TY / kWave;                // interior pixels per lane
+    static constexpr int NIT = T == 16 ? 2 : 3;                 // passes over a class at most
+    static_assert(T == 16 || T == 32, "tile classes 16 and 32");
+    static_assert(TX * TY % kWave == 0, "whole pixels per lane");
 };
 
-// LDS words of one wave: accumulators, then the staged column data
-// (per column: (g0, sm, rlo, rhi), (ab0..ab3), (ab4, ab5), and with T1/T2
-// (g1, g2, m, -), with T6/T7 (r6, r7, c6, c7)).
+// LDS words of one wave: accumulators, the staged column data (per column:
+// (g0, sm, first row, row range), (ab0..ab3), (ab4, ab5), and with T1/T2
+// (g1, g2, m, -), with T6/T7 (r6, r7, c6, c7)), and the marks of the columns'
+// first items.
+template <int T>
+__host__ __device__ constexpr int gather_words(bool do12, bool do67)
+{
+    return GatherShape<T>::ACC + kGatherCols * (4 + 4 + 2 + (do12 ? 4 : 0) + (do67 ? 4 : 0)) +
+           kWave * GatherShape<T>::NIT;
+}
 __host__ __device__ constexpr int gather_wave_words(int T, bool do12, bool do67)
 {
-    return (((T + 2) * (T + 2) + 3) / 4) * 4 +
-           (T == 16 ? 32 : 48) * (4 + 4 + 2 + (do12 ? 4 : 0) + (do67 ? 4 : 0));
+    return T == 16 ? gather_words<16>(do12, do67) : gather_words<32>(do12, do67);
 }
 
 struct GatherImg {
@@ -2828,28 +2845,32 @@ __device__ __forceinline__ void gather_tile_wave(const GatherImg &im, const floa
 {
     constexpr bool do12 = DO12;
     using S = GatherShape<T>;
-    constexpr int P = S::P;
+    constexpr int P = S::P, TX = S::TX, TY = S::TY, NIT = S::NIT;
     const int lane = threadIdx.x & (kWave - 1);
     const int n = im.n;
     const bool do67 = im.rec67 != nullptr;
     float *acc = wl;
     float4 *sA = reinterpret_cast<float4 *>(wl + S::ACC);
-    float4 *sB = sA + S::KMAX;
-    float2 *sC = reinterpret_cast<float2 *>(sB + S::KMAX);
-    float4 *sD = reinterpret_cast<float4 *>(sC + S::KMAX);
-    float4 *sE = sD + (do12 ? S::KMAX : 0);
+    float4 *sB = sA + kGatherCols;
+    float4 *sD = sB + kGatherCols;
+    float4 *sE = sD + (do12 ? kGatherCols : 0);
+    float2 *sC = reinterpret_cast<float2 *>(sE + (do67 ? kGatherCols : 0));
+    uint32_t *mark = reinterpret_cast<uint32_t *>(sC + kGatherCols);  // a byte per class
     const float o = (float)((n - 1) / 2.0);
     const float lim = (float)(n - 1);
     // the tile grown by one pixel, plus a margin far above the float
     // rounding of any sample position (< 1e-3 for n <= 2730), relative to o
     const float dm = 0.01f;
-    const int X0m = X0 - 1, Y0m = Y0 - 1;  // accumulator cell 0 (the halo)
-    const bool interior = X0 >= 2 && X0 + T <= n - 2 && Y0 >= 2 && Y0 + T <= n - 2;
-    const float xa = (float)(X0 - 1) - o - dm, xb = (float)(X0 + T) - o + dm;
-    const float ya = (float)(Y0 - 1) - o - dm, yb = (float)(Y0 + T) - o + dm;
+    const int X0m = X0 - 2, Y0m = Y0 - 2;  // accumulator cell 0 (the halo)
+    const bool interior = X0 >= 2 && X0 + TX <= n - 2 && Y0 >= 2 && Y0 + TY <= n - 2;
+    const float xa = (float)(X0 - 1) - o - dm, xb = (float)(X0 + TX) - o + dm;
+    const float ya = (float)(Y0 - 1) - o - dm, yb = (float)(Y0 + TY) - o + dm;
     const float4 z4 = {0.0f, 0.0f, 0.0f, 0.0f};
     for (int i = lane; i < S::ACC / 4; i += kWave)
         reinterpret_cast<float4 *>(acc)[i] = z4;
+#pragma unroll
+    for (int it = 0; it < NIT; it++)
+        mark[it * kWave + lane] = 0;
     double accd[S::NPIX];
 #pragma unroll
     for (int i = 0; i < S::NPIX; i++)
@@ -2857,14 +2878,14 @@ __device__ __forceinline__ void gather_tile_wave(const GatherImg &im, const floa
     wave_lds_sync();
 
     // Footprint of angle a: the columns [c_lo, c_lo + K) the grown tile
-    // spans, px = c (x - o) - s (y - o) over its corners, and in each column
-    // the rows [rlo, rhi] of the slab kp px + kq py in [lo, hi] with
-    // |kq| >= 1/sqrt 2 (y - o = -s px + c py, or x - o = c px + s py), at
-    // most W of them.
+    // spans, px = c (x - o) - s (y - o) over its corners.  Lane l stages the
+    // column kl = l % 16 of class cc = l / 16 (column index mod 3 == cc), its
+    // k-th of the footprint.
     struct Foot {
-        float c, s, kp, lo, hi, inv;
-        int c_lo, K, W;
+        float c, s;
+        int c_lo, K, k;
     };
+    const int scc = lane >> 4;
     auto footprint = [&](int a) {
         Foot f;
         const float2 cs = trig[a];
@@ -2877,29 +2898,24 @@ __device__ __forceinline__ void gather_tile_wave(const GatherImg &im, const floa
         int c_lo = (int)ceilf(pmin + o), c_hi = (int)floorf(pmax + o);
         c_lo = c_lo < 0 ? 0 : c_lo;
         c_hi = c_hi > n - 1 ? n - 1 : c_hi;
-        // (T + 1.02) (|c| + |s|) bounds the span: at most 25 / 47 columns
-        // for T = 16 / 32, so the clamp never drops one (and a class of
-        // every third column has at most 16)
+        // the diagonal of the grown tile bounds the span: at most 46 columns
+        // (16 a class), so the clamp never drops one
         const int K = c_hi - c_lo + 1;
         f.c_lo = c_lo;
-        f.K = K > S::KMAX ? S::KMAX : K;
-        const bool usey = fabsf(f.c) >= fabsf(f.s);
-        const float kq = usey ? f.c : f.s;
-        f.kp = usey ? -f.s : f.c;
-        f.lo = usey ? ya : xa;
-        f.hi = usey ? yb : xb;
-        f.inv = 1.0f / kq;
-        f.W = (int)((f.hi - f.lo) * fabsf(f.inv)) + 2;
+        f.K = K > kGatherCols - 2 ? kGatherCols - 2 : K;
+        const int koff = scc - c_lo % 3;
+        f.k = 3 * (lane & 15) + (koff < 0 ? koff + 3 : koff);
+        f.k = scc < 3 && f.k < f.K ? f.k : -1;
         return f;
     };
-    // this lane's column record of angle a (lane < K), loaded ahead (global
+    // this lane's column record of angle a (f.k >= 0), loaded ahead (global
     // address space: the loads do not wait on LDS traffic)
     typedef const float __attribute__((address_space(1))) *GF;
     auto ld4 = [](GF q) { return float4{q[0], q[1], q[2], q[3]}; };
     float4 pa4 = z4, pb4 = z4, pd4 = z4, pe4 = z4;
     auto prefetch = [&](const Foot &f, int a) {
-        if (lane < f.K) {
-            const size_t line = (size_t)a * n + f.c_lo + lane;
+        if (f.k >= 0) {
+            const size_t line = (size_t)a * n + f.c_lo + f.k;
             GF r = (GF)(im.rec + line);
             pa4 = ld4(r);
             if (DO345 || do12)
@@ -2914,15 +2930,54 @@ __device__ __forceinline__ void gather_tile_wave(const GatherImg &im, const floa
     prefetch(fn, a0);
     for (int a = a0; a < a1; a++) {
         const Foot f = fn;
-        // stage this angle's columns: (g0, sm, rlo, rhi), (ab0..ab3),
-        // (ab4, ab5), (g1, g2, m, -), (r6, r7, c6, c7)
-        if (lane < f.K) {
-            const float px = (float)(f.c_lo + lane) - o;
-            const float pa = (f.lo - f.kp * px) * f.inv, pb = (f.hi - f.kp * px) * f.inv;
-            int rlo = (int)ceilf(fminf(pa, pb) + o), rhi = (int)floorf(fmaxf(pa, pb) + o);
-            rlo = rlo < 0 ? 0 : rlo;
-            rhi = rhi > n - 1 ? n - 1 : rhi;
-            sA[lane] = float4{pa4.x, pa4.y, __int_as_float(rlo), __int_as_float(rhi)};
+        const float c = f.c, s = f.s;
+        // This lane's column: the rows of both slabs (ya <= -s px + c py <= yb
+        // and xa <= c px + s py <= xb; a slab along the column cuts nothing),
+        // and the number of items they lie in (one that is masked for a
+        // column without rows, so that every column has a first item).
+        int rlo = 0x3fffff, len = 0, first = 0, cnt = 0;
+        if (f.k >= 0) {
+            const float px = (float)(f.c_lo + f.k) - o;
+            float lo = -o, hi = lim - o;
+            if (fabsf(c) > 1e-5f) {
+                const float inv = 1.0f / c;
+                const float u = (ya + s * px) * inv, v = (yb + s * px) * inv;
+                lo = fmaxf(lo, fminf(u, v));
+                hi = fminf(hi, fmaxf(u, v));
+            }
+            if (fabsf(s) > 1e-5f) {
+                const float inv = 1.0f / s;
+                const float u = (xa - c * px) * inv, v = (xb - c * px) * inv;
+                lo = fmaxf(lo, fminf(u, v));
+                hi = fminf(hi, fmaxf(u, v));
+            }
+            cnt = 1;
+            if (lo <= hi) {
+                const int r0 = max((int)ceilf(lo + o), 0), r1 = min((int)floorf(hi + o), n - 1);
+                if (r0 <= r1) {
+                    // (thirds of numbers below 2^16)
+                    const int b0 = (int)(((uint32_t)r0 * 0xAAABu) >> 17);
+                    const int b1 = (int)(((uint32_t)r1 * 0xAAABu) >> 17);
+                    rlo = r0;
+                    len = r1 - r0;
+                    first = 3 * b0;
+                    cnt = b1 - b0 + 1;
+                }
+            }
+        }
+        // items before this column's in its class (16 lanes)
+        int incl = cnt;
+        incl += __builtin_amdgcn_update_dpp(0, incl, 0x111, 0xf, 0xf, true);
+        incl += __builtin_amdgcn_update_dpp(0, incl, 0x112, 0xf, 0xf, true);
+        incl += __builtin_amdgcn_update_dpp(0, incl, 0x114, 0xf, 0xf, true);
+        incl += __builtin_amdgcn_update_dpp(0, incl, 0x118, 0xf, 0xf, true);
+        const int start = incl - cnt;
+        if (f.k >= 0) {
+            // (the class's items number at most 156, or 75 with small tiles:
+            // every mark lies inside NIT passes)
+            reinterpret_cast<unsigned char *>(mark)[4 * start + scc] = 1;
+            sA[lane] = float4{pa4.x, pa4.y, __int_as_float(first - 3 * start),
+                              __int_as_float((rlo << 8) | len)};
             if (DO345) {
                 sB[lane] = float4{pa4.z, pa4.w, pb4.x, pb4.y};
                 sC[lane] = float2{pb4.z, pb4.w};
@@ -2933,144 +2988,163 @@ __device__ __forceinline__ void gather_tile_wave(const GatherImg &im, const floa
                 sE[lane] = pe4;
         }
         wave_lds_sync();
+        uint32_t mk[NIT];
+#pragma unroll
+        for (int it = 0; it < NIT; it++)
+            mk[it] = mark[it * kWave + lane];
+#pragma unroll
+        for (int it = 0; it < NIT; it++)
+            mark[it * kWave + lane] = 0;
         if (a + 1 < a1) {
             fn = footprint(a + 1);
             prefetch(fn, a + 1);
         }
-        const float c = f.c, s = f.s;
-        const int c_lo = f.c_lo, K = f.K;
         // CHK: test the sample positions against the image bounds.  A tile
-        // at least 2 pixels inside the image on every side can skip it: a
-        // position outside [0, n - 1) truncates (negative values to 0) to a
-        // cell outside the tile's grown range, so such a sample is dropped by
-        // the tile test alone, as the bounds test would drop it.
+        // at least 2 pixels inside the image on every side can skip it: its
+        // samples lie in the tile grown by a pixel and the margin, inside the
+        // image.  There the accumulators reach as far as the samples' taps,
+        // so nothing else is tested but the column's row range.
         auto classes = [&](auto chk) {
             constexpr bool CHK = decltype(chk)::value;
-            const float pxc0 = (float)c_lo - o;
-            const int clo3 = c_lo % 3;
-            // one residue class (column, row mod 3) at a time: samples of one
-            // class are pairwise at least 3 apart, so their 2x2 tap footprints
-            // are disjoint and every read-add-write of the class has its own
-            // four targets.  Lane l takes the class's column l % 16 (at most
-            // 16: K <= 47) and its rows 4 apart in the class from l / 16 on.
-            const int kl = lane & 15, jl = lane >> 4;
-            // one column class (col mod 3) at a time: the column's data
-            // serves its three row classes
+            const int clo3 = f.c_lo % 3;
+            // one column class (col mod 3) at a time, and in it one row class
+            // (row mod 3) after the other over all its items: samples of one
+            // residue class are pairwise at least 3 apart, so their 2x2 tap
+            // footprints are disjoint and every read-add-write of the class
+            // has its own four targets, whatever the lanes' order; the order
+            // of the classes is the same for every tiling.
             for (int cc = 0; cc < 3; cc++) {
+                const int N = __builtin_amdgcn_readlane(incl, 16 * cc + 15);
                 const int koff = cc >= clo3 ? cc - clo3 : cc - clo3 + 3;
-                const int K3 = (K - koff + 2) / 3;
-                const bool colok = kl < K3;
-                const int k = colok ? 3 * kl + koff : 0;
-                const float4 ea = sA[k];
-                const float g0 = ea.x;
-                const int sm = __float_as_int(ea.y);
-                const int rlo = __float_as_int(ea.z);
-                const int rhi = colok ? __float_as_int(ea.w) : -1;
-                const int r3 = rlo - 3 * (int)(((uint32_t)rlo * 0xAAABu) >> 17);
-                float4 eb = {}, ed = {}, ee = {};
-                float2 ec = {};
-                if (DO345) {
-                    eb = sB[k];
-                    ec = sC[k];
-                }
-                if (do12)
-                    ed = sD[k];
-                if (do67)
-                    ee = sE[k];
-                // the forward's sample position (rot_sample), bit for bit
-                const float px = pxc0 + (float)k;
-                const float pxc = px * c, pxns = px * (-s);
-                // One sample: its accumulator cell and the four weighted
-                // gradient values of its taps (use: its taps touch the tile).
-                struct Hit {
-                    int cell;  // byte offset of the sample's first accumulator
-                    float w00, w01, w10, w11;
-                    bool use;
+                const float pxc0 = (float)(f.c_lo + koff) - o;
+                uint64_t mask[NIT];
+#pragma unroll
+                for (int it = 0; it < NIT; it++)
+                    mask[it] = __builtin_amdgcn_ballot_w64(((mk[it] >> (8 * cc)) & 1) != 0);
+                struct Item {
+                    float g0, pxc, pxns, py;
+                    int d, len, q, row;  // d: row - first row of the range
+                    float4 eb, ed, ee;
+                    float2 ec;
                 };
-                // py = row - o, stepped by whole rows by the caller (integers
-                // or half-integers far below 2^23: exact)
-                auto sample = [&](int row, float py, int q) {
-                    Hit h;
-                    float x = pxc + py * s;
-                    float y = pxns + py * c;
+                auto load = [&](int it) {
+                    Item t = {};
+                    uint64_t m = mask[0];
+                    int before = 0;
+#pragma unroll
+                    for (int j = 1; j < NIT; j++)
+                        if (it >= j) {
+                            before += __builtin_popcountll(m);
+                            m = mask[j];
+                        }
+                    const uint64_t up = m >> 1;
+                    const int kl = __builtin_amdgcn_mbcnt_hi(
+                        (uint32_t)(up >> 32),
+                        __builtin_amdgcn_mbcnt_lo((uint32_t)up, before + (int)(m & 1) - 1));
+                    const int at = 16 * cc + kl;
+                    const float4 ea = sA[at];
+                    const int w = __float_as_int(ea.w);
+                    t.g0 = ea.x;
+                    t.row = __float_as_int(ea.z) + 3 * (it * kWave + lane);
+                    t.len = w & 255;
+                    t.d = t.row - (w >> 8);
+                    t.q = t.row - __float_as_int(ea.y);
+                    // the forward's sample position (rot_sample), bit for bit;
+                    // coordinates relative to o are integers or half-integers
+                    // far below 2^23: exact
+                    const float px = fmaf(3.0f, (float)kl, pxc0);
+                    t.pxc = px * c;
+                    t.pxns = px * (-s);
+                    t.py = (float)t.row - o;
+                    if (DO345) {
+                        t.eb = sB[at];
+                        t.ec = sC[at];
+                    }
+                    if (do12)
+                        t.ed = sD[at];
+                    if (do67)
+                        t.ee = sE[at];
+                    return t;
+                };
+                auto add = [&](const Item &t, int rc) {
+                    const bool in_range = (unsigned)(t.d + rc) <= (unsigned)t.len;
+                    const float py = t.py + (float)rc;
+                    const int row = t.row + rc, q = t.q + rc;
+                    float x = t.pxc + py * s;
+                    float y = t.pxns + py * c;
                     x = x + o;
                     y = y + o;
-                    int Xb = (int)(uint32_t)x, Yb = (int)(uint32_t)y;
-                    if constexpr (CHK) {
-                        const bool inb = __float_as_uint(x) < __float_as_uint(lim) &&
-                                         __float_as_uint(y) < __float_as_uint(lim);
-                        Xb = inb ? Xb : -8;
-                        Yb = inb ? Yb : -8;
-                    }
+                    const int Xb = (int)(uint32_t)x, Yb = (int)(uint32_t)y;
+                    const bool use = in_range &&
+                                     (!CHK || (__float_as_uint(x) < __float_as_uint(lim) &&
+                                               __float_as_uint(y) < __float_as_uint(lim)));
                     const float fx = __builtin_amdgcn_fractf(x);
                     const float fy = __builtin_amdgcn_fractf(y);
-                    const int xi = Xb - X0m, yi = Yb - Y0m;  // accumulator cell
-                    h.use = (unsigned)xi <= (unsigned)T && (unsigned)yi <= (unsigned)T;
                     // G(row): g0 + [row >= m] (g1 d + g2 d^2)
                     //   + [row > sm] sum_t (alpha_t W_t.re + beta_t W_t.im)[row - sm]
                     //   + [row == r6] c6 + [row == r7] c7
-                    float G = g0;
+                    float G = t.g0;
                     if (do12) {
-                        const int m = __float_as_int(ed.z);
+                        const int m = __float_as_int(t.ed.z);
                         const float d = (float)(row - m);
-                        const float hh = fmaf(d, fmaf(ed.y, d, ed.x), G);
+                        const float hh = fmaf(d, fmaf(t.ed.y, d, t.ed.x), G);
                         G = row >= m ? hh : G;
                     }
                     // (a wave whose active lanes all sit at or before their
                     // sm skips the term: a uniform branch)
-                    if (DO345 && __builtin_amdgcn_ballot_w64(q > 0) != 0) {
-                        // q = row - sm, stepped with the row; table entry 0 is
-                        // zero, so rows at or before sm add nothing; q <= n - 1
-                        // < tabn (row < n <= tabn)
-                        const int qc = q > 0 ? q : 0;
+                    if (DO345 && __builtin_amdgcn_ballot_w64(use && q > 0) != 0) {
+                        // table entry 0 is zero, so rows at or before sm add
+                        // nothing; q <= n - 1 < tabn in the rows that count
+                        const int qc = min(max(q, 0), tabn - 1);
                         const float4 w34 = reinterpret_cast<const float4 *>(s_tab)[qc];
                         const float2 w5 = s_tab[2 * tabn + qc];
-                        G = fmaf(eb.x, w34.x, G);
-                        G = fmaf(eb.y, w34.y, G);
-                        G = fmaf(eb.z, w34.z, G);
-                        G = fmaf(eb.w, w34.w, G);
-                        G = fmaf(ec.x, w5.x, G);
-                        G = fmaf(ec.y, w5.y, G);
+                        G = fmaf(t.eb.x, w34.x, G);
+                        G = fmaf(t.eb.y, w34.y, G);
+                        G = fmaf(t.eb.z, w34.z, G);
+                        G = fmaf(t.eb.w, w34.w, G);
+                        G = fmaf(t.ec.x, w5.x, G);
+                        G = fmaf(t.ec.y, w5.y, G);
                     }
                     if (do67) {
-                        G += row == __float_as_int(ee.x) ? ee.z : 0.0f;
-                        G += row == __float_as_int(ee.y) ? ee.w : 0.0f;
+                        G += row == __float_as_int(t.ee.x) ? t.ee.z : 0.0f;
+                        G += row == __float_as_int(t.ee.y) ? t.ee.w : 0.0f;
                     }
                     const float ofx = 1.0f - fx, ofy = 1.0f - fy;
                     const float ga = G * ofx, gb = G * fx;
-                    // byte offset 4 (xi P + yi) (read only where used, xi <= T):
-                    // a 24-bit multiply, which the compiler would otherwise
-                    // widen to a quarter-rate 32-bit one
-                    int xp;
-                    asm volatile("v_mul_u32_u24 %0, %1, %2" : "=v"(xp) : "n"(4 * P), "v"(xi));
-                    h.cell = xp + 4 * yi;
-                    h.w00 = ga * ofy;
-                    h.w01 = ga * fy;
-                    h.w10 = gb * ofy;
-                    h.w11 = gb * fy;
-                    return h;
-                };
-                for (int rc = 0; rc < 3; rc++) {
-                    // one residue class (column, row mod 3): its samples are
-                    // pairwise at least 3 apart, so their 2x2 tap footprints
-                    // are disjoint and every read-add-write of the class has
-                    // its own four targets
-                    const int roff = rc >= r3 ? rc - r3 : rc - r3 + 3;
-                    const int row0 = rlo + roff + 3 * jl;
-                    float py = (float)row0 - o;
-                    int q = row0 - sm;
-                    for (int row = row0; row <= rhi; row += 12, py += 12.0f, q += 12) {
-                        const Hit a = sample(row, py, q);
-                        if (a.use) {
-                            float *ca = reinterpret_cast<float *>(
-                                reinterpret_cast<char *>(acc) + a.cell);
-                            const float a00 = ca[0], a01 = ca[1], a10 = ca[P], a11 = ca[P + 1];
-                            ca[0] = a00 + a.w00;
-                            ca[1] = a01 + a.w01;
-                            ca[P] = a10 + a.w10;
-                            ca[P + 1] = a11 + a.w11;
-                        }
+                    if (use) {
+                        // cell (Xb - X0m) P + Yb - Y0m: a 24-bit multiply,
+                        // which the compiler would otherwise widen to a
+                        // quarter-rate 32-bit one
+                        int xp;
+                        asm volatile("v_mul_u32_u24 %0, %1, %2" : "=v"(xp) : "n"(4 * P), "v"(Xb));
+                        float *ca = reinterpret_cast<float *>(
+                            reinterpret_cast<char *>(acc) +
+                            (xp + 4 * Yb - 4 * (X0m * P + Y0m)));
+                        const float a00 = ca[0], a01 = ca[1], a10 = ca[P], a11 = ca[P + 1];
+                        ca[0] = a00 + ga * ofy;
+                        ca[1] = a01 + ga * fy;
+                        ca[P] = a10 + gb * ofy;
+                        ca[P + 1] = a11 + gb * fy;
                     }
+                };
+                if (N <= kWave) {
+                    if (N > 0) {
+                        const Item t0 = load(0);
+#pragma unroll
+                        for (int rc = 0; rc < 3; rc++)
+                            add(t0, rc);
+                    }
+                } else if (N <= 2 * kWave) {
+                    const Item t0 = load(0), t1 = load(1);
+#pragma unroll
+                    for (int rc = 0; rc < 3; rc++) {
+                        add(t0, rc);
+                        add(t1, rc);
+                    }
+                } else {
+                    for (int rc = 0; rc < 3; rc++)
+                        for (int it = 0; it * kWave < N && it < NIT; it++)
+                            add(load(it), rc);
                 }
             }
         };
@@ -3084,7 +3158,7 @@ __device__ __forceinline__ void gather_tile_wave(const GatherImg &im, const floa
 #pragma unroll
             for (int i = 0; i < S::NPIX; i++) {
                 const int p = lane + kWave * i;
-                accd[i] += (double)acc[(p / T + 1) * P + p % T + 1];
+                accd[i] += (double)acc[(p / TY + 2) * P + p % TY + 2];
             }
             wave_lds_sync();
             for (int i = lane; i < S::ACC / 4; i += kWave)
@@ -3095,7 +3169,7 @@ __device__ __forceinline__ void gather_tile_wave(const GatherImg &im, const floa
 #pragma unroll
     for (int i = 0; i < S::NPIX; i++) {
         const int p = lane + kWave * i;
-        const int X = X0 + p / T, Y = Y0 + p % T;
+        const int X = X0 + p / TY, Y = Y0 + p % TY;
         if (X < n && Y < n)
             im.out[(size_t)X * n + Y] = (float)accd[i];
     }
@@ -3124,10 +3198,11 @@ __global__ __launch_bounds__(1024) void gather_kernel(GatherParams p)
     float *wl = gather_lds(smem, p.tab345, p.n, DO345, words);
     const int waves = blockDim.x / kWave;
     const int item = blockIdx.x * waves + wave_id();
-    const int tn = (p.n + T - 1) / T;
-    if (item >= tn * tn * p.groups)
+    const int tiles = gather_tiles(p.n, T);
+    if (item >= tiles * p.groups)
         return;
-    const int g = item / (tn * tn), tile = item - g * tn * tn;
+    const int g = item / tiles, tile = item - g * tiles;
+    const int tny = (p.n + gather_ty(T) - 1) / gather_ty(T);
     const int a0 = (int)((long long)p.A * g / p.groups);
     const int a1 = (int)((long long)p.A * (g + 1) / p.groups);
     GatherImg im;
@@ -3136,7 +3211,8 @@ __global__ __launch_bounds__(1024) void gather_kernel(GatherParams p)
     im.out = p.groups > 1 ? p.part + (size_t)g * p.n * p.n : p.dimg;
     im.n = p.n;
     gather_tile_wave<T, DO345, DO12>(im, p.trig, reinterpret_cast<const float2 *>(smem), p.n,
-                                     a0, a1, tile / tn * T, tile % tn * T, wl);
+                                     a0, a1, tile / tny * gather_tx(T),
+                                     tile % tny * gather_ty(T), wl);
 }
 
 // dimg = sum over angle groups of the partial images, in group order.
@@ -3167,7 +3243,7 @@ __global__ __launch_bounds__(1024) void gather_batched_kernel(BatchAdjointParams
                              [](const BatchImage &b) { return b.tile0; });
     const BatchImage &bi = p.images[k];
     const int n = bi.n;
-    const int tn = (n + T - 1) / T;
+    const int tny = (n + gather_ty(T) - 1) / gather_ty(T);
     const int tile = item - bi.tile0;
     GatherImg im;
     im.rec = bi.rec;
@@ -3175,7 +3251,8 @@ __global__ __launch_bounds__(1024) void gather_batched_kernel(BatchAdjointParams
     im.out = bi.dimg;
     im.n = n;
     gather_tile_wave<T, DO345, DO12>(im, p.trig, reinterpret_cast<const float2 *>(smem),
-                                     p.tabn, 0, p.A, tile / tn * T, tile % tn * T, wl);
+                                     p.tabn, 0, p.A, tile / tny * gather_tx(T),
+                                     tile % tny * gather_ty(T), wl);
 }
 
 // dS = J_P^T dC for every sinogram column (P1: sign differences; P2: one-hot
@@ -3899,8 +3976,7 @@ hipError_t launch_gather(const GatherParams &p, hipStream_t s)
     if (p.tile != kGatherTile || p.waves < 1 || p.waves > 16 || p.groups < 1 ||
         (p.groups > 1 && !p.part))
         return hipErrorInvalidValue;
-    const int tn = (p.n + p.tile - 1) / p.tile;
-    const int items = tn * tn * p.groups;
+    const int items = gather_tiles(p.n, p.tile) * p.groups;
     const int blocks = (items + p.waves - 1) / p.waves;
     const size_t shm = gather_lds_bytes(p.tile, p.waves, p.n, p.do345, p.do12,
                                         p.rec67 != nullptr);
