@@ -173,11 +173,18 @@ __global__ __launch_bounds__(kNgThreads) void nos_gemm_kernel(NosGemmBatch bt, i
 // MFMA operands straight from global memory, 16 consecutive doubles per
 // quarter wave, keeping kNsDepth reduction steps in flight.  A workgroup
 // owns a 32 x 32 output block (2 x 2 MFMA blocks); its four waves take
-// consecutive quarters of the reduction and wave 0 adds the other three's
-// partial sums from LDS in wave order.  Workgroup g takes matrix g % count:
+// consecutive quarters of the reduction and put their partial sums into LDS,
+// where each wave adds one MFMA block's in wave order and stores it, and its
+// mirror image, with 16 consecutive doubles per quarter wave (wave 0 alone,
+// with scattered stores, was a third of the time).  The loads keep eight
+// steps in flight: a wave has 22 steps of a 360-row product, and its operands
+// come from beyond the L2 after the previous product's launch.
+// Workgroup g takes matrix g % count:
 // workgroups go to the eight XCDs in turn, so a batch of eight keeps each
 // matrix's operands in one XCD's L2.
-constexpr int kNsDepth = 4;
+constexpr int kNsDepth = 8;
+constexpr int kNsRow = 17;              // doubles per row of a 16 x 16 block in LDS
+constexpr int kNsBlock = 16 * kNsRow;
 constexpr int kNsWaves = kNgThreads / 64;
 
 // POLY: the product is S S of a polynomial step (A = B = S, strided batch);
@@ -192,7 +199,7 @@ __global__ __launch_bounds__(kNgThreads) void nos_gemm_symb_kernel(NosGemmBatch 
                                                                    double alpha, double beta,
                                                                    int bm, NosPolyOut po)
 {
-    __shared__ double s_part[kNsWaves - 1][16][64];
+    __shared__ double s_part[kNsWaves][4][kNsBlock];  // [wave][MFMA block][row][column]
     const int job = blockIdx.x % count;
     const int blk = blockIdx.x / count;
     int bi, bj;
@@ -268,60 +275,72 @@ __global__ __launch_bounds__(kNgThreads) void nos_gemm_symb_kernel(NosGemmBatch 
             }
         }
     }
-    if (w > 0) {
-#pragma unroll
-        for (int r = 0; r < 2; r++)
-#pragma unroll
-            for (int c = 0; c < 2; c++)
-#pragma unroll
-                for (int v = 0; v < 4; v++)
-                    s_part[w - 1][(r * 2 + c) * 4 + v][lane] = acc[r][c][v];
-    }
-    __syncthreads();
-    if (w > 0)
-        return;
-#pragma unroll
-    for (int q = 0; q < kNsWaves - 1; q++)
-#pragma unroll
-        for (int r = 0; r < 2; r++)
-#pragma unroll
-            for (int c = 0; c < 2; c++)
-#pragma unroll
-                for (int v = 0; v < 4; v++)
-                    acc[r][c][v] += s_part[q][(r * 2 + c) * 4 + v][lane];
 #pragma unroll
     for (int r = 0; r < 2; r++)
 #pragma unroll
         for (int c = 0; c < 2; c++)
 #pragma unroll
-            for (int v = 0; v < 4; v++) {
-                const int row = bi * 32 + r * 16 + 4 * v + k4;
-                const int col = bj * 32 + c * 16 + r16;
-                if (row >= m || col >= n || (SYM && row < col))
-                    continue;
-                const size_t o = row + (size_t)col * ldc;
-                const double val = beta != 0.0 ? alpha * acc[r][c][v] + beta * C[o]
-                                                : alpha * acc[r][c][v];
-                C[o] = val;
-                if (SYM && row != col)
-                    C[col + (size_t)row * ldc] = val;
-                if (POLY) {
-                    const double sc = po.scale ? po.scale[job] : 1.0;
-                    const double rr = po.r ? po.r[job] : 1.0;
-                    const double a = sc * A[row + (size_t)col * lda], b = sc * sc * val;
-                    const double d = row == col ? po.c[0] : 0.0;
-                    const double tv = sc * sc * rr * (po.c[3] * a + po.c[4] * b);
-                    const double qv = rr * (d + po.c[1] * a + po.c[2] * b);
-                    const size_t off = (size_t)job * po.stride;
-                    po.T[off + o] = tv;
-                    po.Q[off + o] = qv;
-                    if (row != col) {
-                        const size_t om = col + (size_t)row * ldc;
-                        po.T[off + om] = tv;
-                        po.Q[off + om] = qv;
-                    }
-                }
-            }
+            for (int v = 0; v < 4; v++)
+                s_part[w][r * 2 + c][(4 * v + k4) * kNsRow + r16] = acc[r][c][v];
+    __syncthreads();
+    // this wave's MFMA block, four rows of lanes along the rows of C
+    const int row0 = bi * 32 + (w >> 1) * 16, col0 = bj * 32 + (w & 1) * 16;
+    double out[4], tv[4], qv[4];
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+        const int at = r16 * kNsRow + 4 * t + k4;
+        double sum = s_part[0][w][at];
+#pragma unroll
+        for (int q = 1; q < kNsWaves; q++)
+            sum += s_part[q][w][at];
+        const int row = row0 + r16, col = col0 + 4 * t + k4;
+        out[t] = tv[t] = qv[t] = 0.0;
+        if (row >= m || col >= n || (SYM && row < col))
+            continue;
+        const size_t o = row + (size_t)col * ldc;
+        const double val = beta != 0.0 ? alpha * sum + beta * C[o] : alpha * sum;
+        C[o] = val;
+        out[t] = val;
+        if (POLY) {
+            const double sc = po.scale ? po.scale[job] : 1.0;
+            const double rr = po.r ? po.r[job] : 1.0;
+            const double a = sc * A[row + (size_t)col * lda], b = sc * sc * val;
+            const double d = row == col ? po.c[0] : 0.0;
+            tv[t] = sc * sc * rr * (po.c[3] * a + po.c[4] * b);
+            qv[t] = rr * (d + po.c[1] * a + po.c[2] * b);
+            const size_t off = (size_t)job * po.stride;
+            po.T[off + o] = tv[t];
+            po.Q[off + o] = qv[t];
+        }
+    }
+    if (!SYM)
+        return;
+    // the mirror image, along the rows of the other triangle
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+        const int at = r16 * kNsRow + 4 * t + k4;
+        s_part[0][w][at] = out[t];
+        if (POLY) {
+            s_part[1][w][at] = tv[t];
+            s_part[2][w][at] = qv[t];
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+        const int at = (4 * t + k4) * kNsRow + r16;
+        const int row = row0 + 4 * t + k4, col = col0 + r16;
+        if (row >= m || col >= n || row <= col)
+            continue;
+        const size_t om = col + (size_t)row * ldc;
+        C[om] = s_part[0][w][at];
+        if (POLY) {
+            const size_t off = (size_t)job * po.stride;
+            po.T[off + om] = s_part[1][w][at];
+            po.Q[off + om] = s_part[2][w][at];
+        }
+    }
 }
 
 }  // namespace
