@@ -2776,10 +2776,12 @@ __global__ __launch_bounds__(kBlock) void records_batched_kernel(BatchAdjointPar
 // without gaps: a work item is three consecutive rows of a column, starting
 // at a multiple of three, and the items of every third column (a column
 // class) are numbered through.  A lane finds the column of its item by
-// counting the bits of a wave-uniform mask of column starts.  The old layout
-// (16 columns x 4 rows of a parallelogram, one slab) had 1.7 to 2.5 lane
-// slots per sample; this one has 1.1.  Each sample is evaluated exactly as
-// the forward evaluates it
+// counting the bits of a wave-uniform mask of column starts.  Lanes laid out
+// as 16 columns x 4 rows of a parallelogram cut by one slab had 1.7 to 2.5
+// slots per sample; this has 1.1 (48 images x 720 angles, T0 and T3..T5:
+// 76.5 -> 58.6 ms; VALU issue is 74 % of that and the LDS busy 78 %, half of
+// it bank conflicts of the scattered accumulators).  Each sample is evaluated
+// exactly as the forward evaluates it
 // (rot_sample's float operations: coordinates, strict bounds, truncated taps
 // and modf fractions), its rotated-domain gradient G(row) comes from its
 // column's line record, and G times each of the four tap weights is added

@@ -178,7 +178,8 @@ __global__ __launch_bounds__(kNgThreads) void nos_gemm_kernel(NosGemmBatch bt, i
 // mirror image, with 16 consecutive doubles per quarter wave (wave 0 alone,
 // with scattered stores, was a third of the time).  The loads keep eight
 // steps in flight: a wave has 22 steps of a 360-row product, and its operands
-// come from beyond the L2 after the previous product's launch.
+// come from beyond the L2 after the previous product's launch.  Both took a
+// batch of eight 360 x 360 products from 22.4 to 20.4 us.
 // Workgroup g takes matrix g % count:
 // workgroups go to the eight XCDs in turn, so a batch of eight keeps each
 // matrix's operands in one XCD's L2.
