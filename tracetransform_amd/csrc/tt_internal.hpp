@@ -371,7 +371,7 @@ hipError_t launch_circus_vjp(const CircusVjpParams &p, hipStream_t s);
 // bilinear sample can be negative, a positive value below 2^-96, infinite or
 // NaN, and the kernels take the library's square root), else 0.  bbox
 // holds kBboxInts words: the result, then scratch for the blocks' boxes.
-constexpr int kPairBlocks = 512;  // at most, per image
+constexpr int kPairBlocks = 1024;  // at most, per image
 constexpr int kBboxInts = 8 * (1 + kPairBlocks);
 __host__ __device__ inline size_t image_pair_count(int n)
 {
