@@ -247,7 +247,8 @@ TT_API tt_status tt_batched_launch_shape(tt_context *ctx, int *waves_per_block,
  *     gather_waves waves per workgroup (1..16), of the batched backward's
  *     transposed rotation.
  * A line's results and a pixel's gradient are the same bits whatever the
- * tiles.  Zero fields mean the default (1x64, class 32, the most waves that
+ * tiles.  A workgroup takes fewer waves where the LDS has no room for
+ * gather_waves of them (tt_batched_tiles tells).  Zero fields mean the default (1x64, class 32, the most waves that
  * fit the LDS) or, with autotuning, the tuned choice. */
 typedef struct tt_tiles {
     int32_t line_angles;

@@ -251,3 +251,25 @@ def test_every_tile_gives_the_same_bits(oracle, gpu):
             core.set_tiles(0, gather=(8, 4))
     finally:
         core.set_tiles(0)
+
+
+@pytest.mark.parametrize("n,codes,fit", [(1162, [0, 1, 3], 16), (1163, [0, 1, 3], 15),
+                                         (1800, [0, 1, 3], 14), (1800, [0, 3], 15),
+                                         (1800, [0, 1], 16)])
+def test_forced_gather_waves_beyond_the_lds(gpu, n, codes, fit):
+    # a forced shape whose waves the LDS has no room for runs with those that
+    # fit: the same gradient, and the shape reported
+    img = torch.from_numpy(np.random.default_rng(n).random((n, n), dtype=np.float32)).cuda()
+    b = core.BatchBackward([img], 4, 90.0, codes, [(1,)])
+    b.dcircus_all.fill_(0.5)
+    try:
+        core.set_tiles(0, gather=(32, 4))
+        ref = b.run()[0].clone()
+        core.set_tiles(0, gather=(32, 16))
+        got = b.run()[0].clone()
+        t = core.batched_tiles(0)
+        assert (t["gather_tile"], t["gather_waves"]) == (32, fit)
+        assert torch.equal(got, ref)
+        assert float(ref.abs().max()) > 0
+    finally:
+        core.set_tiles(0)

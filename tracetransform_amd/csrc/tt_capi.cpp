@@ -1006,6 +1006,15 @@ int gather_waves_max(int T, int tabn, bool do345, bool do12)
     return 0;
 }
 
+// Waves per workgroup of the batched gather: the forced count, as far as its
+// LDS fits (class 32 with T1..T5: 16 waves up to 1162 rows, 15 up to 1516, 14
+// beyond), or the most that fit.
+int gather_waves(int T, int tabn, bool do345, bool do12, int forced)
+{
+    const int most = gather_waves_max(T, tabn, do345, do12);
+    return forced > 0 && forced < most ? forced : most;
+}
+
 // Workgroup offsets of a DFT job list for its launch's tile shape (larger
 // tiles when the list is large enough); returns the workgroups.
 int layout_dft_jobs(std::vector<ttk::DftJob> &jobs, bool forward, int *bm, int *bn)
@@ -2325,11 +2334,8 @@ TT_API tt_status tt_backward_batched(tt_context *ctx, const tt_image_grad *image
             TT_HIP(P.y.ensure(sizeof(float) * spec_tot));
         // gather tile: forced, class 32, or tuned below
         int gtile = ctx->force.gather_tile > 0 ? ctx->force.gather_tile : 32;
-        int gwaves = ctx->force.gather_waves > 0 ? ctx->force.gather_waves
-                                                 : gather_waves_max(gtile, nmax, do345, do12);
-        TT_CHECK(gwaves >= 1 && ttk::gather_lds_bytes(gtile, gwaves, nmax, do345, do12,
-                                                      false) <= kLdsLimit,
-                 "gather tile %d with %d waves per workgroup exceeds the LDS", gtile, gwaves);
+        int gwaves = gather_waves(gtile, nmax, do345, do12, ctx->force.gather_waves);
+        TT_CHECK(gwaves >= 1, "gather tile %d exceeds the LDS at %d rows", gtile, nmax);
         std::vector<ttk::DftJob> fj, sj, bj;
         int ftiles = 0, btiles = 0;
         size_t so = 0;
@@ -2507,17 +2513,18 @@ TT_API tt_status tt_backward_batched(tt_context *ctx, const tt_image_grad *image
         P.gather_waves = gwaves;
         if (ctx->autotune && ctx->force.gather_tile == 0) {
             // one eager backward writes the line records; then the gather
-            // alone with each candidate tile (the most waves that fit, and
-            // half as many), the mean of two runs after a first
+            // alone with each candidate tile (the forced waves, or the most
+            // that fit and half as many), the mean of two runs after a first
             TT_HIP(enqueue_backward(ctx, P, own, false));
             hipEvent_t e0, e1;
             TT_HIP(hipEventCreate(&e0));
             TT_HIP(hipEventCreate(&e1));
             float best = 1e30f;
             for (int T : {32, 16}) {
-                const int wmax = gather_waves_max(T, nmax, do345, do12);
-                for (int w : {wmax, wmax / 2}) {
-                    if (w < 1 || (ctx->force.gather_waves > 0 && w != ctx->force.gather_waves))
+                const int forced = ctx->force.gather_waves;
+                const int wmax = gather_waves(T, nmax, do345, do12, forced);
+                for (int w : {wmax, forced > 0 ? 0 : wmax / 2}) {
+                    if (w < 1)
                         continue;
                     P.ap.tiles = layout_gather_tiles(d, T);
                     TT_HIP(hipMemcpy(B.desc.ptr, d.data(), sizeof(ttk::BatchImage) * nimg,
