@@ -87,3 +87,22 @@ def test_t6_t7_widths(oracle, gpu, side):
     assert_same_indices("t7_rank", aux["t7_rank"].cpu(), oaux["t7_rank"])
     assert_same_indices("t7_src", aux["t7_src"].cpu(), oaux["t7_src"])
     assert np.array_equal(sino.cpu().numpy(), o)
+
+
+@pytest.mark.parametrize("n", [3, 64, 513, 2048, 2049])
+@pytest.mark.parametrize("codes", [[1, 0], [0, 3], [0, 3, 1, 0], [2, 0, 1], [0, 2]])
+def test_lists_with_hermite(oracle, gpu, n, codes):
+    # Hermite entries with P1 and P3 in the workgroup kernel, and P1..P3 in the
+    # wave kernel beside them where P2 is in the list
+    rng = np.random.default_rng(10 * n + len(codes))
+    cols = (rng.random((5, n)) * 3).astype(np.float32)
+    pf = [(c,) if c else (0, 1 + q, n // 2) for q, c in enumerate(codes)]
+    got, rank = core.circus(torch.from_numpy(cols[None]).cuda(), pf, with_p2_rank=True)
+    _, aux = oracle.circus(cols, n, 5, pf)
+    want = oracle.circus_f64(cols, n, 5, pf, aux["p2_src"], geometry=1)
+    got = got[0].cpu().numpy()
+    if 2 in codes:
+        q = codes.index(2)
+        assert_same_indices("rank", rank[0, q].cpu(), aux["p2_rank"][q])
+    for q in range(len(pf)):
+        assert normwise_err(got[q], want[q]) <= 1e-5, pf[q]
