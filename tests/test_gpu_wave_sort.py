@@ -106,3 +106,11 @@ def test_lists_with_hermite(oracle, gpu, n, codes):
         assert_same_indices("rank", rank[0, q].cpu(), aux["p2_rank"][q])
     for q in range(len(pf)):
         assert normwise_err(got[q], want[q]) <= 1e-5, pf[q]
+
+
+@pytest.mark.parametrize("n", [2, 3, 64, 65, 66, 449, 512, 513, 514, 577, 1025, 1026, 2047, 2048])
+def test_p1_rows(gpu, n):
+    # whole numbers: every sum is exact, a term left out or taken twice shows
+    x = np.random.default_rng(n).integers(-40, 41, (3, n)).astype(np.float32)
+    got = core.circus(torch.from_numpy(x[None]).cuda(), [(1,)])[0, 0].cpu().numpy()
+    assert np.array_equal(got, np.abs(np.diff(x, axis=1)).sum(axis=1))
