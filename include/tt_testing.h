@@ -17,6 +17,10 @@ extern "C" {
  * exercised; a negative value removes the limit. */
 TT_API tt_status tt_testing_fail_allocations(long long allowed);
 
+/* Makes every workspace allocation of more than `bytes` fail as out of memory,
+ * as on a device without room for it; 0 removes the limit. */
+TT_API tt_status tt_testing_limit_allocation(size_t bytes);
+
 /* Compares the sort kernel's short square root (v_sqrt_f32 and one residual
  * test per neighbour) with the correctly rounded sqrtf on the GPU for the
  * float bit patterns [lo, lo + count), skipping its documented exceptions

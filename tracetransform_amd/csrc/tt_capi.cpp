@@ -60,6 +60,9 @@ tt_status fail(tt_status st, const char *fmt, ...)
 // Allocation-failure hook (tt_testing_fail_allocations): the number of
 // workspace allocations still allowed to succeed, or -1 (no limit).
 std::atomic<long long> g_alloc_budget{-1};
+// The largest workspace allocation that may succeed
+// (tt_testing_limit_allocation), or 0 (no limit).
+std::atomic<size_t> g_alloc_limit{0};
 
 hipError_t workspace_malloc(void **ptr, size_t bytes)
 {
@@ -70,7 +73,13 @@ hipError_t workspace_malloc(void **ptr, size_t bytes)
         if (g_alloc_budget.compare_exchange_weak(left, left - 1))
             break;
     }
-    return hipMalloc(ptr, bytes);
+    const size_t limit = g_alloc_limit.load();
+    if (limit > 0 && bytes > limit)
+        return hipErrorOutOfMemory;
+    hipError_t e = hipMalloc(ptr, bytes);
+    if (e != hipSuccess)
+        (void)hipGetLastError();  // returned here: no later launch reports it
+    return e;
 }
 
 struct DevBuf {
@@ -276,17 +285,41 @@ struct KernelTimer {
     }
 };
 
+// Launches stage after stage on a stream, each bracketed by the timer where
+// there is one; after an error nothing more.
+struct Stages {
+    KernelTimer *timer;
+    hipStream_t stream;
+    hipError_t err = hipSuccess;
+    template <class F> void operator()(int kind, F launch)
+    {
+        if (err == hipSuccess && timer)
+            err = timer->begin(kind, stream);
+        if (err == hipSuccess)
+            err = launch();
+        if (err == hipSuccess && timer)
+            err = timer->end(stream);
+    }
+};
+
 // A batch ready to replay: descriptors, workspaces and the captured graph.
 // It owns copies of the tables it uses so later single-image calls (which
 // rewrite the context's tables) cannot change what the graph reads.
 struct BatchPlan {
+    // Images first .. first + count - 1 of the descriptors (largest first, so
+    // nmax is the first one's side), whose pixel pairs are in the workspace
+    // together: their pair pass and their line items are one launch each.
+    struct LineGroup {
+        int first, count, items, nmax;
+    };
+    std::vector<LineGroup> groups;
     std::vector<int64_t> key;
     DevBuf desc, pairs, trig, tab, counter, bbox, ckpt, spec, jobs;
     ttk::DftParams dft = {};      // P3 spectra of every image (jobs in `jobs`)
     // launch parameters of the captured stages (reused for timed eager runs)
     ttk::BatchSinoParams sp = {};
     ttk::BatchCircusParams cp = {};
-    int nimg = 0, nmax = 0;
+    int nmax = 0;
     bool need_x = false, need_s = false, do345 = false;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
@@ -708,7 +741,7 @@ tt_status image_pairs(tt_context *ctx, const float *d_image, int n)
 {
     const size_t cnt = ttk::image_pair_count(n);
     TT_HIP(ctx->pairs.ensure(2 * sizeof(float2) * cnt));
-    TT_HIP(ctx->bbox.ensure(ttk::kBboxInts * sizeof(int)));
+    TT_HIP(ctx->bbox.ensure(ttk::bbox_ints(n) * sizeof(int)));
     TT_HIP(ctx->timer.begin(TT_KERNEL_AUX, ctx->stream));
     TT_HIP(ttk::launch_image_pairs(d_image, n, ctx->pairs.as<float2>(),
                                    ctx->pairs.as<float2>() + cnt, ctx->bbox.as<int>(),
@@ -975,15 +1008,66 @@ LineTile line_tile_of(const tt_context *ctx)
 }
 
 // Wave items of the batched line kernel with tile t: each image's column
-// tiles and first item (descriptors in launch order); returns the total.
-int layout_line_items(std::vector<ttk::BatchImage> &d, int A, LineTile t)
+// tiles and its first item in its group's launch, and the groups' totals.
+void layout_line_items(std::vector<ttk::BatchImage> &d,
+                       std::vector<BatchPlan::LineGroup> &groups, int A, LineTile t)
 {
-    int items = 0;
-    for (ttk::BatchImage &b : d) {
-        b.item0 = items;
-        items += ttk::line_tile_items(b.n, A, t.a, t.c, &b.nb);
+    for (BatchPlan::LineGroup &g : groups) {
+        g.items = 0;
+        for (int k = g.first; k < g.first + g.count; k++) {
+            d[k].item0 = g.items;
+            g.items += ttk::line_tile_items(d[k].n, A, t.a, t.c, &d[k].nb);
+        }
     }
-    return items;
+}
+
+// Bytes of an image's pixel pairs in both directions.
+size_t pair_bytes(int n) { return 2 * sizeof(float2) * ttk::image_pair_count(n); }
+
+// Pixel pairs of a batch in the workspace at once, 3 % of the device's memory.
+// A group's line kernel ends in a nearly empty round: 520 images of 1449 rows
+// at 8 angles take 17.3 ms in groups of 8 GiB, 16.9 in one; 160 of them 5.7 ms
+// in groups of 2 GiB, 5.3 in one.
+constexpr size_t kPairCap = (size_t)8 << 30;
+
+// The pair workspace of a batch (descriptors largest first): all of it up to
+// kPairCap, else groups of images that share it one after the other, at least
+// one image each.  Where the device has no room for it, smaller groups: pairs
+// are four times their images' bytes, and a batch that fits without them must
+// not fail for them.
+hipError_t reserve_pairs(BatchPlan &B, std::vector<ttk::BatchImage> &d)
+{
+    size_t most = 0;
+    for (size_t cap = kPairCap;; cap = most / 2) {
+        B.groups.clear();
+        size_t used = 0;
+        most = 0;
+        for (int k = 0; k < (int)d.size(); k++) {
+            const size_t bytes = pair_bytes(d[k].n);
+            if (B.groups.empty() || used + bytes > cap) {
+                B.groups.push_back({k, 0, 0, d[k].n});
+                used = 0;
+            }
+            B.groups.back().count++;
+            used += bytes;
+            most = used > most ? used : most;
+        }
+        const hipError_t e = B.pairs.ensure(most);
+        if (e == hipSuccess)
+            break;
+        if (e != hipErrorOutOfMemory || most <= pair_bytes(d[0].n))
+            return e;
+    }
+    for (const BatchPlan::LineGroup &g : B.groups) {
+        float2 *at = B.pairs.as<float2>();
+        for (int k = g.first; k < g.first + g.count; k++) {
+            const size_t cnt = ttk::image_pair_count(d[k].n);
+            d[k].pair = at;
+            d[k].pairT = at + cnt;
+            at += 2 * cnt;
+        }
+    }
+    return hipSuccess;
 }
 
 // First gather tile of each image for tiles of class T; returns the total.
@@ -1033,43 +1117,49 @@ int layout_dft_jobs(std::vector<ttk::DftJob> &jobs, bool forward, int *bm, int *
     return tiles;
 }
 
+// Pair passes and line kernels of a batch, group after group: a group's pair
+// pass overwrites the last one's pairs once its line kernel, ahead of it on the
+// stream, is done.
+void enqueue_lines(Stages &stage, const std::vector<BatchPlan::LineGroup> &groups,
+                   const ttk::BatchSinoParams &sp, bool need_x, bool need_s, bool do345,
+                   int wpb, int blocks, bool with_pairs)
+{
+    const hipStream_t st = stage.stream;
+    for (const BatchPlan::LineGroup &g : groups) {
+        ttk::BatchSinoParams q = sp;
+        q.images = sp.images + g.first;
+        q.nimg = g.count;
+        q.items = g.items;
+        if (with_pairs)
+            stage(TT_KERNEL_AUX, [&] {
+                return ttk::launch_image_pairs_batched(q.images, q.nimg, g.nmax, q.counter, st);
+            });
+        stage(TT_KERNEL_SINO_T05, [&] {
+            // (the pair pass has zeroed the work counter)
+            hipError_t r = with_pairs ? hipSuccess : ttk::launch_reset_counter(q.counter, st);
+            return r == hipSuccess
+                       ? ttk::launch_sino_t05_batched(q, need_x, need_s, do345, wpb, blocks, st)
+                       : r;
+        });
+    }
+}
+
 // Enqueue the batched pass (used for capture and for autotuning).
 // The batched forward's stages on st.  timed: each stage bracketed by the
 // context's kernel timer (never while a graph is being captured).
 hipError_t enqueue_batch(tt_context *ctx, const ttk::BatchSinoParams &sp,
-                         const ttk::BatchCircusParams &cp, int nimg, int nmax,
+                         const ttk::BatchCircusParams &cp, int nmax,
                          bool need_x, bool need_s, bool do345, int wpb, int blocks,
                          bool with_pairs, bool with_circus, hipStream_t st,
                          bool timed = false)
 {
-    KernelTimer *T = timed ? &ctx->timer : nullptr;
-    hipError_t e = hipSuccess;
-    auto stage = [&](int kind, auto launch) {
-        if (e != hipSuccess)
-            return;
-        if (T)
-            e = T->begin(kind, st);
-        if (e == hipSuccess)
-            e = launch();
-        if (T && e == hipSuccess)
-            e = T->end(st);
-    };
-    if (with_pairs)
-        stage(TT_KERNEL_AUX, [&] {
-            return ttk::launch_image_pairs_batched(sp.images, nimg, nmax, sp.counter, st);
-        });
-    stage(TT_KERNEL_SINO_T05, [&] {
-        // (the pair pass has zeroed the work counter)
-        hipError_t r = with_pairs ? hipSuccess : ttk::launch_reset_counter(sp.counter, st);
-        return r == hipSuccess
-                   ? ttk::launch_sino_t05_batched(sp, need_x, need_s, do345, wpb, blocks, st)
-                   : r;
-    });
+    Stages stage = {timed ? &ctx->timer : nullptr, st};
+    enqueue_lines(stage, ctx->batch.groups, sp, need_x, need_s, do345, wpb, blocks, with_pairs);
     if (with_circus && ctx->batch.dft.tiles > 0)
         stage(TT_KERNEL_P3_DFT, [&] { return ttk::launch_dft_gemm(ctx->batch.dft, true, nmax, st); });
     if (with_circus && cp.np > 0)
         stage(TT_KERNEL_CIRCUS, [&] { return ttk::launch_circus_batched(cp, st); });
-    return e;
+    return stage.err;
 }
 
 // The batched backward's stages on st (timed as enqueue_batch).
@@ -1077,28 +1167,11 @@ hipError_t enqueue_backward(tt_context *ctx, const BackwardPlan &P, hipStream_t 
                             bool timed)
 {
     const BatchPlan &B = P.g;
-    KernelTimer *T = timed ? &ctx->timer : nullptr;
-    hipError_t e = hipSuccess;
-    auto stage = [&](int kind, auto launch) {
-        if (e != hipSuccess)
-            return;
-        if (T)
-            e = T->begin(kind, st);
-        if (e == hipSuccess)
-            e = launch();
-        if (T && e == hipSuccess)
-            e = T->end(st);
-    };
+    Stages stage = {timed ? &ctx->timer : nullptr, st};
     const bool p3 = P.p3s.np3 > 0;
     if (!P.saved) {
-        stage(TT_KERNEL_AUX, [&] {
-            return ttk::launch_image_pairs_batched(B.sp.images, B.nimg, B.nmax, B.sp.counter,
-                                                   st);
-        });
-        stage(TT_KERNEL_SINO_T05, [&] {  // (the pair pass has zeroed the work counter)
-            return ttk::launch_sino_t05_batched(B.sp, true, true, B.do345, B.waves_per_block,
-                                                B.blocks, st);
-        });
+        enqueue_lines(stage, B.groups, B.sp, true, true, B.do345, B.waves_per_block, B.blocks,
+                      true);
         if (p3)
             stage(TT_KERNEL_P3_DFT, [&] { return ttk::launch_dft_gemm(P.fdp, true, B.nmax, st); });
         if (P.p2src_on)
@@ -1114,7 +1187,7 @@ hipError_t enqueue_backward(tt_context *ctx, const BackwardPlan &P, hipStream_t 
     stage(TT_KERNEL_GATHER, [&] {
         return ttk::launch_gather_batched(P.ap, P.gather_tile, P.gather_waves, st);
     });
-    return e;
+    return stage.err;
 }
 
 }  // namespace
@@ -1256,14 +1329,13 @@ TT_API tt_status tt_forward_batched(tt_context *ctx, const tt_image *images,
             return images[a].n > images[b].n;
         });
         std::vector<ttk::BatchImage> d(nimg);
-        size_t tot = 0;
-        for (int i = 0; i < nimg; i++)
-            tot += 2 * ttk::image_pair_count(images[i].n);
-        TT_HIP(B.pairs.ensure(sizeof(float2) * tot));
-        TT_HIP(B.bbox.ensure(ttk::kBboxInts * sizeof(int) * (size_t)nimg));
-        size_t ck = 0;  // the line kernel's walk checkpoints, image after image
-        for (int i = 0; i < nimg; i++)
+        // the box scratch and the line kernel's walk checkpoints, image after image
+        size_t bb = 0, ck = 0;
+        for (int i = 0; i < nimg; i++) {
+            bb += ttk::bbox_ints(images[i].n);
             ck += (size_t)ttk::sino_ckpt_blocks(images[i].n) * images[i].n * n_angles;
+        }
+        TT_HIP(B.bbox.ensure(sizeof(int) * bb));
         TT_HIP(B.ckpt.ensure(sizeof(float2) * ck));
         bool p3 = false;
         for (int q = 0; q < np; q++)
@@ -1275,7 +1347,7 @@ TT_API tt_status tt_forward_batched(tt_context *ctx, const tt_image *images,
             TT_HIP(B.spec.ensure(sizeof(float) * spec_tot));
         std::vector<ttk::DftJob> jobs;
         int dft_tiles = 0;
-        size_t off = 0, cko = 0, so = 0;
+        size_t bbo = 0, cko = 0, so = 0;
         int cols = 0;
         bool p2 = false;
         for (int q = 0; q < np; q++)
@@ -1303,12 +1375,10 @@ TT_API tt_status tt_forward_batched(tt_context *ctx, const tt_image *images,
                 jobs.push_back(j);
             }
             b.img = im.d_image;
-            b.bbox = B.bbox.as<int>() + ttk::kBboxInts * k;
+            b.bbox = B.bbox.as<int>() + bbo;
+            bbo += ttk::bbox_ints(im.n);
             b.ckpt = B.ckpt.as<float2>() + cko;
             cko += (size_t)ttk::sino_ckpt_blocks(im.n) * im.n * n_angles;
-            b.pair = B.pairs.as<float2>() + off;
-            b.pairT = b.pair + ttk::image_pair_count(im.n);
-            off += 2 * ttk::image_pair_count(im.n);
             b.sino = im.d_sino;
             // with d_saved the medians and T3..T5 integrals a backward needs
             b.med_x = sv && need_x ? (int32_t *)(sv + SL.med_x) : nullptr;
@@ -1355,8 +1425,9 @@ TT_API tt_status tt_forward_batched(tt_context *ctx, const tt_image *images,
         for (int k = 0; k < 8; k++)
             sp.slot.s[k] = slot[k];
         // descriptors with the line items of tile t
+        TT_HIP(reserve_pairs(B, d));  // last: it takes what there is room for
         auto use_tile = [&](LineTile t) {
-            sp.items = layout_line_items(d, n_angles, t);
+            layout_line_items(d, B.groups, n_angles, t);
             sp.tile_a = t.a;
             sp.tile_c = t.c;
             return hipMemcpy(B.desc.ptr, d.data(), sizeof(ttk::BatchImage) * nimg,
@@ -1382,7 +1453,10 @@ TT_API tt_status tt_forward_batched(tt_context *ctx, const tt_image *images,
         const int cus = device_cus(ctx->device);
         int best_w = 4, best_b = cus * 4;
         if (ctx->autotune) {
-            TT_HIP(ttk::launch_image_pairs_batched(sp.images, nimg, nmax, sp.counter, own));
+            // (groups that share the workspace form their pairs in each trial)
+            const bool shared = B.groups.size() > 1;
+            if (!shared)
+                TT_HIP(ttk::launch_image_pairs_batched(sp.images, nimg, nmax, sp.counter, own));
             hipEvent_t e0, e1;
             TT_HIP(hipEventCreate(&e0));
             TT_HIP(hipEventCreate(&e1));
@@ -1393,8 +1467,8 @@ TT_API tt_status tt_forward_batched(tt_context *ctx, const tt_image *images,
                 for (int rep = 0; rep < 3; rep++) {
                     hipError_t r = hipEventRecord(e0, own);
                     if (r == hipSuccess)
-                        r = enqueue_batch(ctx, sp, cp, nimg, nmax, need_x, need_s, do345, w,
-                                          blocks, false, false, own);
+                        r = enqueue_batch(ctx, sp, cp, nmax, need_x, need_s, do345, w, blocks,
+                                          shared, false, own);
                     if (r == hipSuccess)
                         r = hipEventRecord(e1, own);
                     if (r == hipSuccess)
@@ -1446,15 +1520,14 @@ TT_API tt_status tt_forward_batched(tt_context *ctx, const tt_image *images,
         B.tile_c = best_t.c;
         B.sp = sp;
         B.cp = cp;
-        B.nimg = nimg;
         B.nmax = nmax;
         B.need_x = need_x;
         B.need_s = need_s;
         B.do345 = do345;
 
         TT_HIP(hipStreamBeginCapture(own, hipStreamCaptureModeThreadLocal));
-        hipError_t ce = enqueue_batch(ctx, sp, cp, nimg, nmax, need_x, need_s, do345,
-                                      best_w, best_b, true, true, own);
+        hipError_t ce = enqueue_batch(ctx, sp, cp, nmax, need_x, need_s, do345, best_w, best_b,
+                                      true, true, own);
         hipGraph_t g = nullptr;
         hipError_t ee = hipStreamEndCapture(own, &g);
         TT_HIP(ce);
@@ -1472,7 +1545,7 @@ TT_API tt_status tt_forward_batched(tt_context *ctx, const tt_image *images,
     if (ctx->timer.on) {
         // per-stage kernel times: the captured stages launched directly, each
         // bracketed by HIP events
-        TT_HIP(enqueue_batch(ctx, B.sp, B.cp, B.nimg, B.nmax, B.need_x, B.need_s, B.do345,
+        TT_HIP(enqueue_batch(ctx, B.sp, B.cp, B.nmax, B.need_x, B.need_s, B.do345,
                              B.waves_per_block, B.blocks, true, true, own, true));
     } else {
         TT_HIP(hipGraphLaunch(B.exec, own));
@@ -2302,9 +2375,8 @@ TT_API tt_status tt_backward_batched(tt_context *ctx, const tt_image_grad *image
         std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
             return images[a].n > images[b].n;
         });
-        size_t pr = 0, ln = 0, spec_tot = 0;
+        size_t ln = 0, spec_tot = 0;
         for (int i = 0; i < nimg; i++) {
-            pr += 2 * ttk::image_pair_count(images[i].n);
             ln += (size_t)images[i].n * n_angles;
             spec_tot += (size_t)nt * n_angles * 2 * (images[i].n / 2 + 1);
         }
@@ -2313,15 +2385,17 @@ TT_API tt_status tt_backward_batched(tt_context *ctx, const tt_image_grad *image
         const bool p2src = p2 && nmax <= 2048;
         // without saved line data the forward is recomputed into workspaces
         if (!saved) {
-            TT_HIP(B.pairs.ensure(sizeof(float2) * pr));
             TT_HIP(P.sino.ensure(sizeof(float) * nt * ln));
             TT_HIP(P.z.ensure(sizeof(float2) * 3 * ln));
             TT_HIP(P.medx.ensure(sizeof(int32_t) * ln));
             TT_HIP(P.meds.ensure(sizeof(int32_t) * ln));
-            TT_HIP(B.bbox.ensure(ttk::kBboxInts * sizeof(int) * (size_t)nimg));
-            size_t ck = 0;  // the line kernel's walk checkpoints, image after image
-            for (int i = 0; i < nimg; i++)
+            // the box scratch and the line kernel's walk checkpoints, image after image
+            size_t bb = 0, ck = 0;
+            for (int i = 0; i < nimg; i++) {
+                bb += ttk::bbox_ints(images[i].n);
                 ck += (size_t)ttk::sino_ckpt_blocks(images[i].n) * images[i].n * n_angles;
+            }
+            TT_HIP(B.bbox.ensure(sizeof(int) * bb));
             TT_HIP(B.ckpt.ensure(sizeof(float2) * ck));
             if (p3s.np3 > 0)
                 TT_HIP(P.spec.ensure(sizeof(float) * spec_tot));
@@ -2340,7 +2414,7 @@ TT_API tt_status tt_backward_batched(tt_context *ctx, const tt_image_grad *image
         int ftiles = 0, btiles = 0;
         size_t so = 0;
         std::vector<ttk::BatchImage> d(nimg);
-        size_t po = 0, lo = 0, cko = 0, pro = 0;
+        size_t po = 0, lo = 0, cko = 0, bbo = 0;
         int cols = 0;
         for (int k = 0; k < nimg; k++) {
             const tt_image_grad &im = images[order[k]];
@@ -2367,12 +2441,10 @@ TT_API tt_status tt_backward_batched(tt_context *ctx, const tt_image_grad *image
                 b.spec = (float *)(base + L.spec);
                 b.p2src = p2src ? (int32_t *)(base + L.p2src) : nullptr;
             } else {
-                b.bbox = B.bbox.as<int>() + ttk::kBboxInts * k;
+                b.bbox = B.bbox.as<int>() + bbo;
+                bbo += ttk::bbox_ints(im.n);
                 b.ckpt = B.ckpt.as<float2>() + cko;
                 cko += (size_t)ttk::sino_ckpt_blocks(im.n) * im.n * n_angles;
-                b.pair = B.pairs.as<float2>() + pro;
-                b.pairT = b.pair + ttk::image_pair_count(im.n);
-                pro += 2 * ttk::image_pair_count(im.n);
                 b.sino = P.sino.as<float>() + nt * lo;
                 b.med_x = P.medx.as<int32_t>() + lo;
                 b.med_s = P.meds.as<int32_t>() + lo;
@@ -2412,13 +2484,7 @@ TT_API tt_status tt_backward_batched(tt_context *ctx, const tt_image_grad *image
             lo += l;
         }
         TT_CHECK(po < (1ull << 31) && lo < (1ull << 31), "batch too large");
-        // the recompute's line tile (forced or the default); gather tiles
-        const LineTile lt = line_tile_of(ctx);
-        const int items = layout_line_items(d, n_angles, lt);
-        int tiles = layout_gather_tiles(d, gtile);
         TT_HIP(B.desc.ensure(sizeof(ttk::BatchImage) * nimg));
-        TT_HIP(hipMemcpy(B.desc.ptr, d.data(), sizeof(ttk::BatchImage) * nimg,
-                         hipMemcpyHostToDevice));
         ttk::DftParams fdp = {}, bdp = {};
         ftiles = layout_dft_jobs(fj, true, &fdp.bm, &fdp.bn);
         btiles = layout_dft_jobs(bj, false, &bdp.bm, &bdp.bn);
@@ -2451,11 +2517,19 @@ TT_API tt_status tt_backward_batched(tt_context *ctx, const tt_image_grad *image
         TT_HIP(hipMemcpy(B.tab.ptr, h.data(), sizeof(float2) * h.size(),
                          hipMemcpyHostToDevice));
         TT_HIP(B.counter.ensure(sizeof(unsigned int)));
+        // the recompute's line tile (forced or the default); gather tiles
+        B.groups.clear();
+        if (!saved)
+            TT_HIP(reserve_pairs(B, d));  // last: it takes what there is room for
+        const LineTile lt = line_tile_of(ctx);
+        layout_line_items(d, B.groups, n_angles, lt);
+        int tiles = layout_gather_tiles(d, gtile);
+        TT_HIP(hipMemcpy(B.desc.ptr, d.data(), sizeof(ttk::BatchImage) * nimg,
+                         hipMemcpyHostToDevice));
 
         ttk::BatchSinoParams sp = {};
         sp.images = B.desc.as<ttk::BatchImage>();
         sp.nimg = nimg;
-        sp.items = items;
         sp.tile_a = lt.a;
         sp.tile_c = lt.c;
         sp.trig = B.trig.as<float2>();
@@ -2497,7 +2571,6 @@ TT_API tt_status tt_backward_batched(tt_context *ctx, const tt_image_grad *image
         B.blocks = cus * 4;
         B.sp = sp;
         B.cp = cp;
-        B.nimg = nimg;
         B.nmax = nmax;
         B.do345 = do345;
         P.ap = ap;
@@ -2684,6 +2757,12 @@ TT_API tt_status tt_circus_noalloc(tt_context *ctx, const float *d_sino, int n,
 TT_API tt_status tt_testing_fail_allocations(long long allowed)
 {
     g_alloc_budget.store(allowed < 0 ? -1 : allowed);
+    return TT_OK;
+}
+
+TT_API tt_status tt_testing_limit_allocation(size_t bytes)
+{
+    g_alloc_limit.store(bytes);
     return TT_OK;
 }
 

@@ -370,17 +370,24 @@ hipError_t launch_circus_vjp(const CircusVjpParams &p, hipStream_t s);
 // bbox is 1 when some pixel is neither 0 nor in [2^-45, 2^120] (then a
 // bilinear sample can be negative, a positive value below 2^-96, infinite or
 // NaN, and the kernels take the library's square root), else 0.  bbox
-// holds kBboxInts words: the result, then scratch for the blocks' boxes.
+// holds bbox_ints(n) words: the result, then scratch for the blocks' boxes.
 constexpr int kPairBlocks = 1024;  // at most, per image
-constexpr int kBboxInts = 8 * (1 + kPairBlocks);
+// Blocks of one image's pair pass: one 32 x 32 tile each up to kPairBlocks
+// (1449 rows: 17.9 us with 512 blocks of four tiles, 14.2 us with 1024).
+__host__ __device__ constexpr int pair_blocks(int n)
+{
+    const int tiles = (n + 31) / 32;
+    return tiles * tiles < kPairBlocks ? tiles * tiles : kPairBlocks;
+}
+__host__ __device__ constexpr size_t bbox_ints(int n) { return 8 * (1 + (size_t)pair_blocks(n)); }
 __host__ __device__ inline size_t image_pair_count(int n)
 {
     return (size_t)n * n + 2;  // a sample at the last pixel loads one pair more
 }
 hipError_t launch_image_pairs(const float *img, int n, float2 *pair, float2 *pairT, int *bbox,
                               hipStream_t s);
-// The same for every image of a batch (into images[k].pair, pairT, bbox);
-// counter: a word the same launches set to zero.
+// The same for nimg images of a batch, of up to nmax rows (into
+// images[k].pair, pairT, bbox); counter: a word the same launches set to zero.
 hipError_t launch_image_pairs_batched(const BatchImage *images, int nimg, int nmax,
                                       unsigned int *counter, hipStream_t s);
 hipError_t launch_pad(const float *in, int rows, int cols, float *out, int n,

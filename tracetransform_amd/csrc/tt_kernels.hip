@@ -956,14 +956,6 @@ __global__ void reset_counters_kernel(unsigned int *c, int count)
         c[threadIdx.x] = 0u;
 }
 
-// Blocks of one image's pair pass: one 32 x 32 tile each up to kPairBlocks
-// (1449 rows: 17.9 us with 512 blocks of four tiles, 14.2 us with 1024).
-__host__ __device__ constexpr int pair_blocks(int n)
-{
-    const int tiles = (n + 31) / 32;
-    return tiles * tiles < kPairBlocks ? tiles * tiles : kPairBlocks;
-}
-
 // The pixel pairs of an n x n column-major image and the box of its non-zero
 // pixels (launch_image_pairs): block `block` of nblocks takes 32 x 32 tiles
 // through LDS (33 x 33, the pairs' second pixels included) and leaves its
