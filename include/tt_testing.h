@@ -21,6 +21,12 @@ TT_API tt_status tt_testing_fail_allocations(long long allowed);
  * as on a device without room for it; 0 removes the limit. */
 TT_API tt_status tt_testing_limit_allocation(size_t bytes);
 
+/* The launch shape of a single image's transposed rotation (n x n pixels) on a
+ * device of `cus` CUs, for the gradients of nt T-functionals: waves per
+ * workgroup and angle groups.  Needs no device. */
+TT_API tt_status tt_testing_gather_launch(int n, int n_angles, int cus, const int32_t *tcodes,
+                                          int nt, int *waves, int *groups);
+
 /* Compares the sort kernel's short square root (v_sqrt_f32 and one residual
  * test per neighbour) with the correctly rounded sqrtf on the GPU for the
  * float bit patterns [lo, lo + count), skipping its documented exceptions

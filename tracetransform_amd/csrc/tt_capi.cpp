@@ -1744,39 +1744,41 @@ tt_status forward_for_adjoint(tt_context *ctx, const float *d_image, int n, int 
 // Launch shape of the transposed-rotation gather: tiles of class 32, the
 // most waves per workgroup (16 to 1) whose LDS (the T3..T5 tables once
 // plus each wave's accumulators and staged columns) fits the 160 KiB of a
-// CU, and for a single image enough angle groups that tiles x groups waves
-// fill every SIMD four times over.
+// CU, and for a single image the angle groups that fill the device.
 struct GatherLaunch {
     int tile, waves, groups;
 };
 
-GatherLaunch choose_gather(int tiles32, int A, int cus, int tabn, bool do345, bool do12,
-                           bool do67, bool split_angles)
+GatherLaunch choose_gather(int n, int A, int cus, bool do345, bool do12, bool do67)
 {
+    const int tiles32 = ttk::gather_tiles(n, 32);
     GatherLaunch g = {32, 1, 1};
     for (int waves = 16; waves >= 1; waves--) {
-        if (ttk::gather_lds_bytes(32, waves, tabn, do345, do12, do67) <= kLdsLimit) {
+        if (ttk::gather_lds_bytes(32, waves, n, do345, do12, do67) <= kLdsLimit) {
             g.waves = waves;
             break;
         }
     }
-    if (split_angles) {
-        // Angle groups: the waves (tiles x groups) run in rounds of what the
-        // device holds at once (16 waves per CU: the LDS and 128 VGPRs), each
-        // wave over ceil(A / groups) angles; the group count minimises
-        // rounds x angles per wave, plus a little for each partial image the
-        // reduction reads (a count just above one round's worth would run a
-        // second round for a few waves).
-        const double cap = 16.0 * cus;
-        double best = 1e30;
-        const int gmax = A < 32 ? A : 32;
-        for (int groups = 1; groups <= gmax; groups++) {
-            const double rounds = ceil((double)tiles32 * groups / cap);
-            const double cost = rounds * ceil((double)A / groups) + groups / 8.0;
-            if (cost < best) {
-                best = cost;
-                g.groups = groups;
-            }
+    // Angle groups: the waves (tiles x groups) run in rounds of what the
+    // device holds at once (the workgroups that fit a CU's LDS and, with
+    // 128 VGPRs, its 16 waves), each wave over ceil(A / groups) angles;
+    // the group count minimises rounds x angles per wave, plus the partial
+    // images that the reduction reads (8 us each at 1800 rows, as long as
+    // one angle of a wave).  T0..T7, 15 waves a CU: 725 rows, 360 angles
+    // 781 us with 7 groups, which are 185 waves more than a round, 500
+    // with 20, three full rounds.
+    const size_t lds = ttk::gather_lds_bytes(32, g.waves, n, do345, do12, do67);
+    const int per_cu = std::max(1, std::min((int)(kLdsLimit / lds), 16 / g.waves));
+    const double cap = (double)g.waves * per_cu * cus;
+    const double part = (double)n * n / 4.2e6;
+    double best = 1e30;
+    const int gmax = A < 32 ? A : 32;
+    for (int groups = 1; groups <= gmax; groups++) {
+        const double rounds = ceil((double)tiles32 * groups / cap);
+        const double cost = rounds * ceil((double)A / groups) + groups * part;
+        if (cost < best) {
+            best = cost;
+            g.groups = groups;
         }
     }
     return g;
@@ -1815,8 +1817,8 @@ tt_status image_vjp(tt_context *ctx, int n, int A, const int *slot,
     g.A = A;
     g.do345 = slot[3] >= 0 || slot[4] >= 0 || slot[5] >= 0;
     g.do12 = slot[1] >= 0 || slot[2] >= 0;
-    const GatherLaunch gl = choose_gather(ttk::gather_tiles(n, 32), A, device_cus(ctx->device), n,
-                                          g.do345, g.do12, do67, true);
+    const GatherLaunch gl =
+        choose_gather(n, A, device_cus(ctx->device), g.do345, g.do12, do67);
     g.tile = gl.tile;
     g.waves = gl.waves;
     g.groups = gl.groups;
@@ -2763,6 +2765,21 @@ TT_API tt_status tt_testing_fail_allocations(long long allowed)
 TT_API tt_status tt_testing_limit_allocation(size_t bytes)
 {
     g_alloc_limit.store(bytes);
+    return TT_OK;
+}
+
+TT_API tt_status tt_testing_gather_launch(int n, int n_angles, int cus, const int32_t *tcodes,
+                                          int nt, int *waves, int *groups)
+{
+    TT_CHECK(n >= 3 && n <= 1800 && n_angles >= 1 && cus >= 1 && waves && groups,
+             "invalid sizes");
+    int slot[8];
+    TT_TRY(adjoint_slots(tcodes, nt, slot, true));
+    const GatherLaunch g = choose_gather(
+        n, n_angles, cus, slot[3] >= 0 || slot[4] >= 0 || slot[5] >= 0,
+        slot[1] >= 0 || slot[2] >= 0, slot[6] >= 0 || slot[7] >= 0);
+    *waves = g.waves;
+    *groups = g.groups;
     return TT_OK;
 }
 

@@ -199,7 +199,7 @@ struct GatherParams {
     int do12;                   // T1 or T2 requested
     int tile;                   // tile class, 16 or 32
     int groups;                 // angle groups
-    int waves;                  // waves per workgroup (1..8)
+    int waves;                  // waves per workgroup (1..16)
 };
 // Dynamic LDS bytes of one gather workgroup.
 size_t gather_lds_bytes(int tile, int waves, int tabn, bool do345, bool do12, bool do67);
