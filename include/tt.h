@@ -77,8 +77,9 @@ typedef struct tt_context tt_context;
  * in both directions: 16 n^2 bytes, 34 MB at n = 1449, and the line kernel's
  * median-walk checkpoints: 8 * ceil((n - 1) / 64) * A * n bytes, ~100 MB at
  * n = 1449 and 360 angles) and the cached graph of the batched path.  A batch
- * keeps the pairs of up to 8 GiB of its images at once, of fewer where the
- * device has no room, the checkpoints of all.  No reference counterpart: the
+ * keeps up to 8 GiB of its images' pairs at once (of large batches at few
+ * angles their row-major copies, 4 n^2 bytes), fewer where the device has no
+ * room, and the checkpoints of all.  No reference counterpart: the
  * reference keeps no state between getSinograms calls. */
 TT_API tt_status tt_context_create(int device, tt_context **out);
 TT_API tt_status tt_context_destroy(tt_context *ctx);

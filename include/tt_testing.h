@@ -21,6 +21,11 @@ TT_API tt_status tt_testing_fail_allocations(long long allowed);
  * as on a device without room for it; 0 removes the limit. */
 TT_API tt_status tt_testing_limit_allocation(size_t bytes);
 
+/* Makes the batched line kernels of the plans that follow sample from the
+ * images and their row-major copies (0) or from the pixel pairs (1), whatever
+ * the sizes; negative: the rule's choice. */
+TT_API tt_status tt_testing_line_pairs(int pairs);
+
 /* The launch shape of a single image's transposed rotation (n x n pixels) on a
  * device of `cus` CUs, for the gradients of nt T-functionals: waves per
  * workgroup and angle groups.  Needs no device. */

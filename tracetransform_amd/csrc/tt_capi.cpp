@@ -63,6 +63,9 @@ std::atomic<long long> g_alloc_budget{-1};
 // The largest workspace allocation that may succeed
 // (tt_testing_limit_allocation), or 0 (no limit).
 std::atomic<size_t> g_alloc_limit{0};
+// What the batched line kernels sample from (tt_testing_line_pairs): -1 the
+// rule's choice, 0 the images, 1 pixel pairs.
+std::atomic<int> g_line_pairs{-1};
 
 hipError_t workspace_malloc(void **ptr, size_t bytes)
 {
@@ -1021,8 +1024,41 @@ void layout_line_items(std::vector<ttk::BatchImage> &d,
     }
 }
 
-// Bytes of an image's pixel pairs in both directions.
-size_t pair_bytes(int n) { return 2 * sizeof(float2) * ttk::image_pair_count(n); }
+// Whether a batch's line kernels sample from pixel pairs (one load a sample;
+// 16 bytes a pixel to write, 8 to read an angle) or from the images and their
+// row-major copies (two loads; 4 and 4 bytes).  Pairs, unless the bytes decide:
+// the batch's pairs are beyond the 256 MB cache (8 Mi pixels, 128 MB, has both
+// alike), and neighbouring angles lie too far apart to share the L2: a line's
+// end moves by pi n / A pixels from angle to angle, and up to A = n / 10 (half
+// of the 64 columns a wave takes) the images are the faster.  T0 alone, with
+// little to hide the loads behind, up to 80 angles.  ms with pairs and with
+// images, T0..T5 (T0 alone):
+//   400 x 1449 rows,   8 angles   12.9   8.8    (9.9   6.3)
+//    64 x 1449 rows,  72 angles    9.5   8.4    (6.1   5.2)
+//    64 x 1449 rows, 180 angles   19.8  19.5   (11.9  12.0)
+//   100 x  725 rows,  36 angles    2.4   2.1    (1.5   1.3)
+//   100 x  725 rows, 180 angles    8.2   8.7    (3.8   5.1)
+bool line_pairs(const std::vector<ttk::BatchImage> &d, int A, bool need_x, bool need_s)
+{
+    const int forced = g_line_pairs.load();
+    if (forced >= 0)
+        return forced != 0;
+    double px = 0.0, side = 0.0;  // pixels, and their mean image side
+    for (const ttk::BatchImage &b : d) {
+        px += (double)b.n * b.n;
+        side += (double)b.n * b.n * b.n;
+    }
+    side /= px;
+    if (px < 8.0 * (1 << 20))
+        return true;
+    return A >= (need_x || need_s ? side / 10.0 : std::max(80.0, side / 10.0));
+}
+
+// Bytes of an image's pixel pairs in both directions, or of its row-major copy.
+size_t copy_bytes(int n, bool pairs)
+{
+    return pairs ? 2 * sizeof(float2) * ttk::image_pair_count(n) : sizeof(float) * (size_t)n * n;
+}
 
 // Pixel pairs of a batch in the workspace at once, 3 % of the device's memory.
 // A group's line kernel ends in a nearly empty round: 520 images of 1449 rows
@@ -1035,7 +1071,7 @@ constexpr size_t kPairCap = (size_t)8 << 30;
 // one image each.  Where the device has no room for it, smaller groups: pairs
 // are four times their images' bytes, and a batch that fits without them must
 // not fail for them.
-hipError_t reserve_pairs(BatchPlan &B, std::vector<ttk::BatchImage> &d)
+hipError_t reserve_pairs(BatchPlan &B, std::vector<ttk::BatchImage> &d, bool pairs)
 {
     size_t most = 0;
     for (size_t cap = kPairCap;; cap = most / 2) {
@@ -1043,7 +1079,7 @@ hipError_t reserve_pairs(BatchPlan &B, std::vector<ttk::BatchImage> &d)
         size_t used = 0;
         most = 0;
         for (int k = 0; k < (int)d.size(); k++) {
-            const size_t bytes = pair_bytes(d[k].n);
+            const size_t bytes = copy_bytes(d[k].n, pairs);
             if (B.groups.empty() || used + bytes > cap) {
                 B.groups.push_back({k, 0, 0, d[k].n});
                 used = 0;
@@ -1055,16 +1091,19 @@ hipError_t reserve_pairs(BatchPlan &B, std::vector<ttk::BatchImage> &d)
         const hipError_t e = B.pairs.ensure(most);
         if (e == hipSuccess)
             break;
-        if (e != hipErrorOutOfMemory || most <= pair_bytes(d[0].n))
+        if (e != hipErrorOutOfMemory || most <= copy_bytes(d[0].n, pairs))
             return e;
     }
     for (const BatchPlan::LineGroup &g : B.groups) {
-        float2 *at = B.pairs.as<float2>();
+        unsigned char *at = B.pairs.as<unsigned char>();
         for (int k = g.first; k < g.first + g.count; k++) {
-            const size_t cnt = ttk::image_pair_count(d[k].n);
-            d[k].pair = at;
-            d[k].pairT = at + cnt;
-            at += 2 * cnt;
+            if (pairs) {
+                d[k].pair = reinterpret_cast<float2 *>(at);
+                d[k].pairT = d[k].pair + ttk::image_pair_count(d[k].n);
+            } else {
+                d[k].imgT = reinterpret_cast<float *>(at);
+            }
+            at += copy_bytes(d[k].n, pairs);
         }
     }
     return hipSuccess;
@@ -1132,7 +1171,8 @@ void enqueue_lines(Stages &stage, const std::vector<BatchPlan::LineGroup> &group
         q.items = g.items;
         if (with_pairs)
             stage(TT_KERNEL_AUX, [&] {
-                return ttk::launch_image_pairs_batched(q.images, q.nimg, g.nmax, q.counter, st);
+                return ttk::launch_image_pairs_batched(q.images, q.nimg, g.nmax, q.pairs, q.counter,
+                                                       st);
             });
         stage(TT_KERNEL_SINO_T05, [&] {
             // (the pair pass has zeroed the work counter)
@@ -1290,7 +1330,7 @@ TT_API tt_status tt_forward_batched(tt_context *ctx, const tt_image *images,
     TT_TRY(ctx->set_device());
 
     std::vector<int64_t> key = {nimg, n_angles, (int64_t)(*(const uint32_t *)&angle_step_deg),
-                                nt, np, ctx->autotune};
+                                nt, np, ctx->autotune, g_line_pairs.load()};
     for (int t = 0; t < nt; t++)
         key.push_back(tcodes[t]);
     for (int q = 0; q < np; q++)
@@ -1425,7 +1465,8 @@ TT_API tt_status tt_forward_batched(tt_context *ctx, const tt_image *images,
         for (int k = 0; k < 8; k++)
             sp.slot.s[k] = slot[k];
         // descriptors with the line items of tile t
-        TT_HIP(reserve_pairs(B, d));  // last: it takes what there is room for
+        sp.pairs = line_pairs(d, n_angles, need_x, need_s);
+        TT_HIP(reserve_pairs(B, d, sp.pairs));  // last: it takes what there is room for
         auto use_tile = [&](LineTile t) {
             layout_line_items(d, B.groups, n_angles, t);
             sp.tile_a = t.a;
@@ -1456,7 +1497,8 @@ TT_API tt_status tt_forward_batched(tt_context *ctx, const tt_image *images,
             // (groups that share the workspace form their pairs in each trial)
             const bool shared = B.groups.size() > 1;
             if (!shared)
-                TT_HIP(ttk::launch_image_pairs_batched(sp.images, nimg, nmax, sp.counter, own));
+                TT_HIP(ttk::launch_image_pairs_batched(sp.images, nimg, nmax, sp.pairs, sp.counter,
+                                                       own));
             hipEvent_t e0, e1;
             TT_HIP(hipEventCreate(&e0));
             TT_HIP(hipEventCreate(&e1));
@@ -2349,7 +2391,7 @@ TT_API tt_status tt_backward_batched(tt_context *ctx, const tt_image_grad *image
     }
     TT_TRY(ctx->set_device());
     std::vector<int64_t> key = {nimg, n_angles, (int64_t)(*(const uint32_t *)&angle_step_deg),
-                                nt, np, saved, ctx->autotune};
+                                nt, np, saved, ctx->autotune, g_line_pairs.load()};
     for (int t = 0; t < nt; t++)
         key.push_back(tcodes[t]);
     for (int q = 0; q < np; q++)
@@ -2521,8 +2563,9 @@ TT_API tt_status tt_backward_batched(tt_context *ctx, const tt_image_grad *image
         TT_HIP(B.counter.ensure(sizeof(unsigned int)));
         // the recompute's line tile (forced or the default); gather tiles
         B.groups.clear();
+        const bool pairs = line_pairs(d, n_angles, true, true);
         if (!saved)
-            TT_HIP(reserve_pairs(B, d));  // last: it takes what there is room for
+            TT_HIP(reserve_pairs(B, d, pairs));  // last: it takes what there is room for
         const LineTile lt = line_tile_of(ctx);
         layout_line_items(d, B.groups, n_angles, lt);
         int tiles = layout_gather_tiles(d, gtile);
@@ -2532,6 +2575,7 @@ TT_API tt_status tt_backward_batched(tt_context *ctx, const tt_image_grad *image
         ttk::BatchSinoParams sp = {};
         sp.images = B.desc.as<ttk::BatchImage>();
         sp.nimg = nimg;
+        sp.pairs = pairs;
         sp.tile_a = lt.a;
         sp.tile_c = lt.c;
         sp.trig = B.trig.as<float2>();
@@ -2765,6 +2809,12 @@ TT_API tt_status tt_testing_fail_allocations(long long allowed)
 TT_API tt_status tt_testing_limit_allocation(size_t bytes)
 {
     g_alloc_limit.store(bytes);
+    return TT_OK;
+}
+
+TT_API tt_status tt_testing_line_pairs(int pairs)
+{
+    g_line_pairs.store(pairs < 0 ? -1 : pairs != 0);
     return TT_OK;
 }
 

@@ -62,6 +62,7 @@ struct BatchImage {
     const float *img;     // n x n column-major
     float2 *pair;         // pixel pairs along the columns (see launch_image_pairs)
     float2 *pairT;        // pixel pairs along the rows
+    float *imgT;          // row-major copy (batches without pairs)
     float *sino;          // [nt][A][n]
     int32_t *med_x;
     int32_t *med_s;
@@ -91,6 +92,7 @@ struct BatchSinoParams {
     int items;            // total wave items
     int tile_a;           // angles of one wave item (a multiple of 64 / tile_c)
     int tile_c;           // columns of one wave item: 64, 32 or 16
+    int pairs;            // samples from the pixel pairs, else from img and imgT
     const float2 *trig;   // [A]
     const float2 *tab345; // [3][tabn]
     int tabn;             // largest n of the batch
@@ -387,8 +389,9 @@ __host__ __device__ inline size_t image_pair_count(int n)
 hipError_t launch_image_pairs(const float *img, int n, float2 *pair, float2 *pairT, int *bbox,
                               hipStream_t s);
 // The same for nimg images of a batch, of up to nmax rows (into
-// images[k].pair, pairT, bbox); counter: a word the same launches set to zero.
-hipError_t launch_image_pairs_batched(const BatchImage *images, int nimg, int nmax,
+// images[k].pair, pairT, bbox), or without pairs the row-major copies (into
+// images[k].imgT, bbox); counter: a word the same launches set to zero.
+hipError_t launch_image_pairs_batched(const BatchImage *images, int nimg, int nmax, bool pairs,
                                       unsigned int *counter, hipStream_t s);
 hipError_t launch_pad(const float *in, int rows, int cols, float *out, int n,
                       int dfx, int dfy, hipStream_t s);

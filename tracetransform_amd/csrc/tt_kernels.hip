@@ -17,28 +17,30 @@ namespace ttk {
 namespace {
 
 // 16-byte load from an 8-byte aligned address (legal for global memory on
-// CDNA): two neighbouring pixel pairs.
+// CDNA): two neighbouring pixel pairs; 8-byte load from a 4-byte aligned one:
+// two neighbouring pixels.
 typedef float f4p __attribute__((ext_vector_type(4), aligned(8)));
+typedef float f2p __attribute__((ext_vector_type(2), aligned(4)));
 
 // A pointer every lane of the wave holds, made visibly wave-uniform (its
 // two halves read from the first lane), so that loads from it can take the
 // scalar-base form.
-__device__ __forceinline__ const float2 *uniform_ptr(const float2 *p)
+__device__ __forceinline__ const float *uniform_ptr(const float *p)
 {
     const uint64_t v = reinterpret_cast<uint64_t>(p);
     const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
     const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-    return reinterpret_cast<const float2 *>(((uint64_t)hi << 32) | lo);
+    return reinterpret_cast<const float *>(((uint64_t)hi << 32) | lo);
 }
 
 // Load at a 32-bit byte offset from a wave-uniform base in global memory:
 // the scalar-base + vector-offset form of global loads (no 64-bit VALU
 // math, no flat addressing).
-__device__ __forceinline__ f4p ld4b(const float2 *base, uint32_t byte_off)
+template <class V> __device__ __forceinline__ V ldb(const float *base, uint32_t byte_off)
 {
     typedef const char __attribute__((address_space(1))) *gbyte;
-    typedef const f4p __attribute__((address_space(1))) *gf4;
-    return *(gf4)((gbyte)base + byte_off);
+    typedef const V __attribute__((address_space(1))) *gv;
+    return *(gv)((gbyte)base + byte_off);
 }
 
 __device__ __forceinline__ int wave_id()
@@ -62,8 +64,10 @@ __device__ __forceinline__ int xcd_block()
 // pxc = px*c and pxns = px*(-s) precomputed per lane (each is one rounded
 // product, as in the reference).  Strict bounds 0 <= x,y < n-1; the four
 // taps are evaluated left to right with the reference's association.
-// src is the pixel-pair copy of the image that the lanes step along: TR (along
-// x) pairs of rows, else pairs of columns; the four taps are one 16-byte load.
+// PAIRS: src is the pixel-pair copy of the image that the lanes step along: TR
+// (along x) pairs of rows, else pairs of columns; the four taps are one 16-byte
+// load.  Else src is the image's row-major copy (TR) or the image itself, and
+// the taps are two 8-byte loads.  The taps, hence the results, are the same.
 // The L1 looks up one line per four lanes of a load whatever the load's width,
 // about 25 cycles per load and CU, and two 8-byte loads a sample (one per
 // image row) made that the line kernel's bound: 0.87 ms against 0.59 for the
@@ -80,8 +84,8 @@ struct Tap {
 
 // CHK: test the position against the image's bounds (without it the caller
 // knows that the position is inside).
-template <bool TR, bool CHK>
-__device__ __forceinline__ Tap rot_load(const float2 *__restrict__ src, int n, float lim,
+template <bool TR, bool PAIRS, bool CHK>
+__device__ __forceinline__ Tap rot_load(const float *__restrict__ src, int n, float lim,
                                         float o, float pxc, float pxns, float c, float s,
                                         float py)
 {
@@ -109,7 +113,13 @@ __device__ __forceinline__ Tap rot_load(const float2 *__restrict__ src, int n, f
     }
     const uint32_t un = (uint32_t)n;
     // X, Y < n <= 2730, so X * n fits the 24-bit multiplier
-    t.q = ld4b(src, (TR ? __umul24(Y, un) + X : __umul24(X, un) + Y) * 8u);
+    const uint32_t at = TR ? __umul24(Y, un) + X : __umul24(X, un) + Y;
+    if constexpr (PAIRS) {
+        t.q = ldb<f4p>(src, at * 8u);
+    } else {
+        const f2p a = ldb<f2p>(src, at * 4u), b = ldb<f2p>(src, (at + un) * 4u);
+        t.q = f4p{a.x, b.x, a.y, b.y};
+    }
     return t;
 }
 
@@ -124,12 +134,12 @@ __device__ __forceinline__ float rot_value(const Tap &t)
     return !CHK || t.in ? v : 0.0f;
 }
 
-template <bool TR>
-__device__ __forceinline__ float rot_sample(const float2 *__restrict__ src, int n, float lim,
+template <bool TR, bool PAIRS>
+__device__ __forceinline__ float rot_sample(const float *__restrict__ src, int n, float lim,
                                             float o, float pxc, float pxns, float c, float s,
                                             float py)
 {
-    return rot_value<TR, true>(rot_load<TR, true>(src, n, lim, o, pxc, pxns, c, s, py));
+    return rot_value<TR, true>(rot_load<TR, PAIRS, true>(src, n, lim, o, pxc, pxns, c, s, py));
 }
 
 // Square root of a line sample, correctly rounded.  FS: v_sqrt_f32 and one
@@ -410,8 +420,8 @@ struct LineDst {
 // at 180 angles, one wave per three SIMDs, 58 -> TIME us; bound by VALU issue
 // (about 24 half-rate slots a row in pass 1, of which the bilinear sample is
 // 14; adds and multiplies issue twice as fast as the rest on this chip).
-template <bool TR, bool NEED_X, bool NEED_S, bool DO345, bool CK, bool FS>
-__device__ __forceinline__ void sino_line(const LineDst &p, const float2 *src,
+template <bool TR, bool PAIRS, bool NEED_X, bool NEED_S, bool DO345, bool CK, bool FS>
+__device__ __forceinline__ void sino_line(const LineDst &p, const float *src,
                                           const float2 *s_tab, int a, int col,
                                           bool active, float c, float s, int lo, int hi)
 {
@@ -444,7 +454,7 @@ __device__ __forceinline__ void sino_line(const LineDst &p, const float2 *src,
     const int vb2 = (wave_min_u((ins.y + 1 < n ? ins.y + 1 : n) + dl)) & ~7;    // pass 2
 
     auto load = [&](auto chk, float py) {
-        return rot_load<TR, decltype(chk)::value>(src, n, lim, o, pxc, pxns, c, s, py);
+        return rot_load<TR, PAIRS, decltype(chk)::value>(src, n, lim, o, pxc, pxns, c, s, py);
     };
     struct Half {
         Tap t[4];
@@ -551,7 +561,7 @@ __device__ __forceinline__ void sino_line(const LineDst &p, const float2 *src,
         Sx = 0.0f;
         Ss = 0.0f;
         for (int r = 0; r < n; r++) {
-            const float v = rot_sample<TR>(src, n, lim, o, pxc, pxns, c, s,
+            const float v = rot_sample<TR, PAIRS>(src, n, lim, o, pxc, pxns, c, s,
                                            (float)r - o);
             Sx = r == 0 ? v : Sx + v;
             if (NEED_S)
@@ -567,7 +577,7 @@ __device__ __forceinline__ void sino_line(const LineDst &p, const float2 *src,
         if (a4 > a8 && tail) {
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                const float v = rot_sample<TR>(src, n, lim, o, pxc, pxns, c, s,
+                const float v = rot_sample<TR, PAIRS>(src, n, lim, o, pxc, pxns, c, s,
                                                (float)(a8 + j) - o);
                 const float sv = NEED_S ? line_root<FS>(v) : 0.0f;
                 if (n >= 8) {
@@ -582,7 +592,7 @@ __device__ __forceinline__ void sino_line(const LineDst &p, const float2 *src,
         Sx = (ax[0] + ax[2]) + (ax[1] + ax[3]);
         Ss = (as[0] + as[2]) + (as[1] + as[3]);
         for (int r = a4; tail && r < n; r++) {
-            const float v = rot_sample<TR>(src, n, lim, o, pxc, pxns, c, s,
+            const float v = rot_sample<TR, PAIRS>(src, n, lim, o, pxc, pxns, c, s,
                                            (float)r - o);
             Sx += v;
             if (NEED_S)
@@ -814,9 +824,9 @@ __device__ __forceinline__ void sino_line(const LineDst &p, const float2 *src,
 
 // One line, with the image copy whose fast axis the lanes step along (TR)
 // and the square root the image's bounding-box flag allows (FS).
-template <bool NEED_X, bool NEED_S, bool DO345, bool CK>
-__device__ __forceinline__ void sino_line_any(const LineDst &dst, const float2 *pair,
-                                              const float2 *pairT, const int *bbox,
+template <bool PAIRS, bool NEED_X, bool NEED_S, bool DO345, bool CK>
+__device__ __forceinline__ void sino_line_any(const LineDst &dst, const float *src,
+                                              const float *srcT, const int *bbox,
                                               const float2 *s_tab, int a, int col,
                                               bool active, float2 cs, int lo, int hi)
 {
@@ -824,17 +834,17 @@ __device__ __forceinline__ void sino_line_any(const LineDst &dst, const float2 *
     const bool tr = __builtin_amdgcn_readfirstlane(fabsf(cs.x) > fabsf(cs.y));
     const bool fs = bbox && bbox[4] == 0;
     if (tr && fs)
-        sino_line<true, NEED_X, NEED_S, DO345, CK, true>(dst, pairT, s_tab, a, col, active,
-                                                         cs.x, cs.y, lo, hi);
+        sino_line<true, PAIRS, NEED_X, NEED_S, DO345, CK, true>(dst, srcT, s_tab, a, col, active,
+                                                                cs.x, cs.y, lo, hi);
     else if (tr)
-        sino_line<true, NEED_X, NEED_S, DO345, CK, false>(dst, pairT, s_tab, a, col, active,
-                                                          cs.x, cs.y, lo, hi);
+        sino_line<true, PAIRS, NEED_X, NEED_S, DO345, CK, false>(dst, srcT, s_tab, a, col, active,
+                                                                 cs.x, cs.y, lo, hi);
     else if (fs)
-        sino_line<false, NEED_X, NEED_S, DO345, CK, true>(dst, pair, s_tab, a, col, active,
-                                                          cs.x, cs.y, lo, hi);
+        sino_line<false, PAIRS, NEED_X, NEED_S, DO345, CK, true>(dst, src, s_tab, a, col, active,
+                                                                 cs.x, cs.y, lo, hi);
     else
-        sino_line<false, NEED_X, NEED_S, DO345, CK, false>(dst, pair, s_tab, a, col, active,
-                                                           cs.x, cs.y, lo, hi);
+        sino_line<false, PAIRS, NEED_X, NEED_S, DO345, CK, false>(dst, src, s_tab, a, col, active,
+                                                                  cs.x, cs.y, lo, hi);
 }
 
 // LDS copy of the T3..T5 tables ([3][tabn] float2 in global memory) with the
@@ -872,8 +882,9 @@ __global__ __launch_bounds__(kBlock) void sino_t05_kernel(SinoParams p)
     const float2 cs = p.trig[a];
     const LineDst dst = {p.sino, p.med_x, p.med_s, p.z345, p.ckpt, p.n, p.A, p.n, p.slot};
     const int2 rows = line_rows(p.bbox, p.n, col, cs.x, cs.y);
-    sino_line_any<NEED_X, NEED_S, DO345, true>(dst, p.pair, p.pairT, p.bbox, s_tab, a, col,
-                                               active, cs, rows.x, rows.y);
+    sino_line_any<true, NEED_X, NEED_S, DO345, true>(
+        dst, reinterpret_cast<const float *>(p.pair), reinterpret_cast<const float *>(p.pairT),
+        p.bbox, s_tab, a, col, active, cs, rows.x, rows.y);
 }
 
 // ---------------------------------------------------------------------------
@@ -889,8 +900,9 @@ __global__ __launch_bounds__(kBlock) void sino_t05_kernel(SinoParams p)
 // the one that suits the angle of its first lane; the results of a line do
 // not depend on the tile.
 // ---------------------------------------------------------------------------
-template <bool NEED_X, bool NEED_S, bool DO345>
-__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) void sino_t05_batched_kernel(BatchSinoParams p)
+template <bool PAIRS, bool NEED_X, bool NEED_S, bool DO345>
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4)))
+void sino_t05_batched_kernel(BatchSinoParams p)
 {
     extern __shared__ __align__(16) float2 s_tab[];
     if (DO345) {
@@ -939,8 +951,10 @@ __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(4))) voi
         const LineDst dst = {im.sino, im.med_x, im.med_s, im.z345, im.ckpt, im.n, p.A, p.tabn,
                              p.slot};
         const int2 rows = line_rows(im.bbox, im.n, col, cs.x, cs.y);
-        sino_line_any<NEED_X, NEED_S, DO345, true>(dst, im.pair, im.pairT, im.bbox, s_tab, a,
-                                                   col, active, cs, rows.x, rows.y);
+        const float *src = PAIRS ? reinterpret_cast<const float *>(im.pair) : im.img;
+        const float *srcT = PAIRS ? reinterpret_cast<const float *>(im.pairT) : im.imgT;
+        sino_line_any<PAIRS, NEED_X, NEED_S, DO345, true>(dst, src, srcT, im.bbox, s_tab, a, col,
+                                                          active, cs, rows.x, rows.y);
     }
 }
 
@@ -956,14 +970,16 @@ __global__ void reset_counters_kernel(unsigned int *c, int count)
         c[threadIdx.x] = 0u;
 }
 
-// The pixel pairs of an n x n column-major image and the box of its non-zero
-// pixels (launch_image_pairs): block `block` of nblocks takes 32 x 32 tiles
-// through LDS (33 x 33, the pairs' second pixels included) and leaves its
-// box in box[0..4].
+// The pixel pairs (PAIRS) or the row-major copy of an n x n column-major image
+// and the box of its non-zero pixels (launch_image_pairs): block `block` of
+// nblocks takes 32 x 32 tiles through LDS (33 x 33, the pairs' second pixels
+// included) and leaves its box in box[0..4].
+template <bool PAIRS>
 __device__ __forceinline__ void image_pairs_block(const float *img, int n, float2 *pair,
-                                                  float2 *pairT, int block, int nblocks,
-                                                  int *box)
+                                                  float2 *pairT, float *imgT, int block,
+                                                  int nblocks, int *box)
 {
+    constexpr int S = PAIRS ? 33 : 32;  // pixels of a tile each way
     __shared__ float tile[33][35];
     __shared__ int s_b[5][kBlock / kWave];
     const int tiles = (n + 31) / 32;
@@ -972,8 +988,8 @@ __device__ __forceinline__ void image_pairs_block(const float *img, int n, float
     bool narrow = false;  // a pixel that is not 0 or in [2^-45, 2^120]
     for (int t = block; t < tiles * tiles; t += nblocks) {
         const int bx = (t % tiles) * 32, by = (t / tiles) * 32;
-        for (int i = threadIdx.x; i < 33 * 33; i += kBlock) {
-            const int k = i / 33, r = i - 33 * k;
+        for (int i = threadIdx.x; i < S * S; i += kBlock) {
+            const int k = i / S, r = i - S * k;
             const int col = bx + k, row = by + r;
             const bool in = col < n && row < n;
             const float v = in ? img[(size_t)col * n + row] : 0.0f;
@@ -990,15 +1006,20 @@ __device__ __forceinline__ void image_pairs_block(const float *img, int n, float
 #pragma unroll
         for (int k = ty; k < 32; k += 8) {
             const int col = bx + k, row = by + tx;
-            if (col < n && row < n)
-                pair[(size_t)col * n + row] = float2{tile[k][tx], tile[k + 1][tx]};
             const int rowT = by + k, colT = bx + tx;
-            if (colT < n && rowT < n)
-                pairT[(size_t)rowT * n + colT] = float2{tile[tx][k], tile[tx][k + 1]};
+            if constexpr (PAIRS) {
+                if (col < n && row < n)
+                    pair[(size_t)col * n + row] = float2{tile[k][tx], tile[k + 1][tx]};
+                if (colT < n && rowT < n)
+                    pairT[(size_t)rowT * n + colT] = float2{tile[tx][k], tile[tx][k + 1]};
+            } else {
+                if (colT < n && rowT < n)
+                    imgT[(size_t)rowT * n + colT] = tile[tx][k];
+            }
         }
         __syncthreads();
     }
-    if (block == 0 && threadIdx.x < 2) {  // what a sample's second pair may load
+    if (PAIRS && block == 0 && threadIdx.x < 2) {  // what a sample's second pair may load
         pair[(size_t)n * n + threadIdx.x] = float2{0.0f, 0.0f};
         pairT[(size_t)n * n + threadIdx.x] = float2{0.0f, 0.0f};
     }
@@ -1064,7 +1085,8 @@ __global__ __launch_bounds__(kBlock) void image_pairs_kernel(const float *img, i
                                                              float2 *pair, float2 *pairT,
                                                              int *bb)
 {
-    image_pairs_block(img, n, pair, pairT, blockIdx.x, gridDim.x, bb + 8 * (1 + blockIdx.x));
+    image_pairs_block<true>(img, n, pair, pairT, nullptr, blockIdx.x, gridDim.x,
+                            bb + 8 * (1 + blockIdx.x));
 }
 
 __global__ void image_box_kernel(int n, int nblocks, int *bb)
@@ -1076,14 +1098,15 @@ __global__ void image_box_kernel(int n, int nblocks, int *bb)
 // for the largest; an image's surplus blocks end at once and leave no box
 // (with 256 images of 95 to 725 rows two blocks in three had no tile, and
 // each reduced and stored an empty box: 298 -> 248 us).
+template <bool PAIRS>
 __global__ __launch_bounds__(kBlock) void image_pairs_batched_kernel(const BatchImage *images)
 {
     const BatchImage &im = images[blockIdx.y];
     const int blocks = pair_blocks(im.n);
     if ((int)blockIdx.x >= blocks)
         return;
-    image_pairs_block(im.img, im.n, im.pair, im.pairT, blockIdx.x, blocks,
-                      im.bbox + 8 * (1 + blockIdx.x));
+    image_pairs_block<PAIRS>(im.img, im.n, im.pair, im.pairT, im.imgT, blockIdx.x, blocks,
+                             im.bbox + 8 * (1 + blockIdx.x));
 }
 
 __global__ void image_box_batched_kernel(const BatchImage *images, unsigned int *counter)
@@ -2407,7 +2430,7 @@ __device__ __forceinline__ bool sort_line(const SortTParams &p, int line, int wh
     const float px = (float)col - o;
     const float pxc = px * cs.x, pxns = px * (-cs.y);
     const bool tr = fabsf(cs.y) > fabsf(cs.x);
-    const float2 *src = tr ? p.pairT : p.pair;
+    const float *src = reinterpret_cast<const float *>(tr ? p.pairT : p.pair);
     const bool t6 = which == 0;
     const int base = t6 ? p.med_s[line] : p.med_x[line];
     const int L = n - base;
@@ -2427,7 +2450,7 @@ __device__ __forceinline__ bool sort_line(const SortTParams &p, int line, int wh
         constexpr bool TRC = decltype(trc)::value;
         float pyo = (float)(base + lane) - o;  // exact steps of 64 rows
         for (int i = lane; i < Ls; i += kWave, pyo += (float)kWave) {
-            const float x = rot_sample<TRC>(src, n, lim, o, pxc, pxns, cs.x, cs.y, pyo);
+            const float x = rot_sample<TRC, true>(src, n, lim, o, pxc, pxns, cs.x, cs.y, pyo);
             if (i < M)
                 xs[i] = x;
             last_nz = last_set(x != 0.0f, i - lane, last_nz);
@@ -2482,7 +2505,7 @@ __device__ __forceinline__ int sort_pair(const SortTParams &p, int line, float *
     const float px = (float)col - o;
     const float pxc = px * cs.x, pxns = px * (-cs.y);
     const bool tr = fabsf(cs.y) > fabsf(cs.x);
-    const float2 *src = tr ? p.pairT : p.pair;
+    const float *src = reinterpret_cast<const float *>(tr ? p.pairT : p.pair);
     const int sm = p.med_s[line], m = p.med_x[line];
     const bool fs = p.bbox && p.bbox[4] == 0;  // short square roots (line_sqrt)
     const int L6 = n - sm, L7 = n - m;
@@ -2508,7 +2531,7 @@ __device__ __forceinline__ int sort_pair(const SortTParams &p, int line, float *
         constexpr bool TRC = decltype(trc)::value;
         float pyo = (float)(b0 + lane) - o;  // exact steps of 64 rows
         for (int i = lane; i < Lu; i += kWave, pyo += (float)kWave) {
-            const float x = rot_sample<TRC>(src, n, lim, o, pxc, pxns, cs.x, cs.y, pyo);
+            const float x = rot_sample<TRC, true>(src, n, lim, o, pxc, pxns, cs.x, cs.y, pyo);
             xs[i] = x;
             last_nz = last_set(x != 0.0f, i - lane, last_nz);
             last_bad = last_set(!(x >= 0.0f), i - lane, last_bad);  // negative or NaN
@@ -3886,11 +3909,14 @@ hipError_t launch_image_pairs(const float *img, int n, float2 *pair, float2 *pai
     return hipGetLastError();
 }
 
-hipError_t launch_image_pairs_batched(const BatchImage *images, int nimg, int nmax,
+hipError_t launch_image_pairs_batched(const BatchImage *images, int nimg, int nmax, bool pairs,
                                       unsigned int *counter, hipStream_t s)
 {
-    const int blocks = pair_blocks(nmax);
-    image_pairs_batched_kernel<<<dim3(blocks, nimg), kBlock, 0, s>>>(images);
+    const dim3 grid(pair_blocks(nmax), nimg);
+    if (pairs)
+        image_pairs_batched_kernel<true><<<grid, kBlock, 0, s>>>(images);
+    else
+        image_pairs_batched_kernel<false><<<grid, kBlock, 0, s>>>(images);
     image_box_batched_kernel<<<nimg, kWave, 0, s>>>(images, counter);
     return hipGetLastError();
 }
@@ -3909,20 +3935,28 @@ hipError_t launch_sino_t05_batched(const BatchSinoParams &p, bool need_x,
         return hipErrorInvalidValue;
     const int threads = kWave * waves_per_block;
     const size_t shm = do345 ? sizeof(float2) * 3 * (size_t)p.tabn : 0;
-#define TT_LAUNCH(X, S, D)                                                     \
-    sino_t05_batched_kernel<X, S, D><<<blocks, threads, shm, s>>>(p)
-    if (need_x && need_s && do345)
-        TT_LAUNCH(true, true, true);
-    else if (need_x && need_s)
-        TT_LAUNCH(true, true, false);
-    else if (need_x)
-        TT_LAUNCH(true, false, false);
-    else if (need_s && do345)
-        TT_LAUNCH(false, true, true);
-    else if (need_s)
-        TT_LAUNCH(false, true, false);
+#define TT_LAUNCH(P, X, S, D)                                                  \
+    sino_t05_batched_kernel<P, X, S, D><<<blocks, threads, shm, s>>>(p)
+#define TT_LAUNCH_P(P)                                                         \
+    do {                                                                       \
+        if (need_x && need_s && do345)                                         \
+            TT_LAUNCH(P, true, true, true);                                    \
+        else if (need_x && need_s)                                             \
+            TT_LAUNCH(P, true, true, false);                                   \
+        else if (need_x)                                                       \
+            TT_LAUNCH(P, true, false, false);                                  \
+        else if (need_s && do345)                                              \
+            TT_LAUNCH(P, false, true, true);                                   \
+        else if (need_s)                                                       \
+            TT_LAUNCH(P, false, true, false);                                  \
+        else                                                                   \
+            TT_LAUNCH(P, false, false, false);                                 \
+    } while (0)
+    if (p.pairs)
+        TT_LAUNCH_P(true);
     else
-        TT_LAUNCH(false, false, false);
+        TT_LAUNCH_P(false);
+#undef TT_LAUNCH_P
 #undef TT_LAUNCH
     return hipGetLastError();
 }
