@@ -2183,13 +2183,20 @@ __device__ __forceinline__ void p2_wave(const float *x, int n, float *xs, int la
 }
 
 // P1 of the column x[0..n) (n >= 2) by one wave: the sum of
-// |x[i - 1] - x[i]|.  A lane's terms in row order, the loads of eight under
-// way together: one after the other their latency was the time of a few long
-// columns (45 of 2048 rows: 6.2 -> 4.0 us; 4.5 by a workgroup a column).
+// |x[i - 1] - x[i]|, a lane's terms in row order.  Long columns with the loads
+// of eight terms under way together: one after the other their latency was the
+// time of a few such columns (45 of 2048 rows: 6.2 -> 4.0 us; 4.5 by a
+// workgroup a column).  Short ones have no eight terms a lane (270000 columns
+// of 33 rows: 71 us with the eight loads, 62 without).
 __device__ __forceinline__ float p1_wave(const float *x, int n, int lane)
 {
     constexpr int kDeep = 8;
     float acc = 0.0f;
+    if (n <= kDeep * kWave) {
+        for (int i = 1 + lane; i < n; i += kWave)
+            acc += fabsf(x[i - 1] - x[i]);
+        return wave_sum(acc);
+    }
     for (int i = 1 + lane; i < n; i += kDeep * kWave) {
         float a[kDeep], b[kDeep];
 #pragma unroll
