@@ -1043,14 +1043,14 @@ bool line_pairs(const std::vector<ttk::BatchImage> &d, int A, bool need_x, bool 
     const int forced = g_line_pairs.load();
     if (forced >= 0)
         return forced != 0;
-    double px = 0.0, side = 0.0;  // pixels, and their mean image side
+    double px = 0.0, lines = 0.0;  // pixels, lines of one angle
     for (const ttk::BatchImage &b : d) {
         px += (double)b.n * b.n;
-        side += (double)b.n * b.n * b.n;
+        lines += b.n;
     }
-    side /= px;
     if (px < 8.0 * (1 << 20))
         return true;
+    const double side = px / lines;  // a line's mean length
     return A >= (need_x || need_s ? side / 10.0 : std::max(80.0, side / 10.0));
 }
 
