@@ -26,6 +26,10 @@ TT_API tt_status tt_testing_limit_allocation(size_t bytes);
  * the sizes; negative: the rule's choice. */
 TT_API tt_status tt_testing_line_pairs(int pairs);
 
+/* Rows and columns of the tiles that P3's DFT products (forward or adjoint) of
+ * cols columns of n rows take.  Needs no device. */
+TT_API tt_status tt_testing_dft_shape(int n, int cols, int forward, int *rows, int *columns);
+
 /* The launch shape of a single image's transposed rotation (n x n pixels) on a
  * device of `cus` CUs, for the gradients of nt T-functionals: waves per
  * workgroup and angle groups.  Needs no device. */

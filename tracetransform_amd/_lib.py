@@ -32,7 +32,7 @@ EXPORTED = (
     "tt_circus_noalloc", "tt_saved_offsets", "tt_context_set_tiles", "tt_batched_tiles",
     # test hooks (include/tt_testing.h)
     "tt_testing_fail_allocations", "tt_testing_limit_allocation", "tt_testing_gather_launch",
-    "tt_testing_line_pairs",
+    "tt_testing_line_pairs", "tt_testing_dft_shape",
     "tt_testing_short_sqrt", "tt_testing_line_root", "tt_testing_nos_product",
 )
 
@@ -134,6 +134,7 @@ def load():
         L.tt_saved_offsets.argtypes = [C.c_int, C.c_int, C.c_int, szp, szp, szp, szp, szp]
         L.tt_testing_fail_allocations.argtypes = [C.c_longlong]
         L.tt_testing_limit_allocation.argtypes = [C.c_size_t]
+        L.tt_testing_dft_shape.argtypes = [C.c_int] * 3 + [C.POINTER(C.c_int)] * 2
         L.tt_testing_line_pairs.argtypes = [C.c_int]
         L.tt_testing_gather_launch.argtypes = [C.c_int] * 3 + [C.POINTER(C.c_int32), C.c_int,
                                                                C.POINTER(C.c_int),

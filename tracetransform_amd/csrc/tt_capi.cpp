@@ -2818,6 +2818,14 @@ TT_API tt_status tt_testing_line_pairs(int pairs)
     return TT_OK;
 }
 
+TT_API tt_status tt_testing_dft_shape(int n, int cols, int forward, int *rows, int *columns)
+{
+    TT_CHECK(n >= 2 && n <= 2730 && cols >= 1 && rows && columns, "invalid sizes");
+    ttk::dft_tile_shape(ttk::dft_job_tiles(n, cols, forward != 0, 128, 128),
+                        ttk::dft_job_tiles(n, cols, forward != 0, 64, 128), rows, columns);
+    return TT_OK;
+}
+
 TT_API tt_status tt_testing_gather_launch(int n, int n_angles, int cus, const int32_t *tcodes,
                                           int nt, int *waves, int *groups)
 {

@@ -297,8 +297,11 @@ __global__ __launch_bounds__(kBlock) void p3_vjp_scale_kernel(P3ScaleParams p)
 void dft_tile_shape(long long tiles128, long long tiles64, int *bm, int *bn)
 {
     // 128 x 128 tiles once they give every CU several workgroups, 64 x 128
-    // while those fill the chip, else 64 x 64 (twice the workgroups)
-    *bm = tiles128 >= 1024 ? 128 : 64;
+    // while those fill the chip, else 64 x 64 (twice the workgroups).  Columns
+    // whose cosine or sine rows fit 64 have as many 64-row tiles as 128-row
+    // ones, those half empty (270000 columns of 33 rows: 76 us forward and 62
+    // back with 128 rows, 56 and 43 with 64).
+    *bm = tiles128 >= 1024 && 4 * tiles64 > 5 * tiles128 ? 128 : 64;
     *bn = *bm == 128 || tiles64 >= 256 ? 128 : 64;
 }
 
