@@ -114,3 +114,28 @@ def test_p1_rows(gpu, n):
     x = np.random.default_rng(n).integers(-40, 41, (3, n)).astype(np.float32)
     got = core.circus(torch.from_numpy(x[None]).cuda(), [(1,)])[0, 0].cpu().numpy()
     assert np.array_equal(got, np.abs(np.diff(x, axis=1)).sum(axis=1))
+
+
+@pytest.mark.parametrize("n", [5, 67, 68, 69, 132, 133, 260, 261, 516, 517, 900, 1028, 1029, 1500,
+                               2047, 2048])
+def test_t6_t7_values_without_sources(oracle, gpu, n):
+    # T6 and T7 as a caller without index outputs gets them (T7 sorted by its
+    # values alone), together and each alone.  Two bright rows put the medians
+    # at the lines' starts: tails of 64 keys and powers of two up to 2048, one
+    # more and one less, distinct values in half of the columns and ties in the
+    # others, trailing zeros and zeros in between.
+    rng = np.random.default_rng(n)
+    img = rng.random((n, n), dtype=np.float32)
+    img[::2] = np.round(img[::2] * 64) / 64
+    img[:, 5::11] = 0.0
+    img[:, -2:] = 0.0
+    img[:, :2] = np.float32(n) ** 2
+    A, step = 3, 20.0
+    t = torch.from_numpy(img).cuda()
+    o, oaux = oracle.sinograms(img.ravel(), n, A, step, [6, 7], nthreads=8)
+    if n > 60:
+        assert (n - oaux["med_x"][0] >= n - 2).mean() > 0.9  # long tails at 0 degrees
+    both = core.sinograms(t, A, step, [6, 7]).cpu().numpy()
+    assert np.array_equal(both, o)
+    assert np.array_equal(core.sinograms(t, A, step, [7]).cpu().numpy()[0], o[1])
+    assert np.array_equal(core.sinograms(t, A, step, [6]).cpu().numpy()[0], o[0])
