@@ -289,8 +289,8 @@ class Batch:
 def set_tiles(device: int = 0, line=None, gather=None):
     """Forces the batched paths' tiles on ``device``'s context:
     ``line`` = (angles, columns) of a line-kernel wave item, ``gather`` =
-    (tile side, waves per workgroup) of the backward's transposed rotation;
-    None leaves the default (or the tuned choice)."""
+    (tile class 32 or 16, at most so many waves per workgroup) of the
+    backward's transposed rotation; None leaves the default (or the tuned choice)."""
     t = _lib.tt_tiles()
     if line is not None:
         t.line_angles, t.line_columns = int(line[0]), int(line[1])

@@ -101,8 +101,8 @@ struct BatchSinoParams {
     Slots slot;
 };
 
-// P-functionals over every sinogram column of a batch: one workgroup per
-// column; P3 twiddles are computed per image in LDS.
+// P-functionals over every sinogram column of a batch: one wave per column, or
+// one workgroup where the longest has more than 2048 rows.
 struct BatchCircusParams {
     const BatchImage *images;
     int nimg;
@@ -112,7 +112,6 @@ struct BatchCircusParams {
     int nmax;
     int np;
     int code[kMaxP];
-    int wave_done;        // P1..P3 entries written by circus_wave_batched_kernel (launcher's)
     int with_circus;      // circus_wave_batched_kernel writes circus values
 };
 

@@ -416,10 +416,15 @@ struct LineDst {
 // by the group's end; rows before a lane's median enter with distance 0.
 // Once every lane has passed, a row is its sample and the multiply-adds.
 //
-// T0..T5 of 1449^2 pixels at 360 angles: 1500 -> TIME us, and of 93^2 pixels
-// at 180 angles, one wave per three SIMDs, 58 -> TIME us; bound by VALU issue
-// (about 24 half-rate slots a row in pass 1, of which the bilinear sample is
-// 14; adds and multiplies issue twice as fast as the rest on this chip).
+// T0..T5 of 1449^2 pixels at 360 angles, from the two-load form to pairs and
+// untested groups: 1440 -> 930 us; of 363^2 at 360 194 -> 138; of 91^2 at 180
+// angles, one wave per three SIMDs, 54 -> 43.  Bound by VALU issue (about 24
+// half-rate slots a row in pass 1, of which the bilinear sample is 14; adds and
+// multiplies issue twice as fast as the rest on this chip) and, in a batch, as
+// much by the bytes behind the L2: 256 images of 91 to 725 rows read 53 GB of
+// pairs, 5.9 TB/s, half of the lookups hit, the waves wait for memory 28 % of
+// their cycles and for an issue slot 30 % (one image of 1449 rows: 2.4 GB, two
+// lookups in three hit, 27 and 25 %).
 template <bool TR, bool PAIRS, bool NEED_X, bool NEED_S, bool DO345, bool CK, bool FS>
 __device__ __forceinline__ void sino_line(const LineDst &p, const float *src,
                                           const float2 *s_tab, int a, int col,
@@ -1411,7 +1416,7 @@ __global__ __launch_bounds__(kBlock) void circus_batched_kernel(BatchCircusParam
     const int h = n / 2 + 1;
     circus_column(L, n, p.np, p.code, herm_none, nullptr,
                   im.circus + (size_t)t * p.np * p.A + a, p.A, nullptr,
-                  im.spec ? im.spec + (size_t)lc * 2 * h : nullptr, h, p.wave_done != 0);
+                  im.spec ? im.spec + (size_t)lc * 2 * h : nullptr, h, false);
 }
 
 // ---------------------------------------------------------------------------
@@ -2855,8 +2860,12 @@ constexpr int kGatherCols = 48;     // staged columns per angle, 16 a class
 
 // Tile class T (16 or 32) in pixels: the items of a column class, about
 // (TX + 1) (TY + 1) / 9 plus two thirds per column, just fill one or two
-// waves (30 x 32: 107 to 132 items, 4 % of the classes above 128; a 32 x 32
-// tile would need a third pass for nine classes in ten).
+// waves (30 x 32: 123 items in the middle, 132 in 99 of 100, 144 at right
+// angles, 1.5 % of the classes above 128; a 32 x 32 tile would need a third
+// pass for nine classes in ten).  The bound of ITEMS: the grown tile's chords
+// along every third column add up to at most a third of its area and the
+// longest chord, a chord of length L holds at most L + 1 rows, and r
+// consecutive rows lie in at most (r + 4) / 3 items.
 template <int T>
 struct GatherShape {
     static constexpr int TX = gather_tx(T), TY = gather_ty(T);
@@ -2864,8 +2873,15 @@ struct GatherShape {
     static constexpr int ACC = (((TX + 4) * P + 3) / 4) * 4;    // floats, halo of two cells
     static constexpr int NPIX = TX * TY / kWave;                // interior pixels per lane
     static constexpr int NIT = T == 16 ? 2 : 3;                 // passes over a class at most
+    static constexpr int DIAG = T == 16 ? 31 : 46;              // of the grown tile, rounded up
+    static constexpr int COLS = (DIAG + 2) / 3;                 // columns of a class
+    static constexpr int ITEMS = (int)(((TX + 1.02) * (TY + 1.02) / 3 + DIAG + 5 * COLS) / 3);
     static_assert(T == 16 || T == 32, "tile classes 16 and 32");
     static_assert(TX * TY % kWave == 0, "whole pixels per lane");
+    static_assert((TX + 1.02) * (TX + 1.02) + (TY + 1.02) * (TY + 1.02) < DIAG * DIAG &&
+                      DIAG <= kGatherCols - 2 && COLS <= 16,
+                  "a footprint's columns have their places");
+    static_assert(ITEMS < kWave * NIT, "a class's items lie inside NIT passes");
 };
 
 // LDS words of one wave: accumulators, the staged column data (per column:
@@ -3025,8 +3041,7 @@ __device__ __forceinline__ void gather_tile_wave(const GatherImg &im, const floa
         incl += __builtin_amdgcn_update_dpp(0, incl, 0x118, 0xf, 0xf, true);
         const int start = incl - cnt;
         if (f.k >= 0) {
-            // (the class's items number at most 156, or 75 with small tiles:
-            // every mark lies inside NIT passes)
+            // (inside NIT passes: GatherShape's ITEMS)
             reinterpret_cast<unsigned char *>(mark)[4 * start + scc] = 1;
             sA[lane] = float4{pa4.x, pa4.y, __int_as_float(first - 3 * start),
                               __int_as_float((rlo << 8) | len)};
