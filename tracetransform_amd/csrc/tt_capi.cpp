@@ -1031,8 +1031,9 @@ void layout_line_items(std::vector<ttk::BatchImage> &d,
 // alike), and neighbouring angles lie too far apart to share the L2: a line's
 // end moves by pi n / A pixels from angle to angle, and up to A = n / 10 (half
 // of the 64 columns a wave takes) the images are the faster.  T0 alone, with
-// little to hide the loads behind, up to 80 angles.  ms with pairs and with
-// images, T0..T5 (T0 alone):
+// little to hide the loads behind, up to n / 8, and 80 angles (363 rows at 72
+// angles: 0.95 of the time; where no border is zero, as padding leaves one,
+// 1.25).  ms with pairs and with images, T0..T5 (T0 alone):
 //   400 x 1449 rows,   8 angles   12.9   8.8    (9.9   6.3)
 //    64 x 1449 rows,  72 angles    9.5   8.4    (6.1   5.2)
 //    64 x 1449 rows, 180 angles   19.8  19.5   (11.9  12.0)
@@ -1051,7 +1052,7 @@ bool line_pairs(const std::vector<ttk::BatchImage> &d, int A, bool need_x, bool 
     if (px < 8.0 * (1 << 20))
         return true;
     const double side = px / lines;  // a line's mean length
-    return A >= (need_x || need_s ? side / 10.0 : std::max(80.0, side / 10.0));
+    return A >= (need_x || need_s ? side / 10.0 : std::max(80.0, side / 8.0));
 }
 
 // Bytes of an image's pixel pairs in both directions, or of its row-major copy.
