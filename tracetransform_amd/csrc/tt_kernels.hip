@@ -422,7 +422,7 @@ struct LineDst {
 // half-rate slots a row in pass 1, of which the bilinear sample is 14; adds and
 // multiplies issue twice as fast as the rest on this chip) and, in a batch, as
 // much by the bytes behind the L2: 256 images of 91 to 725 rows read 53 GB of
-// pairs, 5.9 TB/s, half of the lookups hit, the waves wait for memory 28 % of
+// pairs, 5.3 TB/s, half of the lookups hit, the waves wait for memory 28 % of
 // their cycles and for an issue slot 30 % (one image of 1449 rows: 2.4 GB, two
 // lookups in three hit, 27 and 25 %).
 template <bool TR, bool PAIRS, bool NEED_X, bool NEED_S, bool DO345, bool CK, bool FS>
